@@ -327,6 +327,40 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
     } else if (keyType != SORT_KEYS_UINT32) {
         return SORT_STATUS_INVALID_VALUE;
     }
+    if (n <= kLocalSortMaxKeys && e->fnLocal && !(earlyExit && !L.noAlloc)) {
+        // One workgroup runs every pass in LDS and leaves the result on the
+        // side the passes would.
+        int totalBits = 0;
+        for (int p = 0; p < numPasses; ++p) totalBits += widths[p];
+        const int out = numPasses & 1;
+        mgpuLocalArgs la;
+        std::memset(&la, 0, sizeof(la));
+        la.keys_in = keyBuf[0];
+        la.keys_out = keyBuf[out];
+        const int carried = valueCount == -1 ? 1 : valueCount;
+        for (int v = 0; v < carried; ++v) {
+            la.vals_in[v] = valBuf[v][0];
+            la.vals_out[v] = valBuf[v][out];
+        }
+        la.n = n;
+        la.first_bit = (uint32_t)firstBit;
+        la.num_bits = (uint32_t)totalBits;
+        la.vals_mode = valueCount == 0    ? MGPU_VALUES_NONE
+                       : valueCount == -1 ? MGPU_VALUES_INDEX
+                       : valueCount == 1  ? MGPU_VALUES_SINGLE
+                                          : MGPU_VALUES_MULTI;
+        la.num_values = (uint32_t)carried;
+        la.in_lo = toLo;
+        la.in_hi = toHi;
+        // Back: int32 flips the sign bit again; float32 flips the words
+        // whose top bit the mapping cleared.
+        la.out_lo = toHi;
+        la.out_hi = toLo;
+        const sortStatus_t ls = mgpu_launch(e, L.stream, valueCount ? e->fnLocalPay : e->fnLocal, 1,
+                                            MGPU_LOCAL_THREADS, &la, !L.noAlloc);
+        if (!ls && executed) *executed = numPasses;
+        return ls;
+    }
     const SortPlanChoice choice = mgpu_pick_plan(e, n, valueCount);
     const PassVariant& var = *choice.variant;
     const uint32_t tile = var.tile();

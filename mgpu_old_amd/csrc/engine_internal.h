@@ -117,6 +117,12 @@ struct sortEngine_d {
     hipFunction_t fnCountKM = nullptr;    // the two over signed or float keys
     hipFunction_t fnCountColsKM = nullptr;
     hipFunction_t fnScan = nullptr;
+    // One workgroup, every pass in LDS: keys only, and with a payload.  Null
+    // where the atomic-add ranking is off, or where a tile shape or a chain
+    // per XCD was asked for by name (the device-wide passes then run at every
+    // size).
+    hipFunction_t fnLocal = nullptr;
+    hipFunction_t fnLocalPay = nullptr;
     hipFunction_t fnIota = nullptr;
     hipFunction_t fnKeyTransform = nullptr;
     hipFunction_t fnMultiCount = nullptr;      // 256 threads, per-wave histograms
@@ -208,6 +214,11 @@ constexpr uint32_t kXsegMinTilesPerSeg = 128;
 // form faster at 2^12 and below (7.6 against 8.2 us).
 constexpr uint32_t kCountColsMinKeys = 1u << 20;
 const PassVariant& mgpu_pick_variant(const sortEngine_d* e, uint64_t keys);
+// Arrays of at most this many keys are sorted by one workgroup in one launch:
+// all that its LDS holds beside the digit counts (key and payload staged), and
+// still ahead of the device-wide passes there (16384 keys: 18.8 against 38.8
+// us, with one value 23.1 against 44.5, with three 38.9 against 56.0).
+constexpr uint32_t kLocalSortMaxKeys = MGPU_LOCAL_MAX_KEYS;
 
 // Value classes of the sortArray tuning table.
 enum { MGPU_SORT_CLASS_KEYS = 0, MGPU_SORT_CLASS_INDEX = 1, MGPU_SORT_CLASS_KV = 2,

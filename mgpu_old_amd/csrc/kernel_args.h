@@ -328,5 +328,24 @@ struct mgpuPassArgs {
     uint32_t key_types;
 };
 
+// local_sort: one workgroup sorts an array of at most MGPU_LOCAL_MAX_KEYS keys
+// through every digit pass in LDS.
+#define MGPU_LOCAL_THREADS 1024
+#define MGPU_LOCAL_MAX_KEYS 16384
+struct mgpuLocalArgs {
+    const uint32_t* keys_in;
+    uint32_t* keys_out;           // may be keys_in
+    const uint32_t* vals_in[MGPU_MAX_VALUES];
+    uint32_t* vals_out[MGPU_MAX_VALUES];  // each may be its vals_in
+    uint32_t n;
+    uint32_t first_bit;
+    uint32_t num_bits;
+    uint32_t vals_mode;           // MGPU_VALUES_*
+    uint32_t num_values;          // MGPU_VALUES_MULTI only
+    // mgpu_key_map words applied to the keys as they are read and written.
+    uint32_t in_lo, in_hi, out_lo, out_hi;
+    uint32_t pad_;
+};
+
 // Segments per XCD with counting for the next pass: at most this many.
 #define MGPU_XSEG_COUNT_SEGS 8

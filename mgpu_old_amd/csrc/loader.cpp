@@ -241,6 +241,11 @@ sortStatus_t mgpu_engine_load(sortEngine_d* e) {
     st = load_variant(e, smallShape[0], smallShape[1], e->rankMethod, &e->small);
     if (!st) st = load_variant(e, largeShape[0], largeShape[1], e->rankMethod, &e->large);
     if (st) return st;
+    if (e->rankMethod == 1 && !e->xcdForce && !(t && *t)) {
+        st = get_fn(e, e->radixModule, "mgpu_local_sort_k", &e->fnLocal);
+        if (!st) st = get_fn(e, e->radixModule, "mgpu_local_sort_kv", &e->fnLocalPay);
+        if (st) return st;
+    }
     const char* spin = std::getenv("MGPUSORT_SPIN_LIMIT");
     if (spin && *spin) e->spinLimit = (uint32_t)std::strtoul(spin, nullptr, 10);
     const char* ee = std::getenv("MGPUSORT_EE");

@@ -1,0 +1,207 @@
+// Stable LSD sort of up to 16384 keys by one workgroup, all digit passes in
+// registers and LDS: one launch and one read and write of the data, where the
+// device-wide passes take a launch per pass.
+//
+// Bound: a pass is a chain of LDS round trips and four barriers, not
+// bandwidth (16384 pairs are 256 KB): key + value, with the fill of the input,
+// 1000 keys 34.3 -> 6.9 us a sort, 4096 35.8 -> 10.1, 16384 44.5 -> 23.1
+// against the device-wide passes (a launch each, ~6 us whatever the size);
+// keys only 32.2 -> 7.0, 33.2 -> 8.8, 38.8 -> 18.8.  So every slot's rank is requested
+// before the first one is used, and the digit scan runs over all threads at
+// once: thread (digit, group) adds the counts of four waves, and one scan over
+// the threads in that order gives each wave's start of each digit directly.
+#pragma once
+#include "kernel_args.h"
+#include "radix_device.h"
+
+namespace mgpu {
+
+constexpr int kLocalBlock = MGPU_LOCAL_THREADS;
+constexpr int kLocalWaves = kLocalBlock / 64;
+constexpr uint32_t kLocalTile = MGPU_LOCAL_MAX_KEYS;
+// Words from one wave's digit counts to the next: a multiple of 4 for 16-byte
+// clearing, and not of 64, so that the scan's threads (digit, group of four
+// waves) read different banks.
+constexpr uint32_t kLocalRow = MGPU_RADIX + 4;
+static_assert(kLocalBlock == 4 * MGPU_RADIX && kLocalWaves == 16,
+              "the scan gives a thread one digit of four waves");
+
+template <bool PAY>
+struct LocalShared {
+    uint32_t count[kLocalWaves * kLocalRow] __attribute__((aligned(16)));
+    uint32_t tmp[kLocalWaves];
+    uint32_t key[kLocalTile];
+    uint32_t pay[PAY ? kLocalTile : 1];
+};
+
+// Rank of this lane's digit among its wave's keys so far, for IT slots at
+// once (RANK 1 of rank_scatter: one LDS add per key, served in ascending lane
+// order).  A slot whose 64 keys share a digit would serialize 64 adds on one
+// word; when any slot is like that (sorted or low-entropy keys), the slots go
+// one by one and such a slot adds once.  Else no add waits for another.
+template <int IT>
+__device__ __forceinline__ void rank_slots(const uint32_t (&d)[IT], uint32_t* row, uint32_t lane,
+                                           uint32_t (&rank)[IT]) {
+    bool one = false;
+#pragma unroll
+    for (int j = 0; j < IT; ++j)
+        one = one || __builtin_amdgcn_ballot_w64(d[j] == (uint32_t)__builtin_amdgcn_readfirstlane(
+                                                             (int)d[j])) == ~0ull;
+    if (!one) {
+#pragma unroll
+        for (int j = 0; j < IT; ++j)
+            rank[j] = __hip_atomic_fetch_add(&row[d[j]], 1u, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)d[j]);
+        if (__builtin_amdgcn_ballot_w64(d[j] == f) == ~0ull) {
+            uint32_t b = 0;
+            if (lane == 0)
+                b = __hip_atomic_fetch_add(&row[f], 64u, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+            rank[j] = (uint32_t)__builtin_amdgcn_readfirstlane((int)b) + lane;
+        } else {
+            rank[j] = __hip_atomic_fetch_add(&row[d[j]], 1u, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+    }
+}
+
+// Buffer resource over words [0, n) at p: loads past n return 0, stores there
+// are dropped.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t words_rsrc(const uint32_t* p, uint32_t n) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p), 0, (int)(n * 4u),
+                                             0x00020000);
+}
+
+// Sorts elements [begin, begin + n) of the arrays of `a`, 0 < n <= IT *
+// kLocalBlock, by bits [shift0, shift0 + bits) of (key - base).  IT keys per
+// thread: wave w holds keys w * 64 * IT + j * 64 + lane.  Slots past n hold
+// all ones in every digit, so they stay behind every key.
+template <int IT, bool PAY>
+__device__ void local_sort_items(const mgpuLocalArgs& a, LocalShared<PAY>& sh, uint32_t begin,
+                                 uint32_t n, uint32_t base, uint32_t shift0, uint32_t bits) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t first = wave * 64 * IT + lane;  // this lane's key of slot 0
+    const uint32_t off = first * 4u;
+    const uint32_t fill = a.vals_mode;
+    uint32_t key[IT], pay[PAY ? IT : 1];
+    {
+        const __amdgpu_buffer_rsrc_t rk = words_rsrc(a.keys_in + begin, n);
+#pragma unroll
+        for (int j = 0; j < IT; ++j)
+            key[j] = __builtin_amdgcn_raw_buffer_load_b32(rk, (int)(off + j * 256u), 0, 0);
+        if constexpr (PAY) {
+            if (fill == MGPU_VALUES_SINGLE) {
+                const __amdgpu_buffer_rsrc_t rv = words_rsrc(a.vals_in[0] + begin, n);
+#pragma unroll
+                for (int j = 0; j < IT; ++j)
+                    pay[j] = __builtin_amdgcn_raw_buffer_load_b32(rv, (int)(off + j * 256u), 0, 0);
+            } else {
+#pragma unroll
+                for (int j = 0; j < IT; ++j) pay[j] = first + j * 64u;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < IT; ++j)
+        key[j] = first + j * 64u < n ? mgpu_key_map(key[j], a.in_lo, a.in_hi) - base : 0xFFFFFFFFu;
+
+    uint32_t* const row = sh.count + wave * kLocalRow;
+    const uint32_t dq = tid >> 2, g = tid & 3u;  // the scan's digit and group of waves
+    uint32_t* const col = sh.count + g * 4 * kLocalRow + dq;
+    const uint32_t passes = (bits + MGPU_RADIX_BITS - 1) / MGPU_RADIX_BITS;
+    uint32_t shift = shift0, left = bits;
+    for (uint32_t p = 0; p < passes; ++p) {
+        const uint32_t width = left / (passes - p);  // the narrower digits first
+        // The wave's counts are its own between the scans: no barrier.
+        reinterpret_cast<uint4*>(row)[lane] = make_uint4(0u, 0u, 0u, 0u);
+        uint32_t d[IT], pos[IT];
+#pragma unroll
+        for (int j = 0; j < IT; ++j) d[j] = __builtin_amdgcn_ubfe(key[j], shift, width);
+        rank_slots<IT>(d, row, lane, pos);
+        __syncthreads();
+        const uint32_t c0 = col[0], c1 = col[kLocalRow], c2 = col[2 * kLocalRow],
+                       c3 = col[3 * kLocalRow];
+        const uint32_t sum = c0 + c1 + c2 + c3;
+        const uint32_t inc = wave_inclusive_scan_dpp(sum);
+        if (lane == 63) sh.tmp[wave] = inc;
+        __syncthreads();
+        const uint32_t waves = row_inclusive_scan_dpp(sh.tmp[lane & (kLocalWaves - 1)]);
+        uint32_t start = inc - sum;
+        if (wave > 0) start += (uint32_t)__builtin_amdgcn_readlane((int)waves, (int)(wave - 1));
+        col[0] = start;
+        col[kLocalRow] = start + c0;
+        col[2 * kLocalRow] = start + c0 + c1;
+        col[3 * kLocalRow] = start + c0 + c1 + c2;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < IT; ++j) pos[j] += row[d[j]];
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+            sh.key[pos[j]] = key[j];
+            if constexpr (PAY) sh.pay[pos[j]] = pay[j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+            key[j] = sh.key[first + j * 64];
+            if constexpr (PAY) pay[j] = sh.pay[first + j * 64];
+        }
+        shift += width;
+        left -= width;
+    }
+
+    // Every key and carried value was loaded before a barrier above, so the
+    // output may be the input's buffers.
+    {
+        const __amdgpu_buffer_rsrc_t rk = words_rsrc(a.keys_out + begin, n);
+#pragma unroll
+        for (int j = 0; j < IT; ++j)
+            __builtin_amdgcn_raw_buffer_store_b32(mgpu_key_map(key[j] + base, a.out_lo, a.out_hi), rk,
+                                                  (int)(off + j * 256u), 0, 0);
+    }
+    if constexpr (PAY) {
+        if (fill != MGPU_VALUES_MULTI) {
+            const __amdgpu_buffer_rsrc_t rv = words_rsrc(a.vals_out[0] + begin, n);
+#pragma unroll
+            for (int j = 0; j < IT; ++j)
+                __builtin_amdgcn_raw_buffer_store_b32(pay[j], rv, (int)(off + j * 256u), 0, 0);
+        } else {
+            // Two or more arrays: gathered through the source index.
+            for (uint32_t v = 0; v < a.num_values; ++v) {
+                const __amdgpu_buffer_rsrc_t rv = words_rsrc(a.vals_in[v] + begin, n);
+                const __amdgpu_buffer_rsrc_t ro = words_rsrc(a.vals_out[v] + begin, n);
+                uint32_t val[IT];
+#pragma unroll
+                for (int j = 0; j < IT; ++j)
+                    val[j] = __builtin_amdgcn_raw_buffer_load_b32(rv, (int)(pay[j] * 4u), 0, 0);
+                // Every gather of the workgroup has its data before the
+                // first store (the two sides may be one buffer).
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < IT; ++j)
+                    __builtin_amdgcn_raw_buffer_store_b32(val[j], ro, (int)(off + j * 256u), 0, 0);
+            }
+        }
+    }
+}
+
+template <bool PAY>
+__device__ __forceinline__ void local_sort(const mgpuLocalArgs& a, LocalShared<PAY>& sh,
+                                           uint32_t begin, uint32_t n, uint32_t base,
+                                           uint32_t shift, uint32_t bits) {
+    if (n <= 1 * kLocalBlock) local_sort_items<1, PAY>(a, sh, begin, n, base, shift, bits);
+    else if (n <= 2 * kLocalBlock) local_sort_items<2, PAY>(a, sh, begin, n, base, shift, bits);
+    else if (n <= 4 * kLocalBlock) local_sort_items<4, PAY>(a, sh, begin, n, base, shift, bits);
+    else if (n <= 8 * kLocalBlock) local_sort_items<8, PAY>(a, sh, begin, n, base, shift, bits);
+    else if (n <= 12 * kLocalBlock) local_sort_items<12, PAY>(a, sh, begin, n, base, shift, bits);
+    else local_sort_items<16, PAY>(a, sh, begin, n, base, shift, bits);
+}
+
+}  // namespace mgpu

@@ -50,6 +50,35 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x, uint32_t lan
     return x;
 }
 
+// The same by DPP moves, one VALU instruction a step, where a shuffle is an
+// LDS round trip: shifts of 1, 2, 4, 8 inside each row of 16 lanes, then the
+// last lane of a row broadcast to the row after it (row 1 and 3), and lane 31
+// to the upper half.  Lanes without a source add 0.  All 64 lanes active.
+__device__ __forceinline__ uint32_t wave_inclusive_scan_dpp(uint32_t x) {
+#define MGPU_DPP_ADD(CTRL, ROWS) \
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, false)
+    MGPU_DPP_ADD(0x111, 0xF);  // row_shr:1
+    MGPU_DPP_ADD(0x112, 0xF);  // row_shr:2
+    MGPU_DPP_ADD(0x114, 0xF);  // row_shr:4
+    MGPU_DPP_ADD(0x118, 0xF);  // row_shr:8
+    MGPU_DPP_ADD(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
+    MGPU_DPP_ADD(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
+#undef MGPU_DPP_ADD
+    return x;
+}
+
+// Inclusive scan within each row of 16 lanes.
+__device__ __forceinline__ uint32_t row_inclusive_scan_dpp(uint32_t x) {
+#define MGPU_DPP_ADD(CTRL) \
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false)
+    MGPU_DPP_ADD(0x111);
+    MGPU_DPP_ADD(0x112);
+    MGPU_DPP_ADD(0x114);
+    MGPU_DPP_ADD(0x118);
+#undef MGPU_DPP_ADD
+    return x;
+}
+
 // Exclusive scan of x over all threads of the block (threads that do not
 // take part pass 0).  s_tmp holds one word per wave.  Contains barriers:
 // every thread of the block must call it.

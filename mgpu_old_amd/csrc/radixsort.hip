@@ -30,6 +30,7 @@
 #include <stdint.h>
 
 #include "kernel_args.h"
+#include "localsort.h"
 #include "radix_device.h"
 
 namespace {
@@ -1830,6 +1831,18 @@ MGPU_RANK_SCATTER_KM(1024, 16)
 MGPU_PACKED(256, 16)
 MGPU_PACKED(512, 16)
 MGPU_PACKED(1024, 16)
+
+// One workgroup sorts a small array through every pass: keys only, or with a
+// payload (a value, a generated index, or the source index of several values).
+extern "C" __global__ void __launch_bounds__(MGPU_LOCAL_THREADS) mgpu_local_sort_k(mgpuLocalArgs a) {
+    __shared__ mgpu::LocalShared<false> sh;
+    mgpu::local_sort<false>(a, sh, 0u, a.n, 0u, a.first_bit, a.num_bits);
+}
+
+extern "C" __global__ void __launch_bounds__(MGPU_LOCAL_THREADS) mgpu_local_sort_kv(mgpuLocalArgs a) {
+    __shared__ mgpu::LocalShared<true> sh;
+    mgpu::local_sort<true>(a, sh, 0u, a.n, 0u, a.first_bit, a.num_bits);
+}
 
 // Check of the ordering RANK 1 relies on: wave w of one 1024-thread
 // workgroup adds 1 per lane, for 16 rounds, to the count of digit
