@@ -34,42 +34,6 @@ struct LocalShared {
     uint32_t pay[PAY ? kLocalTile : 1];
 };
 
-// Rank of this lane's digit among its wave's keys so far, for IT slots at
-// once (RANK 1 of rank_scatter: one LDS add per key, served in ascending lane
-// order).  A slot whose 64 keys share a digit would serialize 64 adds on one
-// word; when any slot is like that (sorted or low-entropy keys), the slots go
-// one by one and such a slot adds once.  Else no add waits for another.
-template <int IT>
-__device__ __forceinline__ void rank_slots(const uint32_t (&d)[IT], uint32_t* row, uint32_t lane,
-                                           uint32_t (&rank)[IT]) {
-    bool one = false;
-#pragma unroll
-    for (int j = 0; j < IT; ++j)
-        one = one || __builtin_amdgcn_ballot_w64(d[j] == (uint32_t)__builtin_amdgcn_readfirstlane(
-                                                             (int)d[j])) == ~0ull;
-    if (!one) {
-#pragma unroll
-        for (int j = 0; j < IT; ++j)
-            rank[j] = __hip_atomic_fetch_add(&row[d[j]], 1u, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_WORKGROUP);
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < IT; ++j) {
-        const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)d[j]);
-        if (__builtin_amdgcn_ballot_w64(d[j] == f) == ~0ull) {
-            uint32_t b = 0;
-            if (lane == 0)
-                b = __hip_atomic_fetch_add(&row[f], 64u, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-            rank[j] = (uint32_t)__builtin_amdgcn_readfirstlane((int)b) + lane;
-        } else {
-            rank[j] = __hip_atomic_fetch_add(&row[d[j]], 1u, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-    }
-}
-
 // Buffer resource over words [0, n) at p: loads past n return 0, stores there
 // are dropped.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t words_rsrc(const uint32_t* p, uint32_t n) {
@@ -127,13 +91,8 @@ __device__ void local_sort_items(const mgpuLocalArgs& a, LocalShared<PAY>& sh, u
         __syncthreads();
         const uint32_t c0 = col[0], c1 = col[kLocalRow], c2 = col[2 * kLocalRow],
                        c3 = col[3 * kLocalRow];
-        const uint32_t sum = c0 + c1 + c2 + c3;
-        const uint32_t inc = wave_inclusive_scan_dpp(sum);
-        if (lane == 63) sh.tmp[wave] = inc;
-        __syncthreads();
-        const uint32_t waves = row_inclusive_scan_dpp(sh.tmp[lane & (kLocalWaves - 1)]);
-        uint32_t start = inc - sum;
-        if (wave > 0) start += (uint32_t)__builtin_amdgcn_readlane((int)waves, (int)(wave - 1));
+        const uint32_t start =
+            block_exclusive_scan_dpp<kLocalBlock>(c0 + c1 + c2 + c3, sh.tmp, lane, wave);
         col[0] = start;
         col[kLocalRow] = start + c0;
         col[2 * kLocalRow] = start + c0 + c1;

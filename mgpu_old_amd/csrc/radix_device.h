@@ -97,6 +97,23 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t x, uint32_t* s
     return before + inc - x;
 }
 
+// The same by DPP scans, for at most 16 waves, all lanes active; `wave` the
+// same in every lane.  One barrier inside; s_tmp is free again after the
+// caller's next one.
+template <int BLOCK>
+__device__ __forceinline__ uint32_t block_exclusive_scan_dpp(uint32_t x, uint32_t* s_tmp,
+                                                             uint32_t lane, uint32_t wave) {
+    constexpr uint32_t W = BLOCK / 64;
+    static_assert(W <= 16, "one row of lanes holds the waves' totals");
+    const uint32_t inc = wave_inclusive_scan_dpp(x);
+    if (lane == 63) s_tmp[wave] = inc;
+    __syncthreads();
+    const uint32_t waves = row_inclusive_scan_dpp((lane & 15u) < W ? s_tmp[lane & 15u] : 0u);
+    uint32_t start = inc - x;
+    if (wave > 0) start += (uint32_t)__builtin_amdgcn_readlane((int)waves, (int)(wave - 1));
+    return start;
+}
+
 // Stable rank of one key per lane among the 64 lanes of a wave by digit d:
 // returns the number of earlier keys of the wave with the same digit (earlier
 // slots, counted in `count`, plus lower lanes of this slot) and advances
@@ -116,6 +133,42 @@ __device__ __forceinline__ uint32_t wave_rank(uint32_t d, uint32_t lane, uint32_
         __hip_atomic_store(&match[d], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     return old + below;
+}
+
+// Rank of this lane's digit among its wave's keys so far, for IT slots at
+// once (RANK 1 of rank_scatter: one LDS add per key, served in ascending lane
+// order).  A slot whose 64 keys share a digit would serialize 64 adds on one
+// word; when any slot is like that (sorted or low-entropy keys), the slots go
+// one by one and such a slot adds once.  Else no add waits for another.
+template <int IT>
+__device__ __forceinline__ void rank_slots(const uint32_t (&d)[IT], uint32_t* row, uint32_t lane,
+                                           uint32_t (&rank)[IT]) {
+    bool one = false;
+#pragma unroll
+    for (int j = 0; j < IT; ++j)
+        one = one || __builtin_amdgcn_ballot_w64(d[j] == (uint32_t)__builtin_amdgcn_readfirstlane(
+                                                             (int)d[j])) == ~0ull;
+    if (!one) {
+#pragma unroll
+        for (int j = 0; j < IT; ++j)
+            rank[j] = __hip_atomic_fetch_add(&row[d[j]], 1u, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)d[j]);
+        if (__builtin_amdgcn_ballot_w64(d[j] == f) == ~0ull) {
+            uint32_t b = 0;
+            if (lane == 0)
+                b = __hip_atomic_fetch_add(&row[f], 64u, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+            rank[j] = (uint32_t)__builtin_amdgcn_readfirstlane((int)b) + lane;
+        } else {
+            rank[j] = __hip_atomic_fetch_add(&row[d[j]], 1u, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+    }
 }
 
 }  // namespace mgpu

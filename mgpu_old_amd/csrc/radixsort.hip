@@ -66,6 +66,12 @@ __device__ __forceinline__ uint32_t next_lane(uint32_t v, uint32_t lane63) {
     return (uint32_t)__builtin_amdgcn_update_dpp((int)lane63, (int)v, 0x130, 0xF, 0xF, false);
 }
 
+// v of lane ^ off, for off 1 or 2 (DPP quad_perm).
+__device__ __forceinline__ uint32_t quad_xor(uint32_t v, uint32_t off) {
+    return off == 1 ? (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true)
+                    : (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);
+}
+
 // Orders this wave's LDS accesses before and after the call.
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -904,6 +910,14 @@ __device__ void rank_scatter_body(const Args& a) {
     constexpr int W = BLOCK / 64;
     constexpr uint32_t TILE = BLOCK * IPT;
     constexpr uint32_t WAVE_TILE = 64 * IPT;
+    // Threads per digit, in the digit scan and the lookback: thread tid works
+    // on digit tid / G, in the scan on the counts of R waves from (tid % G) * R.
+    constexpr uint32_t G = BLOCK / RADIX;
+    constexpr uint32_t R = W / G;
+    static_assert(G * R == (uint32_t)W, "every wave's counts belong to one thread per digit");
+    // Words from one wave's counts to the next: not a multiple of the banks,
+    // so that the scan's threads of one digit read different ones.
+    constexpr uint32_t ROW = RADIX + 4;
 
     // One value array or generated indices are staged beside the keys.  The
     // in-wave match masks are only live during ranking, before anything is
@@ -914,26 +928,28 @@ __device__ void rank_scatter_body(const Args& a) {
     constexpr uint32_t AUX_WORDS = AUX_WORDS0 > 0 ? AUX_WORDS0 : 2;
     __shared__ uint32_t s_stage[TILE];
     __shared__ __attribute__((aligned(16))) uint32_t s_aux[AUX_WORDS];
-    __shared__ uint32_t s_count[W][RADIX];
+    __shared__ __attribute__((aligned(16))) uint32_t s_count[W][ROW];
     uint64_t(*const s_match)[RADIX] = reinterpret_cast<uint64_t(*)[RADIX]>(s_aux);
     uint32_t* const s_vstage = s_aux;
     __shared__ uint32_t s_global[RADIX];
     __shared__ uint32_t s_tmp[W];
     __shared__ uint32_t s_tile[2];
-    __shared__ uint32_t s_lstart[RADIX];
-    __shared__ uint32_t s_tcount[RADIX];
     // XSEG: this segment's digit starts, and the next pass's digit counts of
-    // the keys this workgroup writes, by destination segment.
+    // the keys this workgroup writes, by destination segment (one row more
+    // for the slots that write nothing).
     constexpr uint32_t NSEG = MGPU_XSEG_COUNT_SEGS;
     __shared__ uint32_t s_dstart[XSINGLE ? RADIX : 1];
-    __shared__ uint32_t s_next[XSINGLE ? NSEG * RADIX : 1];
+    __shared__ uint32_t s_next[XSINGLE ? (NSEG + 1) * RADIX : 1];
     __shared__ uint32_t s_spare[XSINGLE ? 64 : 1];
 
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63;
-    const uint32_t wave = tid >> 6;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t shift = a.shift, mask = a.mask;
     const uint32_t width = (uint32_t)__builtin_popcount(mask);  // mask = 2^width - 1
+    uint32_t* const row = s_count[wave];  // this wave's digit counts
+    const uint32_t gd = tid / G, gk = tid % G;
+    uint32_t* const col = &s_count[gk * R][gd];
 
     // The segment of this workgroup's XCD (XSEG), else the whole array.
     uint32_t seg = 0, seg_first = 0, seg_tiles = a.num_tiles;
@@ -955,23 +971,31 @@ __device__ void rank_scatter_body(const Args& a) {
             seg_tiles = 0;  // no segment for this XCD: nothing to take
         }
     }
-    for (uint32_t i = tid; i < (uint32_t)(W * RADIX); i += BLOCK) {
-        (&s_count[0][0])[i] = 0;
-        if constexpr (RANK == 0) (&s_match[0][0])[i] = 0;
-    }
+    // Each wave clears its own counts (and masks), which no other touches
+    // before the next barrier.
+    auto clear_counts = [&]() {
+        reinterpret_cast<uint4*>(row)[lane] = make_uint4(0u, 0u, 0u, 0u);
+        if constexpr (RANK == 0)
+#pragma unroll
+            for (uint32_t i = 0; i < RADIX; i += 64) s_match[wave][i + lane] = 0;
+    };
+    clear_counts();
     // XSEG: whether this pass counts for the next one, and this segment's
     // digit starts.
     bool count_next = false;
-    // Segment of output position q: ((q / TILE + 1) * S - 1) / T for S
-    // segments of T tiles (the largest x with floor(x * T / S) * TILE <= q),
-    // as fma(num, 1/T, 0.5/T) truncated: num < 2^21 is exact in a float, the
-    // quotient is at least 0.5/T >= 2^-17 from an integer, and the rounding of
-    // 1/T and of the fma errs by less than 2^-19.
+    // Segment of output position q in tile t = q / TILE, for S segments of T
+    // tiles (the largest x with floor(x * T / S) <= t): floor((t * S + S - 1)
+    // / T), as fma(t, S/T, (S - 0.5)/T) truncated: t < 2^16 is exact in a
+    // float, the true quotient, half a step up, is at least 0.5/T >= 2^-17
+    // from an integer, and the roundings of S/T (times t: below 2^-21), of
+    // the constant and of the fma err by less than 2^-19.
     const float seg_rcp = 1.0f / (float)a.num_tiles;
-    const float seg_half = 0.5f * seg_rcp;
+    float seg_mul = 0.f, seg_add = 0.f;
     uint32_t next_mode = RADIX;  // most frequent digit of the next pass
     uint32_t next_width = 0;
     if constexpr (XSINGLE) {
+        seg_mul = (float)a.num_segs * seg_rcp;
+        seg_add = ((float)a.num_segs - 0.5f) * seg_rcp;
         count_next = a.seg_count_out != nullptr;
         if (count_next) {
             next_mode = *a.next_mode;
@@ -990,52 +1014,65 @@ __device__ void rank_scatter_body(const Args& a) {
         }
     }
 
-    while (true) {
-        // The tile comes from the counter in start order (and is sorted right
-        // away), so a tile only ever waits on tiles that are already running.
-        if (tid == 0) {
-            uint32_t t = seg_tiles;  // a workgroup of an XCD without a segment takes none
-            bool grouped = false;
-            if constexpr (MULTI && !XSEG) grouped = a.num_xcds > 1;
-            if (grouped) {
-                if constexpr (MULTI && !XSEG) t = take_grouped_tile(a);
-            } else if (seg_tiles > 0) {
-                t = __hip_atomic_fetch_add(a.tile_counter + seg, 1u, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-            }
-            s_tile[0] = t;
-            s_tile[1] = MULTI && t < seg_tiles ? find_array<MULTI>(a, seg_first + t) : 0u;
+    // The next tile of this workgroup, from the counter in start order, so a
+    // tile only ever waits on tiles that workgroups already running hold and
+    // take in order (thread 0; seg_tiles when there is none left).
+    auto take_tile = [&]() {
+        uint32_t t = seg_tiles;  // a workgroup of an XCD without a segment takes none
+        bool grouped = false;
+        if constexpr (MULTI && !XSEG) grouped = a.num_xcds > 1;
+        if (grouped) {
+            if constexpr (MULTI && !XSEG) t = take_grouped_tile(a);
+        } else if (seg_tiles > 0) {
+            t = __hip_atomic_fetch_add(a.tile_counter + seg, 1u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
         }
-        __syncthreads();
-        // Tile and array indices are the same for every lane: keep them (and all
-        // that is derived from them) in scalar registers.
-        const uint32_t gtile = __builtin_amdgcn_readfirstlane(s_tile[0]);
-        if (gtile >= seg_tiles) {
-            // One tile per workgroup: only a counter left dirty gets here.  A
-            // segment's workgroup: the segment is done.
-            if (!XSEG && tid == 0) set_error(a.error_flag, 2u);
-            break;
-        }
-        // MULTI: tiles are numbered across the arrays; XSINGLE: within the
-        // segment, whose chain starts at its first tile.
-        TileJob job = make_job<MULTI>(a, MULTI ? seg_first + gtile : gtile,
-                                      __builtin_amdgcn_readfirstlane(s_tile[1]));
+        return t;
+    };
+    auto post_tile = [&](uint32_t t) {
+        s_tile[0] = t;
+        if constexpr (MULTI) s_tile[1] = t < seg_tiles ? find_array<MULTI>(a, seg_first + t) : 0u;
+    };
+    // MULTI: tiles are numbered across the arrays; XSINGLE: within the
+    // segment, whose chain starts at its first tile.  Tile and array indices
+    // are the same for every lane: they (and all that is derived from them)
+    // stay in scalar registers.
+    auto posted_job = [&](uint32_t gtile) {
+        TileJob job = make_job<MULTI>(
+            a, MULTI ? seg_first + gtile : gtile,
+            MULTI ? (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[1]) : 0u);
         if constexpr (XSINGLE) {
             job.first = seg_first;
             job.lookback += (size_t)seg_first * RADIX;
         }
+        return job;
+    };
+    uint32_t key[IPT], val[IPT];
+    // Keys and the single value array of a tile, striped, requested together:
+    // ranking starts once the keys are in while the values still load.
+    auto load_tile = [&](const TileJob& job) {
+        const uint32_t wave_base = (job.first + job.tile) * TILE + wave * WAVE_TILE;
+        load_striped<IPT>(job.keys_in, job.n, wave_base, lane, key);
+        if constexpr (VMODE == MGPU_VALUES_SINGLE)
+            load_striped<IPT>(job_vals_in<MULTI>(a, job, 0), job.n, wave_base, lane, val);
+    };
+
+    if (tid == 0) post_tile(take_tile());
+    __syncthreads();
+    uint32_t gtile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
+    // One tile per workgroup: only a counter left dirty finds none.
+    if (!XSEG && gtile >= seg_tiles && tid == 0) set_error(a.error_flag, 2u);
+    TileJob job{};
+    if (gtile < seg_tiles) {
+        job = posted_job(gtile);
+        load_tile(job);
+    }
+    while (gtile < seg_tiles) {
         const uint32_t n = job.n, tile = job.tile;
         const uint32_t base = (job.first + tile) * TILE;
         const uint32_t wave_base = base + wave * WAVE_TILE;
         const uint32_t tile_valid = min(TILE, n - base);
         const bool full = tile_valid == TILE;
-
-        // Keys and the single value array, striped, requested together: ranking
-        // starts as soon as each key slot is in while the values still load.
-        uint32_t key[IPT], val[IPT];
-        load_striped<IPT>(job.keys_in, n, wave_base, lane, key);
-        if constexpr (VMODE == MGPU_VALUES_SINGLE)
-            load_striped<IPT>(job_vals_in<MULTI>(a, job, 0), n, wave_base, lane, val);
         // Signed or float keys (KMAP), in the sort's first pass: to their
         // unsigned order.
         if constexpr (KMAP) {
@@ -1091,33 +1128,33 @@ __device__ void rank_scatter_body(const Args& a) {
                 const uint32_t d = digit_of(j), q = (uint32_t)j * 64 + lane;
                 pos[j] = q - first[d];
                 const uint32_t pd = prev_lane(d, tail);
-                if (q != 0 && pd != d) s_count[wave][pd] = q - first[pd];  // run of pd ends at q
+                if (q != 0 && pd != d) row[pd] = q - first[pd];  // run of pd ends at q
                 tail = __builtin_amdgcn_readlane(d, 63);
             }
             if (lane == 63) {
                 const uint32_t d = digit_of(IPT - 1);
-                s_count[wave][d] = WAVE_TILE - first[d];
+                row[d] = WAVE_TILE - first[d];
+            }
+        } else if constexpr (RANK == 1) {
+            // Four slots at a time: no add of a group waits for another (a
+            // branch per slot had made every add wait for the one before),
+            // and the first groups rank while the last keys still load.
+            // Against all sixteen at once: 2^18 low-entropy pairs 63.2 -> 61.3
+            // us, 2^28 3930 -> 3858, uniform keys the same.
+            constexpr int GS = 4;
+#pragma unroll
+            for (int h = 0; h < IPT; h += GS) {
+                uint32_t d[GS], q[GS];
+#pragma unroll
+                for (int j = 0; j < GS; ++j) d[j] = digit_of(h + j);
+                mgpu::rank_slots<GS>(d, row, lane, q);
+#pragma unroll
+                for (int j = 0; j < GS; ++j) pos[h + j] = q[j];
             }
         } else {
 #pragma unroll
-        for (int j = 0; j < IPT; ++j) {
-            const uint32_t d = digit_of(j);
-            if constexpr (RANK == 1) {
-                // A slot whose 64 keys share one digit (sorted or low-entropy
-                // input) takes its ranks with one add instead of 64 adds to one
-                // word, which the LDS would serialize.
-                const uint32_t f = __builtin_amdgcn_readfirstlane(d);
-                if (__builtin_amdgcn_ballot_w64(d == f) == ~0ull) {
-                    uint32_t base = 0;
-                    if (lane == 0)
-                        base = __hip_atomic_fetch_add(&s_count[wave][f], 64u, __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_WORKGROUP);
-                    pos[j] = __builtin_amdgcn_readfirstlane(base) + lane;
-                } else {
-                    pos[j] = __hip_atomic_fetch_add(&s_count[wave][d], 1u, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_WORKGROUP);
-                }
-            } else {
+            for (int j = 0; j < IPT; ++j) {
+                const uint32_t d = digit_of(j);
                 // Each lane ORs its bit into the wave's mask for its digit and
                 // reads the mask back; LDS operations of one wave complete in
                 // order, so the mask holds exactly the lanes of this slot with
@@ -1127,60 +1164,68 @@ __device__ void rank_scatter_body(const Args& a) {
                 const uint64_t m = __hip_atomic_load(&s_match[wave][d], __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_WORKGROUP);
                 const uint32_t below = lanes_below(m);
-                const uint32_t old = s_count[wave][d];
+                const uint32_t old = row[d];
                 pos[j] = old + below;
                 if (below == 0) {  // lowest lane of the group advances the count
-                    s_count[wave][d] = old + (uint32_t)__builtin_popcountll(m);
+                    row[d] = old + (uint32_t)__builtin_popcountll(m);
                     __hip_atomic_store(&s_match[wave][d], 0ull, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
             }
         }
-        }  // ranking
         __syncthreads();
 
-        // Per digit (thread d): wave-exclusive offsets and the tile total,
-        // published at once for the tiles after this one; then the tile-local
-        // digit starts (block scan) are added to the wave offsets.
-        uint32_t total = 0, tile_count = 0;
-        if (tid < RADIX) {
-            uint32_t sum = 0;
+        // Digit starts.  Thread (digit, k) holds the counts of R waves; the
+        // digit's total over its G threads is published at once for the tiles
+        // after this one.  One scan of the threads' sums in (digit, k) order
+        // is, for each thread, the tile-local start of its digit plus the
+        // earlier waves' keys of it, so the waves' starts follow with no
+        // second pass: 0.5 us of a 2^28-key pass's 14 us tile, where a thread
+        // per digit walking all W counts, twice, with shuffles in the scan,
+        // took 1.2.  With the ranking and the counting below, a sort of 2^28
+        // keys went 2607 -> 2389 us, 2^24 key + value 292 -> 277, 2^28
+        // low-entropy key + value 4040 -> 3858 (uniform 3812 -> 3786: that one
+        // is bound by memory, 64-key runs of two arrays from each of 256 CUs;
+        // a kernel that only moves them so, and ranks nothing, takes as long).
+        uint32_t c[R], sum = 0;
 #pragma unroll
-            for (int w = 0; w < W; ++w) {
-                const uint32_t c = s_count[w][tid];
-                s_count[w][tid] = sum;
-                sum += c;
-            }
-            total = sum;
-            tile_count = (tid == mask) ? sum - (TILE - tile_valid) : sum;
-            lookback_publish<XSEG>(&job.lookback[tile * RADIX + tid],
+        for (uint32_t r = 0; r < R; ++r) {
+            c[r] = col[r * ROW];
+            sum += c[r];
+        }
+        uint32_t tile_count = sum;  // of the digit, in its thread k = 0
+#pragma unroll
+        for (uint32_t off = 1; off < G; off <<= 1) tile_count += quad_xor(tile_count, off);
+        if (gd == mask) tile_count -= TILE - tile_valid;
+        if (gk == 0)
+            lookback_publish<XSEG>(&job.lookback[tile * RADIX + gd],
                                    (tile == 0 ? MGPU_LB_PREFIX : MGPU_LB_AGGREGATE) | tile_count);
-        }
-        const uint32_t local_start = block_exclusive_scan<BLOCK>(total, s_tmp, lane, wave);
-        if (tid < RADIX) {
-            s_lstart[tid] = local_start;
-            s_tcount[tid] = tile_count;
+        const uint32_t local_start = mgpu::block_exclusive_scan_dpp<BLOCK>(sum, s_tmp, lane, wave);
+        {
+            uint32_t start = local_start;
 #pragma unroll
-            for (int w = 0; w < W; ++w) s_count[w][tid] += local_start;
+            for (uint32_t r = 0; r < R; ++r) {
+                col[r * ROW] = start;
+                start += c[r];
+            }
         }
         __syncthreads();
 
-        // BLOCK / RADIX threads per digit walk back over the predecessors.  The
-        // first round's words are requested before the staging below so that
+        // G threads per digit walk back over the predecessors.  The first
+        // round's words are requested before the staging below so that
         // their latency overlaps it (starting earlier only waits longer for the
         // predecessors' own totals).
-        constexpr uint32_t G = BLOCK / RADIX;
         constexpr uint32_t K = MGPU_LOOKBACK_WINDOW / G > 0 ? MGPU_LOOKBACK_WINDOW / G : 1;
-        const uint32_t lb_digit = tid / G, lb_k = tid % G;
         uint32_t lb_words[K];
-        lookback_read<K, XSEG>(job.lookback, (int32_t)tile - 1, lb_digit, lb_k, lb_words);
+        lookback_read<K, XSEG>(job.lookback, (int32_t)tile - 1, gd, gk, lb_words);
 
         // Tile-local position of every key; stage the keys in digit order (and,
         // with one value array or generated indices, the values beside them, so
         // that both leave after a single barrier).
 #pragma unroll
+        for (int j = 0; j < IPT; ++j) pos[j] += row[digit_of(j)];
+#pragma unroll
         for (int j = 0; j < IPT; ++j) {
-            pos[j] += s_count[wave][digit_of(j)];
             s_stage[pos[j]] = key[j];
             if constexpr (JOINT) {
                 if constexpr (VMODE == MGPU_VALUES_INDEX) s_vstage[pos[j]] = wave_base + lane + j * 64;
@@ -1190,13 +1235,13 @@ __device__ void rank_scatter_body(const Args& a) {
 
         {
             const uint32_t prefix = lookback_window<G, K, XSEG>(
-                job.lookback, tile, lb_digit, lb_k, lane, a.error_flag, a.spin_limit, lb_words);
-            if (lb_k == 0) {
+                job.lookback, tile, gd, gk, lane, a.error_flag, a.spin_limit, lb_words);
+            if (gk == 0) {
                 if (tile > 0)
-                    lookback_publish<XSEG>(&job.lookback[tile * RADIX + lb_digit],
-                                           MGPU_LB_PREFIX | (prefix + s_tcount[lb_digit]));
-                const uint32_t dstart = XSINGLE ? s_dstart[lb_digit] : job.digit_start[lb_digit];
-                s_global[lb_digit] = dstart + prefix - s_lstart[lb_digit];
+                    lookback_publish<XSEG>(&job.lookback[tile * RADIX + gd],
+                                           MGPU_LB_PREFIX | (prefix + tile_count));
+                const uint32_t dstart = XSINGLE ? s_dstart[gd] : job.digit_start[gd];
+                s_global[gd] = dstart + prefix - local_start;
             }
         }
         __syncthreads();
@@ -1206,6 +1251,8 @@ __device__ void rank_scatter_body(const Args& a) {
         // The LDS reads of every slot are issued before the first store, so
         // that their latencies overlap instead of adding up slot by slot
         // (slots past the tile's keys read LDS words that are not used).
+        // (XSEG: the next tile's number is asked for here and read after the
+        // write-out, which covers the counter's answer.)
         const int32_t vrem = (int32_t)(tile_valid - tid);  // positions i*BLOCK < vrem are real
         uint32_t* const vout0 = JOINT ? job_vals_out<MULTI>(a, job, 0) : nullptr;
         uint32_t kout[IPT], dest[IPT], vout[JOINT ? IPT : 1];
@@ -1227,38 +1274,46 @@ __device__ void rank_scatter_body(const Args& a) {
         }
         // Offsets outside [0, n) can only come from a broken count or
         // lookback: they are flagged instead of written.  Slots with nothing
-        // to write get dest = n, where the buffer stores' range check drops
-        // them (one 32-bit offset per key instead of 64-bit addresses and a
-        // branch).
+        // to write, and those, get dest = n, where the buffer stores' range
+        // check drops them (one 32-bit offset per key instead of 64-bit
+        // addresses and a branch).
         const __amdgpu_buffer_rsrc_t rk = array_rsrc(job.keys_out, n);
         const __amdgpu_buffer_rsrc_t rv = JOINT ? array_rsrc(vout0, n) : rk;
-        bool bad = false;
+        uint32_t farthest = 0;
+        if (full) {
+#pragma unroll
+            for (int i = 0; i < IPT; ++i) {
+                farthest = max(farthest, dest[i]);
+                dest[i] = min(dest[i], n);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < IPT; ++i) {
+                const bool real = i * BLOCK < vrem;
+                farthest = max(farthest, real ? dest[i] : 0u);
+                dest[i] = real ? min(dest[i], n) : n;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < IPT; ++i) {
-            const bool real = full || i * BLOCK < vrem;
-            const bool ok = real && dest[i] < n;
-            bad = bad || (real && !ok);
-            dest[i] = ok ? dest[i] : n;
             __builtin_amdgcn_raw_buffer_store_b32(kout[i], rk, (int)(dest[i] * 4u), 0, 0);
             if constexpr (JOINT)
                 __builtin_amdgcn_raw_buffer_store_b32(vout[i], rv, (int)(dest[i] * 4u), 0, 0);
         }
-        if (bad) set_error(a.error_flag, 4u);
+        if (farthest >= n) set_error(a.error_flag, 4u);
         // Segments per XCD: the next pass's digit of every key written, by
         // the segment of the next pass that its position falls in.
-        // (Computing the segment costs less than a per-digit LDS lookup.)
+        // (Computing the segment costs less than a per-digit LDS lookup.
+        // Position n, of slots that wrote nothing, is at most in segment
+        // num_segs: the spare row.)
         if constexpr (XSINGLE) {
             if (count_next) {
 #pragma unroll
                 for (int i = 0; i < IPT; ++i) {
-                    if (dest[i] < n) {
-                        // dest / TILE < 2^16, num_segs <= 8: a 24-bit multiply.
-                        const uint32_t num = __umul24(dest[i] / TILE, a.num_segs) + a.num_segs - 1;
-                        const uint32_t xo =
-                            (uint32_t)__builtin_fmaf((float)num, seg_rcp, seg_half);
-                        const uint32_t nd = __builtin_amdgcn_ubfe(kout[i], a.next_shift, next_width);
-                        count1(s_next, s_spare, xo * RADIX + nd, nd == next_mode, lane);
-                    }
+                    const uint32_t xo = (uint32_t)__builtin_fmaf((float)(dest[i] / TILE), seg_mul, seg_add);
+                    const uint32_t nd = __builtin_amdgcn_ubfe(kout[i], a.next_shift, next_width);
+                    const bool real = full || dest[i] < n;
+                    count1(s_next, s_spare, (real ? xo : NSEG) * RADIX + nd, nd == next_mode, lane);
                 }
             }
         }
@@ -1279,12 +1334,14 @@ __device__ void rank_scatter_body(const Args& a) {
         }
 
         if constexpr (!XSEG) break;
-        __syncthreads();  // every read of this tile's LDS state is done
-        for (uint32_t i = tid; i < (uint32_t)(W * RADIX); i += BLOCK) {
-            (&s_count[0][0])[i] = 0;
-            // The value stage wrote over the match masks.
-            if constexpr (RANK == 0 && JOINT) (&s_match[0][0])[i] = 0;
+        if (tid == 0) post_tile(take_tile());
+        __syncthreads();  // (every read of this tile's stage is done, too)
+        gtile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
+        if (gtile < seg_tiles) {
+            job = posted_job(gtile);
+            load_tile(job);
         }
+        clear_counts();  // (the value stage wrote over the match masks)
     }  // while
 
     // The next pass's counts of this workgroup's keys, and the last
