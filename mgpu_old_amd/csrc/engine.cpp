@@ -186,7 +186,8 @@ sortStatus_t mgpu_lane_init(SortLane* l) {
     l->errorDev = static_cast<uint32_t*>(dev);
     l->reportWord = l->errorWord + kLaneReportOffset;
     l->reportDev = l->errorDev + kLaneReportOffset;
-    const size_t words = 2 * kLaneHistWords + MGPU_LANE_COUNTERS + kLaneSegCountWords;
+    const size_t words =
+        2 * kLaneHistWords + MGPU_LANE_COUNTERS + kLaneSegCountWords + kMidPlanWords;
     if (hipMalloc(&l->fixed, words * sizeof(uint32_t)) != hipSuccess) {
         l->fixed = nullptr;
         return SORT_STATUS_DEVICE_ALLOC_FAILED;
@@ -200,6 +201,7 @@ sortStatus_t mgpu_lane_init(SortLane* l) {
     l->digitStart = l->hist + kLaneHistWords;
     l->tileCounters = l->digitStart + kLaneHistWords;
     l->segCount = l->tileCounters + MGPU_LANE_COUNTERS;
+    l->midPlan = reinterpret_cast<mgpuMidPlan*>(l->segCount + kLaneSegCountWords);
     static_assert(MGPU_LANE_COUNTERS % 2 == 0 && kLaneHistWords % 2 == 0,
                   "segCount takes 64-bit atomics: it starts on an 8-byte boundary");
     l->histDirty = false;
@@ -327,37 +329,42 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
     } else if (keyType != SORT_KEYS_UINT32) {
         return SORT_STATUS_INVALID_VALUE;
     }
-    if (n <= kLocalSortMaxKeys && e->fnLocal && !(earlyExit && !L.noAlloc)) {
-        // One workgroup runs every pass in LDS and leaves the result on the
-        // side the passes would.
-        int totalBits = 0;
-        for (int p = 0; p < numPasses; ++p) totalBits += widths[p];
-        const int out = numPasses & 1;
+    if (L.noAlloc) earlyExit = false;
+    const int out = numPasses & 1;  // the side the passes leave the result on
+    int fieldBits = 0;
+    for (int p = 0; p < numPasses; ++p) fieldBits += widths[p];
+    // One workgroup's sort through every pass, of `in` side to `out` side.
+    auto local_args = [&](int in) {
         mgpuLocalArgs la;
         std::memset(&la, 0, sizeof(la));
-        la.keys_in = keyBuf[0];
+        la.keys_in = keyBuf[in];
         la.keys_out = keyBuf[out];
         const int carried = valueCount == -1 ? 1 : valueCount;
         for (int v = 0; v < carried; ++v) {
-            la.vals_in[v] = valBuf[v][0];
+            la.vals_in[v] = valBuf[v][in];
             la.vals_out[v] = valBuf[v][out];
         }
         la.n = n;
         la.first_bit = (uint32_t)firstBit;
-        la.num_bits = (uint32_t)totalBits;
-        la.vals_mode = valueCount == 0    ? MGPU_VALUES_NONE
-                       : valueCount == -1 ? MGPU_VALUES_INDEX
-                       : valueCount == 1  ? MGPU_VALUES_SINGLE
-                                          : MGPU_VALUES_MULTI;
+        la.num_bits = (uint32_t)fieldBits;
+        la.vals_mode = valueCount == 0                ? MGPU_VALUES_NONE
+                       : valueCount == -1 && in == 0  ? MGPU_VALUES_INDEX
+                       : valueCount == -1 || valueCount == 1 ? MGPU_VALUES_SINGLE
+                                                      : MGPU_VALUES_MULTI;
         la.num_values = (uint32_t)carried;
-        la.in_lo = toLo;
-        la.in_hi = toHi;
-        // Back: int32 flips the sign bit again; float32 flips the words
-        // whose top bit the mapping cleared.
+        // Keys back to their type: int32 flips the sign bit again; float32
+        // flips the words whose top bit the mapping cleared.
         la.out_lo = toHi;
         la.out_hi = toLo;
-        const sortStatus_t ls = mgpu_launch(e, L.stream, valueCount ? e->fnLocalPay : e->fnLocal, 1,
-                                            MGPU_LOCAL_THREADS, &la, !L.noAlloc);
+        return la;
+    };
+    hipFunction_t localFn = valueCount ? e->fnLocalPay : e->fnLocal;
+    if (n <= kLocalSortMaxKeys && localFn && !earlyExit) {
+        mgpuLocalArgs la = local_args(0);
+        la.in_lo = toLo;
+        la.in_hi = toHi;
+        const sortStatus_t ls =
+            mgpu_launch(e, L.stream, localFn, 1, MGPU_LOCAL_THREADS, &la, !L.noAlloc);
         if (!ls && executed) *executed = numPasses;
         return ls;
     }
@@ -384,7 +391,6 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
         // Scratch of a fixed size, filled by nothing that allocates or waits.
         if (lbWords > L.lookbackWords) return SORT_STATUS_CONFIG_NOT_SUPPORTED;
         if (L.histDirty) return SORT_STATUS_INTERNAL_ERROR;
-        earlyExit = false;
     } else {
         st = ensure_lookback(L, lbWords);
         if (st) return st;
@@ -402,6 +408,100 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
                 hipSuccess)
             return SORT_STATUS_DEVICE_ERROR;
         L.histDirty = false;
+    }
+
+    // Mid-sized arrays: counts, a scatter into buckets, and a workgroup's sort
+    // per bucket; the passes after the scatter are queued as well and return at
+    // once unless a bucket was too large for a workgroup, which the scatter
+    // finds from the counts on the device (then it is the first of them).
+    if (localFn && e->fnMidCount && var.mid[0] && segs == 1 && n <= kMidSortMaxKeys &&
+        numPasses > 2 && fieldBits >= MGPU_MID_BITS && widths[numPasses - 1] <= MGPU_MID_BITS &&
+        !earlyExit && (typedKeys == 0 || fused)) {
+        mgpuMidCountArgs ma;
+        std::memset(&ma, 0, sizeof(ma));
+        ma.keys = keyBuf[0];
+        ma.hist = L.hist;
+        ma.clear = L.lookback;
+        ma.clear_words = (lbWords + 3) & ~uint64_t(3);
+        ma.n = n;
+        ma.chunk = std::min(16384u, std::max(4096u, ((n + 63) / 64 + 1023) & ~1023u));
+        ma.vec_ok = (reinterpret_cast<uintptr_t>(keyBuf[0]) & 15) == 0;
+        ma.num_passes = (uint32_t)numPasses;
+        ma.bin_shift = (uint32_t)(firstBit + fieldBits - MGPU_MID_BITS);
+        ma.map_lo = toLo;
+        ma.map_hi = toHi;
+        ma.tile_counters = L.tileCounters;
+        ma.num_counters = MGPU_MODE_SLOT;
+        for (int p = 0, bit = firstBit; p < numPasses; bit += widths[p++]) {
+            ma.shift[p] = (uint32_t)bit;
+            ma.width[p] = (uint32_t)widths[p];
+        }
+        L.histDirty = true;
+        st = mgpu_launch(e, L.stream, e->fnMidCount, (n + ma.chunk - 1) / ma.chunk, 1024, &ma, timed);
+        if (st) return st;
+        const int carried = valueCount == -1 ? 1 : valueCount;
+        mgpuPassArgs pa;
+        std::memset(&pa, 0, sizeof(pa));
+        pa.num_values = (uint32_t)carried;
+        pa.error_flag = L.errorDev;
+        pa.spin_limit = e->spinLimit;
+        pa.n = n;
+        pa.num_tiles = numTiles;
+        pa.num_segs = 1;
+        pa.mid_plan = L.midPlan;
+        pa.mid_hist = L.hist;
+        pa.mid_starts = L.digitStart;
+        pa.mid_shift = ma.bin_shift;
+        pa.mid_target = std::max(kMidMinBucket, n / MGPU_RADIX + 1);
+        pa.mid_passes = (uint32_t)numPasses;
+        for (int p = 0; p < numPasses; ++p) pa.mid_field[p] = ma.shift[p] | ma.width[p] << 8;
+        const int firstMode = valueCount == 0    ? MGPU_VALUES_NONE
+                              : valueCount == -1 ? MGPU_VALUES_INDEX
+                              : valueCount == 1  ? MGPU_VALUES_SINGLE
+                                                 : MGPU_VALUES_MULTI;
+        const int laterMode = valueCount == -1 ? MGPU_VALUES_SINGLE : firstMode;
+        const bool oneLaunch = n <= kMidOneLaunchMaxKeys && var.midRest[laterMode];
+        auto pass = [&](int p, hipFunction_t f) {
+            const int in = p & 1;
+            pa.keys_in = keyBuf[in];
+            pa.keys_out = keyBuf[in ^ 1];
+            for (int v = 0; v < carried; ++v) {
+                pa.vals_in[v] = valBuf[v][in];
+                pa.vals_out[v] = valBuf[v][in ^ 1];
+            }
+            pa.digit_start = L.digitStart + p * MGPU_RADIX;
+            pa.lookback = L.lookback + (uint64_t)p * numTiles * MGPU_RADIX;
+            pa.tile_counter = L.tileCounters + MGPU_TILE_COUNTER(p, 0);
+            pa.finished = L.tileCounters + MGPU_FINISHED_SLOT;
+            pa.shift = ma.shift[p];
+            pa.mask = (1u << widths[p]) - 1u;
+            pa.key_types = p == 0 ? kernelKeyType
+                           : p == numPasses - 1 || oneLaunch ? kernelKeyType << 8
+                                                             : 0u;
+            return mgpu_launch(e, L.stream, f, numTiles, var.blockThreads, &pa, timed);
+        };
+        st = pass(0, var.mid[firstMode]);
+        if (st) return st;
+        mgpuLocalArgs la = local_args(1);
+        la.plan = L.midPlan;
+        la.hist = L.hist;
+        la.starts = L.digitStart;
+        la.num_passes = (uint32_t)numPasses;
+        la.last_width = (uint32_t)widths[numPasses - 1];
+        st = mgpu_launch(e, L.stream, localFn, MGPU_RADIX, MGPU_LOCAL_THREADS, &la, timed);
+        if (st) return st;
+        L.histDirty = false;
+        if (oneLaunch) {
+            st = pass(1, var.midRest[laterMode]);
+            if (st) return st;
+        } else {
+            for (int p = 1; p < numPasses; ++p) {
+                st = pass(p, var.midPass[laterMode]);
+                if (st) return st;
+            }
+        }
+        if (executed) *executed = numPasses;
+        return SORT_STATUS_SUCCESS;
     }
 
     // digit_count

@@ -36,6 +36,12 @@ struct PassVariant {
     // mgpu_rank_scatter_b*_i*_r1_km_v<mode> and ..._r1_x_km_v<mode>.
     hipFunction_t passKM[4] = {};
     hipFunction_t xsegKM[4] = {};
+    // Bucketed sorts: the first scatter by value mode, and a pass after it when
+    // the buckets do not fit, or all of them in one launch (no index form: they
+    // read the indices); null where not built.
+    hipFunction_t mid[4] = {};
+    hipFunction_t midPass[4] = {};
+    hipFunction_t midRest[4] = {};
     uint32_t xsegGrid = 0;        // workgroups of an xseg launch: all that fit on the device
     uint32_t tile() const { return blockThreads * itemsPerThread; }
 };
@@ -47,6 +53,9 @@ constexpr size_t kLaneHistWords = (size_t)MGPU_MAX_SEGS * MGPU_MAX_PASSES * MGPU
 // fills in (segments per XCD).
 constexpr size_t kLaneSegCountWords = (size_t)MGPU_MAX_PASSES * MGPU_XSEG_COUNT_SEGS * MGPU_RADIX;
 
+// Words of the plan of a bucketed sort, to a 256-byte boundary.
+constexpr size_t kMidPlanWords = (sizeof(mgpuMidPlan) / sizeof(uint32_t) + 63) & ~size_t(63);
+
 // One in-order queue of sorts: a stream plus the device scratch of the
 // device-wide passes.  The engine owns one (its default lane, on the stream
 // chosen with sortSetStream); the sort server owns one per in-flight batch.
@@ -57,6 +66,7 @@ struct SortLane {
     uint32_t* digitStart = nullptr;
     uint32_t* tileCounters = nullptr;
     uint32_t* segCount = nullptr;  // [MGPU_MAX_PASSES][MGPU_XSEG_COUNT_SEGS][MGPU_RADIX]
+    mgpuMidPlan* midPlan = nullptr;  // of a bucketed sort
     bool histDirty = false;  // hist/tileCounters may hold a partial sort's counts
     uint32_t* lookback = nullptr;  // grow-only
     uint64_t lookbackWords = 0;
@@ -123,6 +133,7 @@ struct sortEngine_d {
     // size).
     hipFunction_t fnLocal = nullptr;
     hipFunction_t fnLocalPay = nullptr;
+    hipFunction_t fnMidCount = nullptr;  // counts of a bucketed sort (null as above)
     hipFunction_t fnIota = nullptr;
     hipFunction_t fnKeyTransform = nullptr;
     hipFunction_t fnMultiCount = nullptr;      // 256 threads, per-wave histograms
@@ -219,6 +230,18 @@ const PassVariant& mgpu_pick_variant(const sortEngine_d* e, uint64_t keys);
 // still ahead of the device-wide passes there (16384 keys: 18.8 against 38.8
 // us, with one value 23.1 against 44.5, with three 38.9 against 56.0).
 constexpr uint32_t kLocalSortMaxKeys = MGPU_LOCAL_MAX_KEYS;
+// Larger arrays of up to this many keys, by more than two passes, are sorted in
+// buckets: evenly spread keys fill 256 buckets of n / 256 keys plus one bin of
+// n / 1024, which stay below MGPU_LOCAL_MAX_KEYS up to here.
+constexpr uint32_t kMidSortMaxKeys = 3u << 20;
+// The passes queued for keys whose buckets do not fit are one launch up to this
+// many keys, else a launch each.  One launch moves its data through the point
+// of coherence, which costs those passes 2% at 2^17 keys, 5% at 2^20 and 17% at
+// 3 * 2^20 (low-entropy key + value), and saves evenly spread keys the empty
+// launches (3 us each).
+constexpr uint32_t kMidOneLaunchMaxKeys = 1u << 19;
+// Keys of a bucket of bins, about.
+constexpr uint32_t kMidMinBucket = 1024;
 
 // Value classes of the sortArray tuning table.
 enum { MGPU_SORT_CLASS_KEYS = 0, MGPU_SORT_CLASS_INDEX = 1, MGPU_SORT_CLASS_KV = 2,

@@ -285,6 +285,8 @@ struct mgpuMultiPassArgs {
 // Parts (arrays) per packed tile of W waves.
 #define MGPU_PACK_MAX_PARTS(W) ((W) / 2)
 
+struct mgpuMidPlan;
+
 // rank_scatter: one stable digit pass (rank in the tile, decoupled lookback
 // across tiles, LDS-staged scatter).  With num_segs > 1 the workgroups of XCD
 // x take the tiles of segment x (kernels built for it only).
@@ -326,12 +328,29 @@ struct mgpuPassArgs {
     // type the keys it writes go back to (its last pass, which counts nothing
     // for a next one).  One word: the kernels run short of scalar registers.
     uint32_t key_types;
+    uint32_t pad_;
+    // Bucketed sort: the plan (its first scatter writes it, the launches of
+    // the passes after that return at once when it says that buckets are used),
+    // and for the first scatter the histogram of mid_count, the bin field and
+    // the bucket size.
+    // One launch of all of those passes reads side 1 first (keys_in, vals_in),
+    // tile_counter is the counter of its items and finished[p - 1] counts the
+    // tiles done of pass p.
+    mgpuMidPlan* mid_plan;
+    const uint32_t* mid_hist;
+    const uint32_t* mid_starts;   // [MGPU_MAX_PASSES][MGPU_RADIX]: digit starts, for one launch of all
+    uint32_t mid_shift;           // of the bins
+    uint32_t mid_target;
+    uint32_t mid_passes;
+    uint32_t pad2_;
+    uint32_t mid_field[MGPU_MAX_PASSES];  // each pass's shift | width << 8
 };
 
 // local_sort: one workgroup sorts an array of at most MGPU_LOCAL_MAX_KEYS keys
 // through every digit pass in LDS.
 #define MGPU_LOCAL_THREADS 1024
 #define MGPU_LOCAL_MAX_KEYS 16384
+struct mgpuMidPlan;
 struct mgpuLocalArgs {
     const uint32_t* keys_in;
     uint32_t* keys_out;           // may be keys_in
@@ -345,6 +364,53 @@ struct mgpuLocalArgs {
     // mgpu_key_map words applied to the keys as they are read and written.
     uint32_t in_lo, in_hi, out_lo, out_hi;
     uint32_t pad_;
+    // Bucketed sort: workgroup b sorts bucket b of the plan (nothing when the
+    // plan does not use buckets), and workgroup p < num_passes makes pass p's
+    // digit starts of mid_count's histogram and zeroes it.
+    const mgpuMidPlan* plan;
+    uint32_t* hist;
+    uint32_t* starts;        // [MGPU_MAX_PASSES][MGPU_RADIX]
+    uint32_t num_passes;
+    uint32_t last_width;     // of the last pass's digit
+};
+
+// Bucketed sort of mid-sized arrays: mid_count counts the top MGPU_MID_BITS
+// bits of the field (bins) and the digits of every pass but the last; the
+// first scatter (bucket_scatter) groups the bins into at most MGPU_RADIX
+// buckets of about `target` keys and, when every bucket fits a workgroup,
+// moves the keys to their bucket, which local_sort then finishes; otherwise it
+// is the first of the usual passes.
+#define MGPU_MID_BITS 10
+#define MGPU_MID_BINS (1 << MGPU_MID_BITS)
+// Histogram words: the bins, then 256 counts a pass.
+#define MGPU_MID_HIST_WORDS (MGPU_MID_BINS + MGPU_MAX_PASSES * MGPU_RADIX)
+struct mgpuMidCountArgs {
+    const uint32_t* keys;
+    uint32_t* hist;          // [MGPU_MID_HIST_WORDS], zero on entry
+    uint32_t* clear;         // words zeroed on the way (the lookback words)
+    uint64_t clear_words;    // multiple of 4
+    uint32_t n;
+    uint32_t chunk;          // keys per workgroup, multiple of 4
+    uint32_t vec_ok;         // keys pointer is 16-byte aligned
+    uint32_t num_passes;
+    uint32_t bin_shift;
+    uint32_t map_lo, map_hi; // mgpu_key_map words
+    uint32_t num_counters;
+    uint32_t* tile_counters; // [num_counters] -> zeroed
+    uint32_t shift[MGPU_MAX_PASSES];
+    uint32_t width[MGPU_MAX_PASSES];
+};
+
+// What bucket_scatter leaves for the launches after it: whether buckets are
+// used, and each bucket's first output position, what to take off its keys and
+// the bits, from the field's first one up, that are left to sort by.
+struct mgpuMidPlan {
+    uint32_t buckets;  // 1: local_sort finishes; 0: the digit passes go on
+    uint32_t pad_[3];
+    uint32_t start[MGPU_RADIX + 1];
+    uint32_t base[MGPU_RADIX];
+    uint32_t bits[MGPU_RADIX];
+    uint32_t pad2_[3];
 };
 
 // Segments per XCD with counting for the next pass: at most this many.

@@ -79,6 +79,29 @@ sortStatus_t load_variant(sortEngine_d* e, uint32_t threads, uint32_t items, uin
         e->kernelNames[f] = name;
         e->kernelNames[fx] = namex;
     }
+    // Bucketed-sort forms, likewise.
+    for (int m = 0; m < 4 && rank == 1; ++m) {
+        char name[96];
+        hipFunction_t f = nullptr;
+        std::snprintf(name, sizeof(name), "mgpu_rank_scatter_b%u_i%u_r1_m_v%d", threads, items, m);
+        if (hipModuleGetFunction(&f, e->radixModule, name) != hipSuccess) break;
+        v->mid[m] = f;
+        e->kernelNames[f] = name;
+        if (m == MGPU_VALUES_INDEX) continue;
+        std::snprintf(name, sizeof(name), "mgpu_rank_scatter_b%u_i%u_r1_c_v%d", threads, items, m);
+        if (hipModuleGetFunction(&f, e->radixModule, name) != hipSuccess) {
+            v->mid[m] = nullptr;
+            break;
+        }
+        v->midPass[m] = f;
+        e->kernelNames[f] = name;
+        std::snprintf(name, sizeof(name), "mgpu_rank_scatter_b%u_i%u_r1_f_v%d", threads, items, m);
+        if (hipModuleGetFunction(&f, e->radixModule, name) != hipSuccess) continue;
+        v->midRest[m] = f;
+        e->kernelNames[f] = name;
+    }
+    if (!v->mid[MGPU_VALUES_MULTI])
+        for (int m = 0; m < 4; ++m) v->mid[m] = v->midPass[m] = nullptr;
     // Packed multi-array forms, likewise.
     bool packed = rank == 1;
     for (int m = 0; m < 4 && packed; ++m) {
@@ -244,6 +267,7 @@ sortStatus_t mgpu_engine_load(sortEngine_d* e) {
     if (e->rankMethod == 1 && !e->xcdForce && !(t && *t)) {
         st = get_fn(e, e->radixModule, "mgpu_local_sort_k", &e->fnLocal);
         if (!st) st = get_fn(e, e->radixModule, "mgpu_local_sort_kv", &e->fnLocalPay);
+        if (!st) st = get_fn(e, e->radixModule, "mgpu_mid_count", &e->fnMidCount);
         if (st) return st;
     }
     const char* spin = std::getenv("MGPUSORT_SPIN_LIMIT");

@@ -21,14 +21,16 @@ namespace {
 
 // Layout of `scratch`, in 32-bit words: histograms and digit starts of up to
 // MGPU_MAX_SEGS segments, the tile counters (padded to 256 words), the
-// per-segment counts of each pass, then the lookback words: 4 passes of
+// per-segment counts of each pass, the plan of a bucketed sort, then the
+// lookback words: 4 passes of
 // 256 words per tile for SORT_NOALLOC_MAX_ELEMENTS keys in tiles of 8192 (the
 // smaller of the engine's two tile shapes).
 constexpr size_t kHistOff = 0;
 constexpr size_t kStartOff = kHistOff + kLaneHistWords;
 constexpr size_t kCounterOff = kStartOff + kLaneHistWords;
 constexpr size_t kSegCountOff = kCounterOff + 256;
-constexpr size_t kLookbackOff = kSegCountOff + kLaneSegCountWords;
+constexpr size_t kMidPlanOff = kSegCountOff + kLaneSegCountWords;
+constexpr size_t kLookbackOff = kMidPlanOff + kMidPlanWords;
 constexpr size_t kLookbackWords =
     (size_t)MGPU_MAX_PASSES * ((size_t)SORT_NOALLOC_MAX_ELEMENTS / 8192) * MGPU_RADIX;
 constexpr size_t kScratchWords = kLookbackOff + kLookbackWords;
@@ -91,6 +93,7 @@ sortStatus_t SORTAPI sortArrayNoAlloc(sortEngine_t engine, sortData_t data) {
     v.digitStart = ptr + kStartOff;
     v.tileCounters = ptr + kCounterOff;
     v.segCount = ptr + kSegCountOff;
+    v.midPlan = reinterpret_cast<mgpuMidPlan*>(ptr + kMidPlanOff);
     v.lookback = ptr + kLookbackOff;
     v.lookbackWords = kLookbackWords;
     v.errorWord = engine->lane.errorWord;

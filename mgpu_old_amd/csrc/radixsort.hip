@@ -406,6 +406,98 @@ __device__ void digit_count_body(const mgpuCountArgs& a) {
 }
 
 // ---------------------------------------------------------------------------
+// mid_count: the counts of a bucketed sort: the bins of the field's top
+// MGPU_MID_BITS bits and the digits of every pass but the last (whose digits
+// are sums of bins), in one read.  Also zeroes the lookback words.  One LDS
+// histogram per workgroup in MID_COPIES copies, by lane, so that equal digits
+// of neighbouring lanes hit different words (2^20 low-entropy keys: 4 copies
+// 74.8 us a sort, 16 copies 70.5; evenly spread ones pay 1 us for clearing and
+// adding up the copies).
+constexpr uint32_t MID_COPIES = 16;
+template <int BLOCK>
+__device__ void mid_count_body(const mgpuMidCountArgs& a) {
+    __shared__ __attribute__((aligned(16))) uint32_t s_hist[MGPU_MID_HIST_WORDS * MID_COPIES];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t words = MGPU_MID_BINS + (a.num_passes - 1) * RADIX;
+    for (uint32_t i = tid; i < words * MID_COPIES / 4; i += BLOCK)
+        reinterpret_cast<uint4*>(s_hist)[i] = make_uint4(0u, 0u, 0u, 0u);
+    {
+        uint4* c = reinterpret_cast<uint4*>(a.clear);
+        const uint64_t nvec = a.clear_words >> 2;
+        for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + tid; i < nvec;
+             i += (uint64_t)gridDim.x * BLOCK)
+            c[i] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    if (blockIdx.x == 0 && tid < a.num_counters) a.tile_counters[tid] = 0;
+    const uint32_t begin = min(a.n, blockIdx.x * a.chunk), end = min(a.n, begin + a.chunk);
+    uint32_t* const mine = s_hist + (tid & (MID_COPIES - 1));
+    auto add = [&](uint32_t w, uint32_t v) {
+        __hip_atomic_fetch_add(&mine[w * MID_COPIES], v, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    auto count = [&](uint32_t k) {
+        k = mgpu_key_map(k, a.map_lo, a.map_hi);
+        add(__builtin_amdgcn_ubfe(k, a.bin_shift, MGPU_MID_BITS), 1u);
+#pragma unroll
+        for (int p = 0; p < MGPU_MAX_PASSES - 1; ++p)
+            if ((uint32_t)p + 1 < a.num_passes)
+                add(MGPU_MID_BINS + p * RADIX + __builtin_amdgcn_ubfe(k, a.shift[p], a.width[p]), 1u);
+    };
+    __syncthreads();
+    uint32_t done = begin;
+    if (a.vec_ok) {
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        const u32x4* v = reinterpret_cast<const u32x4*>(a.keys + begin);
+        const uint32_t nvec = (end - begin) >> 2;
+        for (uint32_t i0 = tid; i0 < nvec; i0 += 4 * BLOCK) {
+            u32x4 q[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (i0 + u * BLOCK < nvec) q[u] = v[i0 + u * BLOCK];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (i0 + u * BLOCK >= nvec) break;
+                // Equal keys in every lane (constant input): one add a word.
+                const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)q[u].x);
+                const uint64_t exec = __builtin_amdgcn_read_exec();
+                const bool same = q[u].x == f && q[u].y == f && q[u].z == f && q[u].w == f;
+                if (__builtin_amdgcn_ballot_w64(same) == exec) {
+                    if (lanes_below(exec) == 0) {
+                        const uint32_t m = 4u * (uint32_t)__builtin_popcountll(exec);
+                        const uint32_t k = mgpu_key_map(f, a.map_lo, a.map_hi);
+                        add(__builtin_amdgcn_ubfe(k, a.bin_shift, MGPU_MID_BITS), m);
+                        for (uint32_t p = 0; p + 1 < a.num_passes; ++p)
+                            add(MGPU_MID_BINS + p * RADIX +
+                                    __builtin_amdgcn_ubfe(k, a.shift[p], a.width[p]), m);
+                    }
+                    continue;
+                }
+                count(q[u].x);
+                count(q[u].y);
+                count(q[u].z);
+                count(q[u].w);
+            }
+        }
+        done = begin + 4 * nvec;
+    }
+    for (uint32_t i = done + tid; i < end; i += BLOCK) count(a.keys[i]);
+    __syncthreads();
+    for (uint32_t i = tid; i < words; i += BLOCK) {
+        uint32_t sum = 0;
+#pragma unroll
+        for (uint32_t c = 0; c < MID_COPIES / 4; ++c) {
+            // (Starting at a copy of its own, a thread reads other banks than
+            // its neighbours.)
+            const uint4 q = reinterpret_cast<const uint4*>(
+                s_hist)[i * (MID_COPIES / 4) + ((c + i) & (MID_COPIES / 4 - 1))];
+            sum += q.x + q.y + q.z + q.w;
+        }
+        if (sum)
+            __hip_atomic_fetch_add(&a.hist[i], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // digit_scan: one workgroup of 256 threads per pass (workgroup p: pass p;
 // thread d: digit d).  A pass's output holds the digits in order and, within
 // a digit, the segments in order: run (x, d) starts at the keys of smaller
@@ -873,14 +965,154 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t array_rsrc(const uint32_t* p, 
                                              kBufferDword3);
 }
 
-template <int IPT>
+// Cache policy (sc1) of accesses that other XCDs' workgroups of the same launch
+// must see, or whose data they wrote: loads past this XCD's L2, stores through
+// it, as agent-scope atomics have it.
+constexpr int kCoherentAux = 16;
+
+template <int IPT, int AUX = kTileLoadAux>
 __device__ __forceinline__ void load_striped(const uint32_t* src, uint32_t n, uint32_t wave_base,
                                              uint32_t lane, uint32_t* out) {
     const __amdgpu_buffer_rsrc_t r = array_rsrc(src, n);
     const uint32_t off = (wave_base + lane) * 4u;
 #pragma unroll
     for (int j = 0; j < IPT; ++j)
-        out[j] = __builtin_amdgcn_raw_buffer_load_b32(r, (int)(off + j * 256u), 0, kTileLoadAux);
+        out[j] = __builtin_amdgcn_raw_buffer_load_b32(r, (int)(off + j * 256u), 0, AUX);
+}
+
+// A bucketed sort takes a scatter and one workgroup's sort per bucket where the
+// digit passes take a scatter each, all of them bound by latency at these
+// sizes (10-12 us a launch).  Digit passes -> buckets, a sort with the fill of
+// its input: 20001 pairs 47.4 -> 26.4 us, 150000 51.1 -> 27.7, 2^19 61.0 ->
+// 35.0, 1000003 74.4 -> 46.7, 3000001 96.2 -> 66.8; normal floats 150000
+// 53.3 -> 42.5.  Keys that no grouping spreads: 1.0-1.08x up to 2^20 keys, at
+// 3000001 112 against 108 us (the counts and the empty bucket launch).
+//
+// The digits of a bucketed sort's first scatter, worked out by every workgroup
+// from the counts while its keys load (1024 bins: a few KB from the L2 and a
+// scan; a launch of its own would cost as much).  A bucket is 4 bins, that is
+// the field's top 8 bits, when no such digit exceeds what one workgroup sorts:
+// the bits below are then whole digits.  Else (skewed keys, as normal floats)
+// the bins are grouped by their counts: the bucket of a bin is the keys before
+// it over `target`, so a bucket holds less than target keys plus its last
+// bin's.  Else, where every key has the same last digit (small numbers in wide
+// keys), the digit below is tried, down to the second one: a bucket is then a
+// value of the highest digit that is not constant.  When a bucket is still too
+// large, the digits are the first pass's.
+// s_start: each digit's first output position; shift, width: the field that is
+// the digit or, when the result is true, the bin whose digit s_map holds; mask:
+// the digit of the padding keys (all ones) of the last tile.  s_work: at least
+// 3 * RADIX words.  c: this thread's bins, digit0: its first-pass digit's count (both read by the
+// caller ahead of the tile's loads, whose return they would otherwise wait
+// for).
+template <int BLOCK>
+__device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MID_BINS / BLOCK],
+                              uint32_t digit0, uint32_t* s_map, uint32_t* s_start,
+                              uint32_t* s_tmp, uint32_t* s_work, uint32_t& shift, uint32_t& width,
+                              uint32_t& mask) {
+    constexpr uint32_t PER = MGPU_MID_BINS / BLOCK;  // consecutive bins a thread holds
+    constexpr uint32_t GROUP = MGPU_MID_BINS / RADIX, LANES = GROUP / PER;
+    static_assert(LANES == 2 || LANES == 4, "a group of bins is held by neighbouring lanes");
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const bool last_group = blockIdx.x + 1 == gridDim.x;
+    const uint32_t field_shift = a.mid_field[0] & 0xFFu;
+    auto put_plan = [&](uint32_t b, uint32_t start, uint32_t base, uint32_t bits) {
+        a.mid_plan->start[b] = start;
+        a.mid_plan->base[b] = base;
+        a.mid_plan->bits[b] = bits;
+    };
+    uint32_t sum = 0, most = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < PER; ++i) {
+        sum += c[i];
+        most = max(most, c[i]);
+    }
+    uint32_t group = sum;
+#pragma unroll
+    for (uint32_t off = 1; off < LANES; off <<= 1) group += quad_xor(group, off);
+    uint32_t before = mgpu::block_exclusive_scan_dpp<BLOCK>(sum, s_tmp, lane, wave);
+    if (last_group && tid == 0) a.mid_plan->start[RADIX] = a.n;
+    if (__syncthreads_and(group <= MGPU_LOCAL_MAX_KEYS)) {
+        const uint32_t g = tid / LANES;
+        if (tid % LANES == 0) {
+            s_start[g] = before;
+            if (last_group)
+                put_plan(g, before, g * GROUP << a.mid_shift, a.mid_shift - field_shift + 2);
+        }
+        if (last_group && tid == 0) a.mid_plan->buckets = 1;
+        shift = a.mid_shift + MGPU_MID_BITS - MGPU_RADIX_BITS;
+        width = MGPU_RADIX_BITS;
+        mask = RADIX - 1;
+        __syncthreads();
+        return false;
+    }
+    uint32_t* const s_keys = s_work;              // keys of each bucket
+    uint32_t* const s_first = s_work + RADIX;     // its first bin
+    uint32_t* const s_bins = s_work + 2 * RADIX;  // the bin after its last
+    bool fits = __syncthreads_and(most <= MGPU_LOCAL_MAX_KEYS) != 0;
+    bool one = __syncthreads_or(group == a.n) != 0;
+    int digit = -1;  // the digit whose values are the buckets; -1: bins
+    uint32_t digit_shift = a.mid_shift, keys = 0;
+    if (fits) {
+        if (tid < RADIX) {
+            s_keys[tid] = 0;
+            s_first[tid] = MGPU_MID_BINS;
+            s_bins[tid] = 0;
+        }
+        __syncthreads();
+        // Quotients by one float reciprocal, corrected by one step: before <
+        // 2^24.
+        const float rcp = 1.0f / (float)a.mid_target;
+#pragma unroll
+        for (uint32_t i = 0; i < PER; ++i) {
+            uint32_t b = (uint32_t)((float)before * rcp);
+            if ((b + 1) * a.mid_target <= before) ++b;
+            else if (b * a.mid_target > before) --b;
+            s_map[tid * PER + i] = b;
+            if (c[i]) {  // an empty bin belongs to no bucket
+                atomicAdd(&s_keys[b], c[i]);
+                atomicMin(&s_first[b], tid * PER + i);
+                atomicMax(&s_bins[b], tid * PER + i + 1);
+            }
+            before += c[i];
+        }
+        __syncthreads();
+        keys = tid < RADIX ? s_keys[tid] : 0u;
+        fits = __syncthreads_and(keys <= MGPU_LOCAL_MAX_KEYS) != 0;
+    }
+    for (int p = (int)a.mid_passes - 2; one && !fits && p > 0; --p) {
+        // One top value: the digit below, while that is not constant too.
+        keys = tid < RADIX ? a.mid_hist[MGPU_MID_BINS + p * RADIX + tid] : 0u;
+        fits = __syncthreads_and(keys <= MGPU_LOCAL_MAX_KEYS) != 0;
+        one = __syncthreads_or(keys == a.n) != 0;
+        if (fits) {
+            digit = p;
+            digit_shift = a.mid_field[p] & 0xFFu;
+        }
+    }
+    if (last_group && tid == 0) a.mid_plan->buckets = fits ? 1u : 0u;
+    const uint32_t start =
+        mgpu::block_exclusive_scan_dpp<BLOCK>(fits ? keys : digit0, s_tmp, lane, wave);
+    if (tid < RADIX) {
+        s_start[tid] = start;
+        if (last_group && fits) {
+            // The keys of a bucket of bins lie above its first bin, and the
+            // bits that number its bins are left to sort by; the keys of a
+            // digit's bucket differ below the digit only.
+            const uint32_t first = s_first[tid], bins = s_bins[tid] - first;
+            uint32_t bits = digit_shift - field_shift;
+            if (digit < 0 && keys && bins > 1) bits += 32u - (uint32_t)__builtin_clz(bins - 1);
+            put_plan(tid, start, digit < 0 ? first << digit_shift : 0u, bits);
+        }
+    }
+    __syncthreads();
+    if (fits) {
+        shift = digit_shift;
+        width = digit < 0 ? MGPU_MID_BITS : a.mid_field[digit] >> 8;
+        mask = digit < 0 ? s_map[MGPU_MID_BINS - 1] : (1u << width) - 1u;
+    }
+    return fits && digit < 0;
 }
 
 // RANK 0: in-wave ranking by LDS match masks (documented behaviour only).
@@ -900,9 +1132,23 @@ __device__ __forceinline__ void load_striped(const uint32_t* src, uint32_t n, ui
 // per wave instead of per block in a count kernel).  Its keys then stage to
 // consecutive LDS words, free of bank conflicts; a tile whose waves all are in
 // order, and in order across waves, stages every key to its own place.
+// MID (a bucketed sort of one array): 1 is its first scatter, whose digits are
+// buckets looked up by the key's bin when the counts allow it, else the first
+// pass's digits; 2 is a pass after it, which returns at once when buckets were
+// used; 3 is all of those passes in one launch (returning at once costs ~3 us a
+// launch).  Its work items, (pass, tile) in order, come from one counter; an item waits
+// for the pass before it to be complete, that is for items handed out earlier
+// to workgroups that run, so no number of resident workgroups is needed.  Data
+// goes between XCDs inside the launch: loads and stores are coherent ones.
 template <int BLOCK, int IPT, int RANK, int VMODE, bool MULTI, bool XSEG, bool EE, bool KMAP,
-          typename Args>
+          int MID, typename Args>
 __device__ void rank_scatter_body(const Args& a) {
+    static_assert(MID == 0 || (RANK == 1 && !MULTI && !XSEG && !EE), "one array, one chain");
+    if constexpr (MID == 2 || MID == 3) {
+        if (a.mid_plan->buckets) return;
+    }
+    constexpr int LAUX = MID == 3 ? kCoherentAux : kTileLoadAux;
+    constexpr int SAUX = MID == 3 ? kCoherentAux : 0;
     static_assert(!EE || RANK == 1, "early exit builds on the atomic-add ranking");
     static_assert(!(EE && MULTI), "early exit is for single arrays");
     constexpr bool XSINGLE = XSEG && !MULTI;  // one array cut into segments per XCD
@@ -945,8 +1191,9 @@ __device__ void rank_scatter_body(const Args& a) {
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const uint32_t shift = a.shift, mask = a.mask;
-    const uint32_t width = (uint32_t)__builtin_popcount(mask);  // mask = 2^width - 1
+    uint32_t shift = a.shift, mask = a.mask;
+    uint32_t width = (uint32_t)__builtin_popcount(mask);  // mask = 2^width - 1
+    __shared__ uint32_t s_map[MID == 1 ? MGPU_MID_BINS : 1];  // bin (or digit) -> digit
     uint32_t* const row = s_count[wave];  // this wave's digit counts
     const uint32_t gd = tid / G, gk = tid % G;
     uint32_t* const col = &s_count[gk * R][gd];
@@ -1050,23 +1297,94 @@ __device__ void rank_scatter_body(const Args& a) {
     uint32_t key[IPT], val[IPT];
     // Keys and the single value array of a tile, striped, requested together:
     // ranking starts once the keys are in while the values still load.
+    uint32_t pass = 0;  // MID 3: the item's pass, odd ones from side 1 to side 0
+    auto vals_in = [&](const TileJob& job, uint32_t v) -> const uint32_t* {
+        if constexpr (MID == 3) return pass & 1 ? a.vals_in[v] : a.vals_out[v];
+        else return job_vals_in<MULTI>(a, job, v);
+    };
+    auto vals_out = [&](const TileJob& job, uint32_t v) -> uint32_t* {
+        if constexpr (MID == 3) return pass & 1 ? a.vals_out[v] : const_cast<uint32_t*>(a.vals_in[v]);
+        else return job_vals_out<MULTI>(a, job, v);
+    };
     auto load_tile = [&](const TileJob& job) {
         const uint32_t wave_base = (job.first + job.tile) * TILE + wave * WAVE_TILE;
-        load_striped<IPT>(job.keys_in, job.n, wave_base, lane, key);
+        load_striped<IPT, LAUX>(job.keys_in, job.n, wave_base, lane, key);
         if constexpr (VMODE == MGPU_VALUES_SINGLE)
-            load_striped<IPT>(job_vals_in<MULTI>(a, job, 0), job.n, wave_base, lane, val);
+            load_striped<IPT, LAUX>(vals_in(job, 0), job.n, wave_base, lane, val);
+    };
+    uint32_t key_types = 0;
+    if constexpr (KMAP) key_types = a.key_types;
+    // MID 3: the next item, once the pass before its own is complete.
+    auto take_item = [&](TileJob& job) -> bool {
+        if constexpr (MID == 3) {
+        const uint32_t items = a.num_tiles * (a.mid_passes - 1);
+        if (tid == 0) {
+            const uint32_t t = __hip_atomic_fetch_add(a.tile_counter, 1u, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+            s_tile[0] = t;
+            const uint32_t p = t / a.num_tiles;  // passes of the launch before it
+            if (t < items && p > 0) {
+                uint32_t spins = 0;
+                while (ld_agent(a.finished + p - 1) < a.num_tiles) {
+                    if (++spins > a.spin_limit) {
+                        set_error(a.error_flag, 1u);
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(1);
+                }
+            }
+        }
+        __syncthreads();
+        const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
+        if (t >= items) return false;
+        const uint32_t p = t / a.num_tiles;
+        pass = p + 1;
+        job.tile = t - p * a.num_tiles;
+        job.n = a.n;
+        job.first = 0;
+        job.sd = nullptr;
+        job.keys_in = pass & 1 ? a.keys_in : a.keys_out;
+        job.keys_out = pass & 1 ? a.keys_out : const_cast<uint32_t*>(a.keys_in);
+        job.digit_start = a.mid_starts + pass * RADIX;
+        job.lookback = a.lookback + (size_t)p * a.num_tiles * RADIX;
+        shift = a.mid_field[pass] & 0xFFu;
+        width = a.mid_field[pass] >> 8;
+        mask = (1u << width) - 1u;
+        key_types = pass + 1 == a.mid_passes ? a.key_types : 0u;
+        load_tile(job);
+        return true;
+        } else {
+            (void)job;
+            return false;
+        }
     };
 
-    if (tid == 0) post_tile(take_tile());
-    __syncthreads();
-    uint32_t gtile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
-    // One tile per workgroup: only a counter left dirty finds none.
-    if (!XSEG && gtile >= seg_tiles && tid == 0) set_error(a.error_flag, 2u);
-    TileJob job{};
-    if (gtile < seg_tiles) {
-        job = posted_job(gtile);
-        load_tile(job);
+    constexpr uint32_t MID_PER = MID == 1 ? MGPU_MID_BINS / BLOCK : 1;
+    uint32_t mid_bins[MID_PER], mid_digit0 = 0;
+    bool mapped = false;  // MID 1: digits are looked up in s_map
+    if constexpr (MID == 1) {
+#pragma unroll
+        for (uint32_t i = 0; i < MID_PER; ++i) mid_bins[i] = a.mid_hist[tid * MID_PER + i];
+        if (tid < RADIX) mid_digit0 = a.mid_hist[MGPU_MID_BINS + tid];
     }
+    TileJob job{};
+    uint32_t gtile;
+    if constexpr (MID == 3) {
+        gtile = take_item(job) ? 0u : seg_tiles;
+    } else {
+        if (tid == 0) post_tile(take_tile());
+        __syncthreads();
+        gtile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
+        // One tile per workgroup: only a counter left dirty finds none.
+        if (!XSEG && gtile >= seg_tiles && tid == 0) set_error(a.error_flag, 2u);
+        if (gtile < seg_tiles) {
+            job = posted_job(gtile);
+            load_tile(job);
+        }
+    }
+    if constexpr (MID == 1)
+        mapped = mid_plan_tile<BLOCK>(a, mid_bins, mid_digit0, s_map, s_global, s_tmp, s_stage, shift, width,
+                             mask);
     while (gtile < seg_tiles) {
         const uint32_t n = job.n, tile = job.tile;
         const uint32_t base = (job.first + tile) * TILE;
@@ -1076,7 +1394,7 @@ __device__ void rank_scatter_body(const Args& a) {
         // Signed or float keys (KMAP), in the sort's first pass: to their
         // unsigned order.
         if constexpr (KMAP) {
-            const uint32_t tin = a.key_types & 0xFFu;
+            const uint32_t tin = key_types & 0xFFu;
             if (tin != 0) {
 #pragma unroll
                 for (int j = 0; j < IPT; ++j) key[j] = mgpu_key_to_radix(key[j], tin);
@@ -1091,7 +1409,19 @@ __device__ void rank_scatter_body(const Args& a) {
 #pragma unroll
             for (int j = 0; j < IPT; ++j) key[j] = j * 64 < rem ? key[j] : 0xFFFFFFFFu;
         }
-        auto digit_of = [&](int j) -> uint32_t { return __builtin_amdgcn_ubfe(key[j], shift, width); };
+        uint32_t dig[MID == 1 ? IPT : 1];
+        if constexpr (MID == 1) {
+#pragma unroll
+            for (int j = 0; j < IPT; ++j) dig[j] = __builtin_amdgcn_ubfe(key[j], shift, width);
+            if (mapped) {
+#pragma unroll
+                for (int j = 0; j < IPT; ++j) dig[j] = s_map[dig[j]];
+            }
+        }
+        auto digit_of = [&](int j) -> uint32_t {
+            if constexpr (MID == 1) return dig[j];
+            else return __builtin_amdgcn_ubfe(key[j], shift, width);
+        };
 
         // Rank within the wave: pos[j] = earlier same-digit keys of this wave.
         uint32_t pos[IPT];
@@ -1240,7 +1570,10 @@ __device__ void rank_scatter_body(const Args& a) {
                 if (tile > 0)
                     lookback_publish<XSEG>(&job.lookback[tile * RADIX + gd],
                                            MGPU_LB_PREFIX | (prefix + tile_count));
-                const uint32_t dstart = XSINGLE ? s_dstart[gd] : job.digit_start[gd];
+                uint32_t dstart;
+                if constexpr (XSINGLE) dstart = s_dstart[gd];
+                else if constexpr (MID == 1) dstart = s_global[gd];
+                else dstart = job.digit_start[gd];
                 s_global[gd] = dstart + prefix - local_start;
             }
         }
@@ -1254,19 +1587,22 @@ __device__ void rank_scatter_body(const Args& a) {
         // (XSEG: the next tile's number is asked for here and read after the
         // write-out, which covers the counter's answer.)
         const int32_t vrem = (int32_t)(tile_valid - tid);  // positions i*BLOCK < vrem are real
-        uint32_t* const vout0 = JOINT ? job_vals_out<MULTI>(a, job, 0) : nullptr;
+        uint32_t* const vout0 = JOINT ? vals_out(job, 0) : nullptr;
         uint32_t kout[IPT], dest[IPT], vout[JOINT ? IPT : 1];
 #pragma unroll
         for (int i = 0; i < IPT; ++i) kout[i] = s_stage[i * BLOCK + tid];
 #pragma unroll
         for (int i = 0; i < IPT; ++i) {
-            dest[i] = s_global[__builtin_amdgcn_ubfe(kout[i], shift, width)] + i * BLOCK + tid;
+            uint32_t d = __builtin_amdgcn_ubfe(kout[i], shift, width);
+            if constexpr (MID == 1)
+                if (mapped) d = s_map[d];
+            dest[i] = s_global[d] + i * BLOCK + tid;
             if constexpr (JOINT) vout[i] = s_vstage[i * BLOCK + tid];
         }
         // Signed or float keys (KMAP), in the sort's last pass: back to their
         // type (no pass after it reads their digits).
         if constexpr (KMAP) {
-            const uint32_t tout = a.key_types >> 8;
+            const uint32_t tout = key_types >> 8;
             if (tout != 0) {
 #pragma unroll
                 for (int i = 0; i < IPT; ++i) kout[i] = mgpu_key_from_radix(kout[i], tout);
@@ -1296,9 +1632,9 @@ __device__ void rank_scatter_body(const Args& a) {
         }
 #pragma unroll
         for (int i = 0; i < IPT; ++i) {
-            __builtin_amdgcn_raw_buffer_store_b32(kout[i], rk, (int)(dest[i] * 4u), 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(kout[i], rk, (int)(dest[i] * 4u), 0, SAUX);
             if constexpr (JOINT)
-                __builtin_amdgcn_raw_buffer_store_b32(vout[i], rv, (int)(dest[i] * 4u), 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(vout[i], rv, (int)(dest[i] * 4u), 0, SAUX);
         }
         if (farthest >= n) set_error(a.error_flag, 4u);
         // Segments per XCD: the next pass's digit of every key written, by
@@ -1321,18 +1657,34 @@ __device__ void rank_scatter_body(const Args& a) {
         // Two or more value arrays: one after the other through the key stage.
         if constexpr (VMODE == MGPU_VALUES_MULTI) {
             for (uint32_t v = 0; v < a.num_values; ++v) {
-                load_striped<IPT>(job_vals_in<MULTI>(a, job, v), n, wave_base, lane, val);
-                uint32_t* dstv = job_vals_out<MULTI>(a, job, v);
+                load_striped<IPT, LAUX>(vals_in(job, v), n, wave_base, lane, val);
+                uint32_t* dstv = vals_out(job, v);
                 __syncthreads();
 #pragma unroll
                 for (int j = 0; j < IPT; ++j) s_stage[pos[j]] = val[j];
                 __syncthreads();
 #pragma unroll
-                for (int i = 0; i < IPT; ++i)
-                    if (dest[i] < n) dstv[dest[i]] = s_stage[i * BLOCK + tid];
+                for (int i = 0; i < IPT; ++i) {
+                    if constexpr (MID == 3)
+                        __builtin_amdgcn_raw_buffer_store_b32(s_stage[i * BLOCK + tid], array_rsrc(dstv, n),
+                                                              (int)(dest[i] * 4u), 0, SAUX);
+                    else if (dest[i] < n) dstv[dest[i]] = s_stage[i * BLOCK + tid];
+                }
             }
         }
 
+        if constexpr (MID == 3) {
+            // The stores have been taken at the point of coherence before the
+            // tile counts as done.
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (tid == 0)
+                __hip_atomic_fetch_add(a.finished + pass - 1, 1u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+            clear_counts();
+            if (!take_item(job)) break;
+            continue;
+        }
         if constexpr (!XSEG) break;
         if (tid == 0) post_tile(take_tile());
         __syncthreads();  // (every read of this tile's stage is done, too)
@@ -1755,6 +2107,10 @@ extern "C" __global__ void __launch_bounds__(1024) mgpu_digit_count_cols_km(mgpu
     digit_count_body<1024, 32, true>(a);
 }
 
+extern "C" __global__ void __launch_bounds__(1024) mgpu_mid_count(mgpuMidCountArgs a) {
+    mid_count_body<1024>(a);
+}
+
 extern "C" __global__ void __launch_bounds__(256) mgpu_digit_scan(mgpuScanArgs a) {
     digit_scan_body(a);
 }
@@ -1802,29 +2158,29 @@ extern "C" __global__ void __launch_bounds__(256) mgpu_multi_scan(mgpuMultiScanA
 #define MGPU_RANK_SCATTER_MODE(B, I, R, V, MODE)                                             \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r##R##_v##V(mgpuPassArgs a) {                         \
-        rank_scatter_body<B, I, R, MODE, false, false, false, false>(a);                      \
+        rank_scatter_body<B, I, R, MODE, false, false, false, false, 0>(a);                      \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r##R##_x_v##V(mgpuPassArgs a) {                       \
-        rank_scatter_body<B, I, R, MODE, false, true, false, false>(a);                       \
+        rank_scatter_body<B, I, R, MODE, false, true, false, false, 0>(a);                       \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_multi_scatter_b##B##_i##I##_r##R##_v##V(mgpuMultiPassArgs a) {                   \
-        rank_scatter_body<B, I, R, MODE, true, false, false, false>(a);                       \
+        rank_scatter_body<B, I, R, MODE, true, false, false, false, 0>(a);                       \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_multi_scatter_b##B##_i##I##_r##R##_x_v##V(mgpuMultiPassArgs a) {                 \
-        rank_scatter_body<B, I, R, MODE, true, true, false, false>(a);                        \
+        rank_scatter_body<B, I, R, MODE, true, true, false, false, 0>(a);                        \
     }
 // Early-exit forms (atomic-add ranking only): one chain, and a chain per XCD.
 #define MGPU_RANK_SCATTER_EE_MODE(B, I, V, MODE)                                              \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_ee_v##V(mgpuPassArgs a) {                          \
-        rank_scatter_body<B, I, 1, MODE, false, false, true, false>(a);                       \
+        rank_scatter_body<B, I, 1, MODE, false, false, true, false, 0>(a);                       \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_x_ee_v##V(mgpuPassArgs a) {                        \
-        rank_scatter_body<B, I, 1, MODE, false, true, true, false>(a);                        \
+        rank_scatter_body<B, I, 1, MODE, false, true, true, false, 0>(a);                        \
     }
 // Forms that map signed or float keys to their unsigned order as they read
 // them, or back as they write them (atomic-add ranking only): the first and
@@ -1832,11 +2188,11 @@ extern "C" __global__ void __launch_bounds__(256) mgpu_multi_scan(mgpuMultiScanA
 #define MGPU_RANK_SCATTER_KM_MODE(B, I, V, MODE)                                              \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_km_v##V(mgpuPassArgs a) {                          \
-        rank_scatter_body<B, I, 1, MODE, false, false, false, true>(a);                       \
+        rank_scatter_body<B, I, 1, MODE, false, false, false, true, 0>(a);                       \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_x_km_v##V(mgpuPassArgs a) {                        \
-        rank_scatter_body<B, I, 1, MODE, false, true, false, true>(a);                        \
+        rank_scatter_body<B, I, 1, MODE, false, true, false, true, 0>(a);                        \
     }
 #define MGPU_RANK_SCATTER_KM(B, I)                                                            \
     MGPU_RANK_SCATTER_KM_MODE(B, I, 0, MGPU_VALUES_NONE)                                      \
@@ -1881,6 +2237,27 @@ MGPU_RANK_SCATTER(1024, 16, 0)
 MGPU_RANK_SCATTER(256, 16, 1)
 MGPU_RANK_SCATTER(512, 16, 1)
 MGPU_RANK_SCATTER(1024, 16, 1)
+// A bucketed sort's first scatter (_m_) and the passes after it when buckets
+// do not fit: each a launch (_c_), or all in one (_f_); they read no generated
+// indices.
+#define MGPU_RANK_SCATTER_MID_MODE(B, I, T, M, V, MODE)                                       \
+    extern "C" __global__ void __launch_bounds__(B)                                           \
+        mgpu_rank_scatter_b##B##_i##I##_r1_##T##_v##V(mgpuPassArgs a) {                       \
+        rank_scatter_body<B, I, 1, MODE, false, false, false, true, M>(a);                    \
+    }
+#define MGPU_RANK_SCATTER_MID(B, I)                                                           \
+    MGPU_RANK_SCATTER_MID_MODE(B, I, m, 1, 0, MGPU_VALUES_NONE)                               \
+    MGPU_RANK_SCATTER_MID_MODE(B, I, m, 1, 1, MGPU_VALUES_INDEX)                              \
+    MGPU_RANK_SCATTER_MID_MODE(B, I, m, 1, 2, MGPU_VALUES_SINGLE)                             \
+    MGPU_RANK_SCATTER_MID_MODE(B, I, m, 1, 3, MGPU_VALUES_MULTI)                              \
+    MGPU_RANK_SCATTER_MID_MODE(B, I, c, 2, 0, MGPU_VALUES_NONE)                               \
+    MGPU_RANK_SCATTER_MID_MODE(B, I, c, 2, 2, MGPU_VALUES_SINGLE)                             \
+    MGPU_RANK_SCATTER_MID_MODE(B, I, c, 2, 3, MGPU_VALUES_MULTI)
+MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 0, MGPU_VALUES_NONE)
+MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 2, MGPU_VALUES_SINGLE)
+MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 3, MGPU_VALUES_MULTI)
+MGPU_RANK_SCATTER_MID(512, 16)
+MGPU_RANK_SCATTER_MID(1024, 16)
 MGPU_RANK_SCATTER_EE(512, 16)
 MGPU_RANK_SCATTER_EE(1024, 16)
 MGPU_RANK_SCATTER_KM(512, 16)
@@ -1889,16 +2266,49 @@ MGPU_PACKED(256, 16)
 MGPU_PACKED(512, 16)
 MGPU_PACKED(1024, 16)
 
-// One workgroup sorts a small array through every pass: keys only, or with a
-// payload (a value, a generated index, or the source index of several values).
+// One workgroup sorts a small array, or a bucket of a mid-sized one, through
+// every pass: keys only, or with a payload (a value, a generated index, or the
+// source index of several values).
+template <bool PAY>
+__device__ __forceinline__ void local_sort_array(const mgpuLocalArgs& a) {
+    __shared__ mgpu::LocalShared<PAY> sh;
+    if (!a.plan) {
+        mgpu::local_sort<PAY>(a, sh, 0u, a.n, 0u, a.first_bit, a.num_bits);
+        return;
+    }
+    // The counts go back to zero; when the digit passes go on, workgroup p first
+    // makes pass p's digit starts of them (the last digits are the bins' top
+    // bits).
+    const uint32_t b = blockIdx.x;
+    if (b < a.num_passes) {
+        const uint32_t tid = threadIdx.x, first = b + 1 == a.num_passes ? 0u : MGPU_MID_BINS + b * RADIX;
+        uint32_t* const h = a.hist + first;
+        uint32_t cnt = 0;
+        if (first == 0) {
+            const uint32_t per = MGPU_MID_BINS >> a.last_width;
+            if (tid < (1u << a.last_width))
+                for (uint32_t i = 0; i < per; ++i) cnt += h[tid * per + i];
+        } else if (tid < RADIX) {
+            cnt = h[tid];
+        }
+        const uint32_t st = mgpu::block_exclusive_scan_dpp<MGPU_LOCAL_THREADS>(
+            cnt, sh.tmp, tid & 63, (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)));
+        if (tid < RADIX) a.starts[b * RADIX + tid] = st;
+        __syncthreads();
+        if (first == 0 || tid < RADIX) h[tid] = 0;
+    }
+    if (!a.plan->buckets) return;
+    const uint32_t begin = a.plan->start[b], n = a.plan->start[b + 1] - begin;
+    if (n == 0 || n > MGPU_LOCAL_MAX_KEYS) return;
+    mgpu::local_sort<PAY>(a, sh, begin, n, a.plan->base[b], a.first_bit, a.plan->bits[b]);
+}
+
 extern "C" __global__ void __launch_bounds__(MGPU_LOCAL_THREADS) mgpu_local_sort_k(mgpuLocalArgs a) {
-    __shared__ mgpu::LocalShared<false> sh;
-    mgpu::local_sort<false>(a, sh, 0u, a.n, 0u, a.first_bit, a.num_bits);
+    local_sort_array<false>(a);
 }
 
 extern "C" __global__ void __launch_bounds__(MGPU_LOCAL_THREADS) mgpu_local_sort_kv(mgpuLocalArgs a) {
-    __shared__ mgpu::LocalShared<true> sh;
-    mgpu::local_sort<true>(a, sh, 0u, a.n, 0u, a.first_bit, a.num_bits);
+    local_sort_array<true>(a);
 }
 
 // Check of the ordering RANK 1 relies on: wave w of one 1024-thread

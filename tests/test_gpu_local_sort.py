@@ -45,7 +45,7 @@ def test_one_launch_sort(engine, oracle, n, vc, kind):
         g.run(engine)
         names = set(engine.read_timing())
         engine.enable_timing(False)
-        assert any("local_sort" in k for k in names) == (n <= MAX), names
+        assert (len(names) == 1) == (n <= MAX), names
         rk, rv = oracle.stable_sort(keys, vals, value_count=vc, first_bit=fb, end_bit=eb)
         assert np.array_equal(g.keys(), rk)
         for o, r in zip(g.values(), rv):
