@@ -968,7 +968,12 @@ sortStatus_t SORTAPI sortArrayTyped(sortEngine_t engine, sortData_t data, int ke
 }
 
 // sortArrayEx (mgpusort.cpp:618-648): the caller's digit width sets the pass
-// count; the widths are split evenly with narrower passes first.
+// count, and with it the buffer side of the result and the parity; the widths
+// are split evenly with narrower passes first.  The order does not depend on
+// the split, so as few passes as 8-bit digits need run instead where they end
+// on the same side (one more when the parities differ; 500000 pairs by 6-bit
+// digits 60.1 -> 31.7 us).  Early exit keeps the caller's passes: which of
+// them are skipped shows in the parity.
 sortStatus_t SORTAPI sortArrayEx(sortEngine_t engine, sortData_t data, int numSortThreads,
                                  int valuesPerThread, int bitPass, bool useTransList) {
     (void)useTransList;
@@ -985,6 +990,15 @@ sortStatus_t SORTAPI sortArrayEx(sortEngine_t engine, sortData_t data, int numSo
     if (bitPass > numBits) bitPass = numBits;
     int widths[32];
     int passes = mgpu_plan_passes(numBits, bitPass, widths);
+    if (!data->earlyExit) {
+        int fewest = mgpu_plan_passes(numBits, MGPU_RADIX_BITS, nullptr);
+        fewest += (passes ^ fewest) & 1;
+        if (fewest < passes && fewest <= MGPU_MAX_PASSES) {
+            passes = fewest;
+            for (int p = 0; p < passes; ++p)
+                widths[p] = numBits / passes + (p >= passes - numBits % passes ? 1 : 0);
+        }
+    }
     // More than MGPU_MAX_PASSES passes: run them in groups (each group one
     // digit_count + scan); parity and swaps stay per pass.
     int done = 0, bit = data->firstBit;

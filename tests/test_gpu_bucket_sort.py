@@ -144,3 +144,23 @@ def test_captured(oracle):
             _check(oracle, keys, g, [vals], 1)
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("fb,eb", [(0, 32), (0, 31), (5, 30), (0, 24), (4, 20), (0, 13), (0, 7)])
+@pytest.mark.parametrize("n", [3000, 40_001, 3 * (1 << 20) + 5])
+def test_ex_runs_fewer_passes(engine, oracle, fb, eb, n):
+    """sortArrayEx with every digit width: the order, the parity and the side of
+    the result are those of the caller's passes, however many run."""
+    if n > 1 << 20 and (fb, eb) not in ((0, 32), (0, 24)):
+        return
+    keys = _keys("even", n)
+    vals = [np.arange(n, dtype=np.uint32)]
+    rk, (rv,) = oracle.stable_sort(keys, vals, first_bit=fb, end_bit=eb)
+    for bit_pass in (1, 2, 3, 4, 5, 6):
+        g = GpuSort(keys, vals, first_bit=fb, end_bit=eb)
+        g.run(engine, ex=(256, 8, bit_pass, False))
+        engine.check_device()
+        assert np.array_equal(g.keys(), rk) and np.array_equal(g.values()[0], rv)
+        passes = -(-(eb - fb) // min(bit_pass, eb - fb))
+        assert g.data.parity == passes % 2
+        assert g.data.keys[g.data.parity] == g.start_keys
