@@ -17,22 +17,28 @@
 namespace mgpu {
 
 constexpr int kLocalBlock = MGPU_LOCAL_THREADS;
-constexpr int kLocalWaves = kLocalBlock / 64;
 constexpr uint32_t kLocalTile = MGPU_LOCAL_MAX_KEYS;
 // Words from one wave's digit counts to the next: a multiple of 4 for 16-byte
 // clearing, and not of 64, so that the scan's threads (digit, group of four
 // waves) read different banks.
 constexpr uint32_t kLocalRow = MGPU_RADIX + 4;
-static_assert(kLocalBlock == 4 * MGPU_RADIX && kLocalWaves == 16,
-              "the scan gives a thread one digit of four waves");
 
-template <bool PAY>
+template <int BLOCK, uint32_t TILE, bool PAY>
 struct LocalShared {
-    uint32_t count[kLocalWaves * kLocalRow] __attribute__((aligned(16)));
-    uint32_t tmp[kLocalWaves];
-    uint32_t key[kLocalTile];
-    uint32_t pay[PAY ? kLocalTile : 1];
+    uint32_t count[BLOCK / 64 * kLocalRow] __attribute__((aligned(16)));
+    uint32_t tmp[BLOCK / 64];
+    uint32_t key[TILE];
+    uint32_t pay[PAY ? TILE : 1];
 };
+
+// The words of it a sort uses.
+struct LocalMem {
+    uint32_t *count, *tmp, *key, *pay;
+};
+template <int BLOCK, uint32_t TILE, bool PAY>
+__device__ __forceinline__ LocalMem local_mem(LocalShared<BLOCK, TILE, PAY>& sh) {
+    return {sh.count, sh.tmp, sh.key, sh.pay};
+}
 
 // Buffer resource over words [0, n) at p: loads past n return 0, stores there
 // are dropped.
@@ -41,27 +47,46 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t words_rsrc(const uint32_t* p, 
                                              0x00020000);
 }
 
-// Sorts elements [begin, begin + n) of the arrays of `a`, 0 < n <= IT *
-// kLocalBlock, by bits [shift0, shift0 + bits) of (key - base).  IT keys per
-// thread: wave w holds keys w * 64 * IT + j * 64 + lane.  Slots past n hold
-// all ones in every digit, so they stay behind every key.
-template <int IT, bool PAY>
-__device__ void local_sort_items(const mgpuLocalArgs& a, LocalShared<PAY>& sh, uint32_t begin,
-                                 uint32_t n, uint32_t base, uint32_t shift0, uint32_t bits) {
+// Where a sort of a whole array or a bucket reads and writes (elements from
+// `begin` of the arrays of `a`); the sorts below take any type with these
+// members.
+struct LocalArrays {
+    const mgpuLocalArgs& a;
+    uint32_t begin;
+    __device__ __forceinline__ const uint32_t* keys_in() const { return a.keys_in + begin; }
+    __device__ __forceinline__ uint32_t* keys_out() const { return a.keys_out + begin; }
+    __device__ __forceinline__ const uint32_t* vals_in(uint32_t v) const { return a.vals_in[v] + begin; }
+    __device__ __forceinline__ uint32_t* vals_out(uint32_t v) const { return a.vals_out[v] + begin; }
+    __device__ __forceinline__ uint32_t mode() const { return a.vals_mode; }
+    __device__ __forceinline__ uint32_t num_values() const { return a.num_values; }
+    __device__ __forceinline__ uint32_t read(uint32_t k) const { return mgpu_key_map(k, a.in_lo, a.in_hi); }
+    __device__ __forceinline__ uint32_t write(uint32_t k) const { return mgpu_key_map(k, a.out_lo, a.out_hi); }
+};
+
+// Sorts the n elements of `io`, 0 < n <= IT * BLOCK, by bits [shift0, shift0 +
+// bits) of (key - base).  IT keys per thread: wave w holds keys w * 64 * IT +
+// j * 64 + lane.  Slots past n hold all ones in every digit, so they stay
+// behind every key.
+template <int BLOCK, int IT, bool PAY, typename IO>
+__device__ __forceinline__ void local_sort_items(const IO& io, const LocalMem& sh, uint32_t n, uint32_t base,
+                                 uint32_t shift0, uint32_t bits) {
+    constexpr uint32_t G = BLOCK / MGPU_RADIX;  // threads per digit in the scan
+    static_assert(BLOCK % MGPU_RADIX == 0 && BLOCK / 64 == 4 * G,
+                  "the scan gives a thread one digit of four waves");
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t first = wave * 64 * IT + lane;  // this lane's key of slot 0
     const uint32_t off = first * 4u;
-    const uint32_t fill = a.vals_mode;
+    const uint32_t fill = io.mode();
     uint32_t key[IT], pay[PAY ? IT : 1];
     {
-        const __amdgpu_buffer_rsrc_t rk = words_rsrc(a.keys_in + begin, n);
+        const __amdgpu_buffer_rsrc_t rk = words_rsrc(io.keys_in(), n);
 #pragma unroll
         for (int j = 0; j < IT; ++j)
             key[j] = __builtin_amdgcn_raw_buffer_load_b32(rk, (int)(off + j * 256u), 0, 0);
         if constexpr (PAY) {
             if (fill == MGPU_VALUES_SINGLE) {
-                const __amdgpu_buffer_rsrc_t rv = words_rsrc(a.vals_in[0] + begin, n);
+                const __amdgpu_buffer_rsrc_t rv = words_rsrc(io.vals_in(0), n);
 #pragma unroll
                 for (int j = 0; j < IT; ++j)
                     pay[j] = __builtin_amdgcn_raw_buffer_load_b32(rv, (int)(off + j * 256u), 0, 0);
@@ -73,10 +98,10 @@ __device__ void local_sort_items(const mgpuLocalArgs& a, LocalShared<PAY>& sh, u
     }
 #pragma unroll
     for (int j = 0; j < IT; ++j)
-        key[j] = first + j * 64u < n ? mgpu_key_map(key[j], a.in_lo, a.in_hi) - base : 0xFFFFFFFFu;
+        key[j] = first + j * 64u < n ? io.read(key[j]) - base : 0xFFFFFFFFu;
 
     uint32_t* const row = sh.count + wave * kLocalRow;
-    const uint32_t dq = tid >> 2, g = tid & 3u;  // the scan's digit and group of waves
+    const uint32_t dq = tid / G, g = tid % G;  // the scan's digit and group of waves
     uint32_t* const col = sh.count + g * 4 * kLocalRow + dq;
     const uint32_t passes = (bits + MGPU_RADIX_BITS - 1) / MGPU_RADIX_BITS;
     uint32_t shift = shift0, left = bits;
@@ -92,7 +117,7 @@ __device__ void local_sort_items(const mgpuLocalArgs& a, LocalShared<PAY>& sh, u
         const uint32_t c0 = col[0], c1 = col[kLocalRow], c2 = col[2 * kLocalRow],
                        c3 = col[3 * kLocalRow];
         const uint32_t start =
-            block_exclusive_scan_dpp<kLocalBlock>(c0 + c1 + c2 + c3, sh.tmp, lane, wave);
+            block_exclusive_scan_dpp<BLOCK>(c0 + c1 + c2 + c3, sh.tmp, lane, wave);
         col[0] = start;
         col[kLocalRow] = start + c0;
         col[2 * kLocalRow] = start + c0 + c1;
@@ -114,27 +139,33 @@ __device__ void local_sort_items(const mgpuLocalArgs& a, LocalShared<PAY>& sh, u
         shift += width;
         left -= width;
     }
+    // (No pass, as for a bucket of one value: the loads above still come
+    // before every store.)
+    if (passes == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
 
     // Every key and carried value was loaded before a barrier above, so the
     // output may be the input's buffers.
     {
-        const __amdgpu_buffer_rsrc_t rk = words_rsrc(a.keys_out + begin, n);
+        const __amdgpu_buffer_rsrc_t rk = words_rsrc(io.keys_out(), n);
 #pragma unroll
         for (int j = 0; j < IT; ++j)
-            __builtin_amdgcn_raw_buffer_store_b32(mgpu_key_map(key[j] + base, a.out_lo, a.out_hi), rk,
+            __builtin_amdgcn_raw_buffer_store_b32(io.write(key[j] + base), rk,
                                                   (int)(off + j * 256u), 0, 0);
     }
     if constexpr (PAY) {
         if (fill != MGPU_VALUES_MULTI) {
-            const __amdgpu_buffer_rsrc_t rv = words_rsrc(a.vals_out[0] + begin, n);
+            const __amdgpu_buffer_rsrc_t rv = words_rsrc(io.vals_out(0), n);
 #pragma unroll
             for (int j = 0; j < IT; ++j)
                 __builtin_amdgcn_raw_buffer_store_b32(pay[j], rv, (int)(off + j * 256u), 0, 0);
         } else {
             // Two or more arrays: gathered through the source index.
-            for (uint32_t v = 0; v < a.num_values; ++v) {
-                const __amdgpu_buffer_rsrc_t rv = words_rsrc(a.vals_in[v] + begin, n);
-                const __amdgpu_buffer_rsrc_t ro = words_rsrc(a.vals_out[v] + begin, n);
+            for (uint32_t v = 0; v < io.num_values(); ++v) {
+                const __amdgpu_buffer_rsrc_t rv = words_rsrc(io.vals_in(v), n);
+                const __amdgpu_buffer_rsrc_t ro = words_rsrc(io.vals_out(v), n);
                 uint32_t val[IT];
 #pragma unroll
                 for (int j = 0; j < IT; ++j)
@@ -151,16 +182,17 @@ __device__ void local_sort_items(const mgpuLocalArgs& a, LocalShared<PAY>& sh, u
     }
 }
 
-template <bool PAY>
-__device__ __forceinline__ void local_sort(const mgpuLocalArgs& a, LocalShared<PAY>& sh,
-                                           uint32_t begin, uint32_t n, uint32_t base,
-                                           uint32_t shift, uint32_t bits) {
-    if (n <= 1 * kLocalBlock) local_sort_items<1, PAY>(a, sh, begin, n, base, shift, bits);
-    else if (n <= 2 * kLocalBlock) local_sort_items<2, PAY>(a, sh, begin, n, base, shift, bits);
-    else if (n <= 4 * kLocalBlock) local_sort_items<4, PAY>(a, sh, begin, n, base, shift, bits);
-    else if (n <= 8 * kLocalBlock) local_sort_items<8, PAY>(a, sh, begin, n, base, shift, bits);
-    else if (n <= 12 * kLocalBlock) local_sort_items<12, PAY>(a, sh, begin, n, base, shift, bits);
-    else local_sort_items<16, PAY>(a, sh, begin, n, base, shift, bits);
+// The same with the least IT that holds n <= 16 * kLocalBlock elements.
+template <bool PAY, typename IO>
+__device__ __forceinline__ void local_sort(const IO& io, const LocalMem& sh, uint32_t n,
+                                           uint32_t base, uint32_t shift, uint32_t bits) {
+    constexpr int B = kLocalBlock;
+    if (n <= 1 * B) local_sort_items<B, 1, PAY>(io, sh, n, base, shift, bits);
+    else if (n <= 2 * B) local_sort_items<B, 2, PAY>(io, sh, n, base, shift, bits);
+    else if (n <= 4 * B) local_sort_items<B, 4, PAY>(io, sh, n, base, shift, bits);
+    else if (n <= 8 * B) local_sort_items<B, 8, PAY>(io, sh, n, base, shift, bits);
+    else if (n <= 12 * B) local_sort_items<B, 12, PAY>(io, sh, n, base, shift, bits);
+    else local_sort_items<B, 16, PAY>(io, sh, n, base, shift, bits);
 }
 
 }  // namespace mgpu

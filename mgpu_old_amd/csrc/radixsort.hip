@@ -2271,9 +2271,10 @@ MGPU_PACKED(1024, 16)
 // source index of several values).
 template <bool PAY>
 __device__ __forceinline__ void local_sort_array(const mgpuLocalArgs& a) {
-    __shared__ mgpu::LocalShared<PAY> sh;
+    __shared__ mgpu::LocalShared<mgpu::kLocalBlock, mgpu::kLocalTile, PAY> sh;
     if (!a.plan) {
-        mgpu::local_sort<PAY>(a, sh, 0u, a.n, 0u, a.first_bit, a.num_bits);
+        mgpu::local_sort<PAY>(mgpu::LocalArrays{a, 0u}, local_mem(sh), a.n, 0u, a.first_bit,
+                              a.num_bits);
         return;
     }
     // The counts go back to zero; when the digit passes go on, workgroup p first
@@ -2300,7 +2301,8 @@ __device__ __forceinline__ void local_sort_array(const mgpuLocalArgs& a) {
     if (!a.plan->buckets) return;
     const uint32_t begin = a.plan->start[b], n = a.plan->start[b + 1] - begin;
     if (n == 0 || n > MGPU_LOCAL_MAX_KEYS) return;
-    mgpu::local_sort<PAY>(a, sh, begin, n, a.plan->base[b], a.first_bit, a.plan->bits[b]);
+    mgpu::local_sort<PAY>(mgpu::LocalArrays{a, begin}, local_mem(sh), n, a.plan->base[b],
+                          a.first_bit, a.plan->bits[b]);
 }
 
 extern "C" __global__ void __launch_bounds__(MGPU_LOCAL_THREADS) mgpu_local_sort_k(mgpuLocalArgs a) {

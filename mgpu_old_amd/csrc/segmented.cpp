@@ -148,7 +148,8 @@ sortStatus_t mgpu_seg_load(sortEngine_d* e) {
     // (written by the autotuner), else the built-in default.  Rows
     // "<max ceil(log2 n)> <radix bits> <keys per thread> [<threads>]" pick the
     // persistent kernel per size bucket; a row "wide <min keys> <chunk>
-    // <auto|small|large>" sets the device-wide passes.
+    // <auto|small|large> [<auto|packed|unpacked> [<kept keys>]]" sets the
+    // device-wide passes.
     e->segTable.assign(std::begin(kDefaultTable), std::end(kDefaultTable));
     e->segWide = SegWideTune();
     std::ifstream f(e->kernelPath + "mgpusort_seg_tuning.txt");
@@ -169,6 +170,8 @@ sortStatus_t mgpu_seg_load(sortEngine_d* e) {
                         e->segWide.chunk = clamp_chunk(chunk);
                         e->segWide.tile = tile == "small" ? 1 : tile == "large" ? 2 : 0;
                         e->segWide.pack = pack == "packed" ? 1 : pack == "unpacked" ? 0 : -1;
+                        long keep = 0;
+                        e->segWide.keepKeys = is >> keep && keep > 0 ? (uint32_t)keep : 0u;
                     }
                 }
                 continue;
@@ -218,6 +221,37 @@ void pick_variant(const sortEngine_d* e, uint32_t n, int* rb, int* ipt, int* blo
     *rb = 8;
     *ipt = 16;
     *block = 256;
+}
+
+bool seg_fits_tile(const sortEngine_d* e, uint32_t n) {
+    int rb, ipt, block;
+    pick_variant(e, n, &rb, &ipt, &block);
+    return rb == 8 && n <= (uint32_t)(block * ipt) && n <= e->segWide.keepKeys;
+}
+
+// Segments of wide.minKeys keys or more, up to wide.keepKeys, that fit the
+// tile of the kernel the table gives them (the shipped one: 8192 keys with 16
+// keys per thread) stay with one workgroup each, in one launch, while the batch's still longer segments hold
+// at most as many keys as they do.  With more than that the device-wide passes
+// run over most of the keys anyway, and the shorter segments cost less in them
+// than in a kernel beside them that holds 80 KB of LDS on every CU.
+// MGPUSORT_SEG_WIDE_MIN sends all of its segments to the device-wide passes.
+// Plan replays, device-wide -> one workgroup each, keys only / key + value /
+// two values, us: 40 segments in [4097, 8192] 46 -> 30 / 53 -> 29 / 73 -> 33;
+// 3000 in [4097, 9000] 296 -> 254 / 440 -> 308 / 816 -> 415; 16000 log-uniform
+// in [1, 8192] 220 -> 156 / 271 -> 183 / 398 -> 218; 8000 in [64, 10000] 236 ->
+// 196 / 308 -> 235 / 487 -> 315; past the line the two come out alike (6000 in
+// [64, 16384] 272 / 268, 4096 in [1, 2^16] 321 / 333 us, keys only).
+bool keep_in_workgroups(const sortEngine_d* e, const mgpuSegDesc* segs, int numSegments,
+                        uint32_t wideMin) {
+    if (e->segWide.keepKeys < wideMin || std::getenv("MGPUSORT_SEG_WIDE_MIN") != nullptr ||
+        e->rankMethod != 1)
+        return false;
+    uint64_t fit = 0, longer = 0;
+    for (int i = 0; i < numSegments; ++i)
+        if (segs[i].n >= wideMin)
+            (seg_fits_tile(e, segs[i].n) ? fit : longer) += segs[i].n;
+    return longer <= fit;
 }
 
 }  // namespace
@@ -294,6 +328,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
 
     // Group segments by kernel variant; very large ones go device-wide.
     const uint32_t wideMin = device_wide_min(e), chunkKeys = wide_chunk(e);
+    const bool keepFit = keep_in_workgroups(e, segs, numSegments, wideMin);
     struct Group {
         std::vector<uint32_t> big, small;
     };
@@ -301,7 +336,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
     for (int i = 0; i < numSegments; ++i) {
         const uint32_t n = segs[i].n;
         if (n == 0 || P.numBits == 0) continue;
-        if (n >= wideMin) {
+        if (n >= wideMin && !(keepFit && seg_fits_tile(e, n))) {
             P.wide.push_back((uint32_t)i);
             continue;
         }

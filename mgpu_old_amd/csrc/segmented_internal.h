@@ -51,6 +51,8 @@ struct SegWideTune {
     uint32_t chunk = 1u << 14;
     int tile = 0;
     int pack = -1;
+    uint32_t keepKeys = 0;  // up to here one workgroup sorts a segment that fits its tile, while
+                            // few keys are in longer ones (0: no segment of minKeys or more)
 };
 
 // One persistent launch of one kernel variant.

@@ -27,6 +27,7 @@
 #include <stdint.h>
 
 #include "kernel_args.h"
+#include "localsort.h"
 #include "radix_device.h"
 
 namespace {
@@ -89,7 +90,7 @@ struct SegShared {
     static constexpr int MAXP = (32 + RB - 1) / RB;
     static_assert(64 * IPT >= RADIX, "a wave's stage slice holds its match-mask table");
     uint64_t stage[TILE];
-    uint32_t count[W][RADIX];
+    uint32_t count[W][RADIX + 4] __attribute__((aligned(16)));
     uint32_t base[MAXP][RADIX];  // global routine: per-pass digit starts
     uint32_t run[RADIX];         // global routine: running digit offsets
     uint32_t dst[RADIX];         // global routine: output base per digit for a tile
@@ -172,7 +173,7 @@ __device__ __forceinline__ void load_slots(const mgpuSegArgs& a, const mgpuSegDe
 
 // ---- one wave, whole segment in registers + this wave's LDS slice ---------
 template <int RB, int IPT, int BLOCK>
-__device__ void wave_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShared<RB, IPT, BLOCK>& sh,
+__device__ __forceinline__ void wave_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShared<RB, IPT, BLOCK>& sh,
                           uint32_t lane, uint32_t wave) {
     constexpr int RADIX = SegShared<RB, IPT, BLOCK>::RADIX;
     constexpr int DPL = RADIX >= 64 ? RADIX / 64 : 1;  // digits per lane in the scan
@@ -243,7 +244,7 @@ __device__ void wave_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShared<
 // would leave it; each lane then takes its key and payload from the lane its
 // compare key came from.  No LDS and no atomics: two shuffles per step, 21
 // steps.
-__device__ void wave_bitonic64(const mgpuSegArgs& a, const mgpuSegDesc& s, uint32_t lane) {
+__device__ __forceinline__ void wave_bitonic64(const mgpuSegArgs& a, const mgpuSegDesc& s, uint32_t lane) {
     const uint32_t n = s.n;
     uint32_t idx[1] = {lane}, key[1], pay[1];
     load_slots<1>(a, s, n, idx, key, pay);
@@ -274,7 +275,7 @@ __device__ void wave_bitonic64(const mgpuSegArgs& a, const mgpuSegDesc& s, uint3
 
 // ---- one workgroup, whole segment in registers + LDS ----------------------
 template <int RB, int IPT, int BLOCK>
-__device__ void block_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShared<RB, IPT, BLOCK>& sh,
+__device__ __forceinline__ void block_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShared<RB, IPT, BLOCK>& sh,
                            uint32_t tid, uint32_t lane, uint32_t wave) {
     constexpr int RADIX = SegShared<RB, IPT, BLOCK>::RADIX;
     constexpr int W = BLOCK / 64;
@@ -288,7 +289,7 @@ __device__ void block_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShared
         pass_field(a, p, shift, mask);
         // (The previous pass's reads of the stage end before this barrier,
         // and its writes of the next pass come after two more.)
-        for (uint32_t i = tid; i < (uint32_t)(W * RADIX); i += BLOCK) (&sh.count[0][0])[i] = 0;
+        for (uint32_t i = tid; i < (uint32_t)(W * (RADIX + 4)); i += BLOCK) (&sh.count[0][0])[i] = 0;
         __syncthreads();
         clear_match(a, sh, lane, wave);
         uint32_t rank[IPT];
@@ -333,7 +334,7 @@ __device__ void block_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShared
 
 // ---- one workgroup, passes through global memory ---------------------------
 template <int RB, int IPT, int BLOCK>
-__device__ void global_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShared<RB, IPT, BLOCK>& sh,
+__device__ __forceinline__ void global_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShared<RB, IPT, BLOCK>& sh,
                             uint32_t tid, uint32_t lane, uint32_t wave) {
     constexpr int RADIX = SegShared<RB, IPT, BLOCK>::RADIX;
     uint32_t* const st = reinterpret_cast<uint32_t*>(sh.stage);  // TILE words of it
@@ -370,7 +371,7 @@ __device__ void global_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShare
         const auto ko = mgpu::to_global(s.keys[out]);
         if (tid < (uint32_t)RADIX) sh.run[tid] = sh.base[p][tid];
         for (uint32_t tb = 0; tb < n; tb += TILE) {
-            for (uint32_t i = tid; i < (uint32_t)(W * RADIX); i += BLOCK) (&sh.count[0][0])[i] = 0;
+            for (uint32_t i = tid; i < (uint32_t)(W * (RADIX + 4)); i += BLOCK) (&sh.count[0][0])[i] = 0;
             __syncthreads();
             clear_match(a, sh, lane, wave);
             uint32_t key[IPT], rank[IPT], pos[IPT], dest[IPT];
@@ -467,18 +468,295 @@ __device__ void global_sort(const mgpuSegArgs& a, const mgpuSegDesc& s, SegShare
     }
 }
 
+// ---- 8-bit digits ranked by ordered LDS adds --------------------------------
+// (What the shipped table's kernels run; the routines above serve the other
+// digit widths and the match-mask ranking.)
+//
+// Bound by LDS round trips and, in the small list, by the chain of reads from
+// a list entry to its keys: a batch's bytes pass in a few microseconds.  So
+// the ranks of all slots are requested before the first is used, keys and
+// payloads lie in 32-bit words of their own, a segment takes no more slots per
+// thread than it fills, and the small list's reads run ahead of the sorts.
+// Plan replays, the routines above -> these, keys only / key + value / two
+// values, us: 60000 segments log-uniform in [1, 512] 109 -> 75 / 123 -> 85 /
+// 135 -> 95; 130000 in [1, 64] 143 -> 85 / 162 -> 98 / 186 -> 112; 20000 in
+// [64, 4096] 297 -> 186 / 357 -> 214 / 411 -> 261; 5000 of 512 105 -> 72 /
+// 125 -> 79 / 134 -> 85.
+
+// A segment's arrays.  Its descriptor does not change while the kernel runs,
+// so it is read through the constant address space: scalar loads, once a wave.
+struct SegArrays {
+    const uint32_t *ki, *vi;  // keys and the first values, input side
+    uint32_t *ko, *vo;        // result side
+    uint32_t seg, n;
+};
+
+typedef const __attribute__((address_space(4))) mgpuSegDesc* ConstDesc;
+typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
+
+__device__ __forceinline__ SegArrays seg_arrays(const mgpuSegArgs& a, uint32_t seg) {
+    const ConstDesc d = (ConstDesc)(a.segs + seg);
+    SegArrays s;
+    s.ki = d->keys[0];
+    s.ko = a.result_side ? d->keys[1] : d->keys[0];
+    s.vi = d->vals[0][0];
+    s.vo = a.result_side ? d->vals[0][1] : d->vals[0][0];
+    s.seg = seg;
+    s.n = d->n;
+    return s;
+}
+__device__ __forceinline__ const uint32_t* seg_vals_in(const mgpuSegArgs& a, const SegArrays& s, uint32_t v) {
+    return ((ConstDesc)(a.segs + s.seg))->vals[v][0];
+}
+__device__ __forceinline__ uint32_t* seg_vals_out(const mgpuSegArgs& a, const SegArrays& s, uint32_t v) {
+    return ((ConstDesc)(a.segs + s.seg))->vals[v][a.result_side];
+}
+
+// The same for local_sort_items.
+struct SegIO {
+    const mgpuSegArgs& a;
+    const SegArrays& s;
+    __device__ __forceinline__ const uint32_t* keys_in() const { return s.ki; }
+    __device__ __forceinline__ uint32_t* keys_out() const { return s.ko; }
+    __device__ __forceinline__ const uint32_t* vals_in(uint32_t v) const { return seg_vals_in(a, s, v); }
+    __device__ __forceinline__ uint32_t* vals_out(uint32_t v) const { return seg_vals_out(a, s, v); }
+    __device__ __forceinline__ uint32_t mode() const {
+        return a.index_mode          ? MGPU_VALUES_INDEX
+               : a.num_values == 1   ? MGPU_VALUES_SINGLE
+                                     : MGPU_VALUES_MULTI;
+    }
+    __device__ __forceinline__ uint32_t num_values() const { return a.num_values; }
+    __device__ __forceinline__ uint32_t read(uint32_t k) const { return k; }
+    __device__ __forceinline__ uint32_t write(uint32_t k) const { return k; }
+};
+
+// One wave, at most 64 keys, one per lane: a key's place is the number of keys
+// before it in the stable order, counted against each key in turn (a scalar
+// broadcast, two compares and an add with carry).  No LDS, no dependence on
+// the sort's width, and the work is n steps where a bitonic network takes 21
+// of two LDS shuffles whatever n.  Every store goes straight to its place.
+__device__ __forceinline__ void wave_place64(const mgpuSegArgs& a, const SegArrays& s, uint32_t lane,
+                                             uint32_t key, uint32_t pay) {
+    const uint32_t n = s.n;
+    const uint32_t f = lane < n ? (a.num_bits >= 32 ? key : __builtin_amdgcn_ubfe(key, a.first_bit, a.num_bits))
+                                : 0xFFFFFFFFu;
+    uint32_t place = 0;
+    for (uint32_t j = 0; j < n; j += 4) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            // (Lanes past n hold all ones and lie after every key: counting
+            // against them changes nothing.)
+            const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)f, (int)((j + i) & 63u));
+            place += (o < f || (o == f && lane > j + i)) ? 1u : 0u;
+        }
+    }
+    const uint32_t off = lane < n ? place * 4u : n * 4u;  // past the range: dropped
+    __builtin_amdgcn_raw_buffer_store_b32(key, mgpu::words_rsrc(s.ko, n), (int)off, 0, 0);
+    if (a.num_values == 0) return;
+    if (a.index_mode || a.num_values == 1) {
+        __builtin_amdgcn_raw_buffer_store_b32(a.index_mode ? lane : pay, mgpu::words_rsrc(s.vo, n),
+                                              (int)off, 0, 0);
+        return;
+    }
+    for (uint32_t v = 0; v < a.num_values; ++v) {
+        const uint32_t val = __builtin_amdgcn_raw_buffer_load_b32(mgpu::words_rsrc(seg_vals_in(a, s, v), n),
+                                                                  (int)(lane * 4u), 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(val, mgpu::words_rsrc(seg_vals_out(a, s, v), n), (int)off, 0, 0);
+    }
+}
+
+// One wave, at most 64 * IT keys, in the wave's rows of the counts and the
+// stage: no barriers.  Slots past n hold all ones, so they stay behind every
+// key.  taken() is called once kin and pin have been read.
+template <int IT, bool PAY, typename Taken>
+__device__ __forceinline__ void wave_sort8(const mgpuSegArgs& a, const SegArrays& s, uint32_t* row,
+                                           uint32_t* skey, uint32_t* spay, uint32_t lane,
+                                           const uint32_t* kin, const uint32_t* pin, Taken taken) {
+    const uint32_t n = s.n;
+    uint32_t key[IT], pay[PAY ? IT : 1];
+    // The slots that the caller has not read.
+    uint32_t more_k[8] = {}, more_v[8] = {};
+    if constexpr (IT > 8) {
+        const __amdgpu_buffer_rsrc_t rk = mgpu::words_rsrc(s.ki, n);
+#pragma unroll
+        for (int j = 8; j < IT; ++j)
+            more_k[j - 8] =
+                __builtin_amdgcn_raw_buffer_load_b32(rk, (int)((j * 64 + lane) * 4u), 0, 0);
+        if (PAY && !a.index_mode && a.num_values == 1) {
+            const __amdgpu_buffer_rsrc_t rv = mgpu::words_rsrc(s.vi, n);
+#pragma unroll
+            for (int j = 8; j < IT; ++j)
+                more_v[j - 8] =
+                    __builtin_amdgcn_raw_buffer_load_b32(rv, (int)((j * 64 + lane) * 4u), 0, 0);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        key[j] = j * 64 + lane < n ? (j < 8 ? kin[j & 7] : more_k[j & 7]) : 0xFFFFFFFFu;
+        if constexpr (PAY)
+            pay[j] = a.index_mode || a.num_values > 1 ? j * 64 + lane
+                     : j < 8                          ? pin[j & 7]
+                                                      : more_v[j & 7];
+    }
+    taken();
+    uint32_t shift = a.first_bit, left = a.num_bits;
+    for (uint32_t p = 0; p < a.num_passes; ++p) {
+        const uint32_t width = left / (a.num_passes - p);
+        reinterpret_cast<uint4*>(row)[lane] = make_uint4(0u, 0u, 0u, 0u);
+        uint32_t d[IT], pos[IT];
+#pragma unroll
+        for (int j = 0; j < IT; ++j) d[j] = __builtin_amdgcn_ubfe(key[j], shift, width);
+        mgpu::rank_slots<IT>(d, row, lane, pos);
+        wave_sync();
+        const uint4 c = reinterpret_cast<const uint4*>(row)[lane];
+        const uint32_t sum = c.x + c.y + c.z + c.w;
+        const uint32_t at = mgpu::wave_inclusive_scan_dpp(sum) - sum;
+        reinterpret_cast<uint4*>(row)[lane] =
+            make_uint4(at, at + c.x, at + c.x + c.y, at + c.x + c.y + c.z);
+        wave_sync();
+#pragma unroll
+        for (int j = 0; j < IT; ++j) pos[j] += row[d[j]];
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+            skey[pos[j]] = key[j];
+            if constexpr (PAY) spay[pos[j]] = pay[j];
+        }
+        wave_sync();
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+            key[j] = skey[j * 64 + lane];
+            if constexpr (PAY) pay[j] = spay[j * 64 + lane];
+        }
+        wave_sync();
+        shift += width;
+        left -= width;
+    }
+    const __amdgpu_buffer_rsrc_t rk = mgpu::words_rsrc(s.ko, n);
+#pragma unroll
+    for (int j = 0; j < IT; ++j)
+        __builtin_amdgcn_raw_buffer_store_b32(key[j], rk, (int)((j * 64 + lane) * 4u), 0, 0);
+    if constexpr (PAY) {
+        if (a.index_mode || a.num_values == 1) {
+            const __amdgpu_buffer_rsrc_t rv = mgpu::words_rsrc(s.vo, n);
+#pragma unroll
+            for (int j = 0; j < IT; ++j)
+                __builtin_amdgcn_raw_buffer_store_b32(pay[j], rv, (int)((j * 64 + lane) * 4u), 0, 0);
+            return;
+        }
+        for (uint32_t v = 0; v < a.num_values; ++v) {
+            const __amdgpu_buffer_rsrc_t ri = mgpu::words_rsrc(seg_vals_in(a, s, v), n);
+            const __amdgpu_buffer_rsrc_t ro = mgpu::words_rsrc(seg_vals_out(a, s, v), n);
+            uint32_t val[IT];
+#pragma unroll
+            for (int j = 0; j < IT; ++j)
+                val[j] = __builtin_amdgcn_raw_buffer_load_b32(ri, (int)(pay[j] * 4u), 0, 0);
+            // Every gather has its data before the first store (the result
+            // side may be the input side).
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int j = 0; j < IT; ++j)
+                __builtin_amdgcn_raw_buffer_store_b32(val[j], ro, (int)((j * 64 + lane) * 4u), 0, 0);
+        }
+    }
+}
+
+// One workgroup, with the least keys per thread that hold the segment.
+template <int IPT, int BLOCK, bool PAY>
+__device__ __forceinline__ void block_sort8(const mgpuSegArgs& a, const SegArrays& s,
+                                            const mgpu::LocalMem& mem) {
+    const SegIO io{a, s};
+    const uint32_t n = s.n;
+    if (n <= 2 * BLOCK) mgpu::local_sort_items<BLOCK, 2, PAY>(io, mem, n, 0u, a.first_bit, a.num_bits);
+    else if (n <= 4 * BLOCK) mgpu::local_sort_items<BLOCK, 4, PAY>(io, mem, n, 0u, a.first_bit, a.num_bits);
+    else if (n <= 6 * BLOCK) mgpu::local_sort_items<BLOCK, 6, PAY>(io, mem, n, 0u, a.first_bit, a.num_bits);
+    else if (n <= 8 * BLOCK) mgpu::local_sort_items<BLOCK, 8, PAY>(io, mem, n, 0u, a.first_bit, a.num_bits);
+    else if constexpr (IPT > 8) {
+        if (n <= 12 * BLOCK) mgpu::local_sort_items<BLOCK, 12, PAY>(io, mem, n, 0u, a.first_bit, a.num_bits);
+        else mgpu::local_sort_items<BLOCK, 16, PAY>(io, mem, n, 0u, a.first_bit, a.num_bits);
+    }
+}
+
+// The small list, one segment per wave at a time, dealt round-robin over the
+// grid's waves.  A wave's segments are a chain of dependent reads (list,
+// descriptor, keys) and little else, so the list entry is read three segments
+// ahead, the descriptor two and the keys one.
+template <int IPT, int BLOCK, bool PAY>
+__device__ __forceinline__ void wave_phase8(const mgpuSegArgs& a, uint32_t* row, uint32_t* skey, uint32_t* spay,
+                            uint32_t lane, uint32_t wave) {
+    const uint32_t stride = gridDim.x * (BLOCK / 64);
+    const ConstWords list = (ConstWords)a.small_list;
+    uint32_t item = blockIdx.x * (BLOCK / 64) + wave;
+    if (item >= a.num_small) return;
+    const uint32_t last = a.num_small - 1;
+    const bool value = PAY && !a.index_mode && a.num_values == 1;
+    // (Of a segment of more than 512 keys the first 512: with all 16 slots the
+    // kernel took 201 registers, one workgroup of 512 threads to a CU.)
+    constexpr int AHEAD = 8;
+    uint32_t key[AHEAD], pay[PAY ? AHEAD : 1];
+    auto load = [&](const SegArrays& s) {
+        const __amdgpu_buffer_rsrc_t rk = mgpu::words_rsrc(s.ki, s.n);
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+            if (j == 0 || s.n > j * 64u)
+                key[j] = __builtin_amdgcn_raw_buffer_load_b32(rk, (int)((j * 64 + lane) * 4u), 0, 0);
+        if constexpr (PAY) {
+            if (value) {
+                const __amdgpu_buffer_rsrc_t rv = mgpu::words_rsrc(s.vi, s.n);
+#pragma unroll
+                for (int j = 0; j < AHEAD; ++j)
+                    if (j == 0 || s.n > j * 64u)
+                        pay[j] = __builtin_amdgcn_raw_buffer_load_b32(
+                            rv, (int)((j * 64 + lane) * 4u), 0, 0);
+            }
+        }
+    };
+    // (Past the end the last segment is read again and not used.)
+    SegArrays cur = seg_arrays(a, list[item]);
+    uint32_t ahead = list[min(item + stride, last)];
+    load(cur);
+    while (true) {
+        const SegArrays next = seg_arrays(a, ahead);
+        ahead = list[min(item + 2 * stride, last)];
+        const bool more = item + stride < a.num_small;
+        auto taken = [&] {
+            if (more) load(next);
+        };
+        if (cur.n <= 64) {
+            const uint32_t k = key[0], v = PAY ? pay[0] : 0u;
+            taken();
+            wave_place64(a, cur, lane, k, v);
+        } else if (cur.n <= 128) {
+            wave_sort8<2, PAY>(a, cur, row, skey, spay, lane, key, pay, taken);
+        } else if (cur.n <= 256) {
+            wave_sort8<4, PAY>(a, cur, row, skey, spay, lane, key, pay, taken);
+        } else if (IPT == 8 || cur.n <= 512) {
+            wave_sort8<8, PAY>(a, cur, row, skey, spay, lane, key, pay, taken);
+        } else {
+            wave_sort8<IPT, PAY>(a, cur, row, skey, spay, lane, key, pay, taken);
+        }
+        if (!more) break;
+        item += stride;
+        cur = next;
+    }
+}
+
 // GLOBAL: the kernel carries the one-workgroup routine for segments larger
 // than a workgroup's LDS tile.  That routine sets the kernel's register
-// count (r8, 16 keys per thread, 512 threads: 221 VGPRs and 96 bytes of
-// scratch with it, 141 and none without; 8 keys per thread: 132 -> 89), so
+// count (r8, 8 keys per thread, 512 threads: 132 VGPRs with it, and half the
+// waves of the 96 that the one without is held to), so
 // launches whose block-list segments all fit the tile take the kernel
 // without it, which fits more waves per SIMD.
 template <int RB, int IPT, int BLOCK, bool GLOBAL>
-__device__ void segsort_body(const mgpuSegArgs& a) {
+__device__ __forceinline__ void segsort_body(const mgpuSegArgs& a) {
     static_assert(BLOCK >= (1 << RB), "a thread per digit in the block scans");
     constexpr int W = BLOCK / 64;
     __shared__ SegShared<RB, IPT, BLOCK> sh;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+
+    // 8-bit digits and the ordered adds: the routines written for them.
+    const bool fast = RB == 8 && a.rank1 != 0;
+    uint32_t* const words = reinterpret_cast<uint32_t*>(sh.stage);
+    const mgpu::LocalMem mem{&sh.count[0][0], sh.tmp, words, words + SegShared<RB, IPT, BLOCK>::TILE};
 
     // Workgroup phase: block and global segments, largest first, from a
     // shared cursor.  (Dealt round-robin like the small ones below, they
@@ -494,7 +772,13 @@ __device__ void segsort_body(const mgpuSegArgs& a) {
         __syncthreads();
         if (item >= a.num_big) break;
         const mgpuSegDesc& s = a.segs[a.big_list[item]];
-        if (s.n <= (uint32_t)SegShared<RB, IPT, BLOCK>::TILE) {
+        if (fast && s.n <= (uint32_t)SegShared<RB, IPT, BLOCK>::TILE) {
+            if constexpr (RB == 8) {
+                const SegArrays io = seg_arrays(a, (uint32_t)__builtin_amdgcn_readfirstlane((int)a.big_list[item]));
+                if (a.num_values == 0) block_sort8<IPT, BLOCK, false>(a, io, mem);
+                else block_sort8<IPT, BLOCK, true>(a, io, mem);
+            }
+        } else if (s.n <= (uint32_t)SegShared<RB, IPT, BLOCK>::TILE) {
             block_sort<RB, IPT, BLOCK>(a, s, sh, tid, lane, wave);
         } else if constexpr (GLOBAL) {
             global_sort<RB, IPT, BLOCK>(a, s, sh, tid, lane, wave);
@@ -504,11 +788,22 @@ __device__ void segsort_body(const mgpuSegArgs& a) {
         __syncthreads();
     }
 
+    if constexpr (RB == 8) {
+        if (fast) {
+            const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
+            uint32_t* const slice = words + w * (2 * 64 * IPT);  // keys, then payloads
+            if (a.num_values == 0)
+                wave_phase8<IPT, BLOCK, false>(a, sh.count[w], slice, slice + 64 * IPT, lane, w);
+            else
+                wave_phase8<IPT, BLOCK, true>(a, sh.count[w], slice, slice + 64 * IPT, lane, w);
+        }
+    }
     // Wave phase: one small segment per wave at a time, dealt round-robin
     // over the grid's waves.  (A shared cursor costs a device-wide atomic on
     // one word per segment: ~25 ns each, serialized, which bounded a batch
     // of 130K segments of up to 64 keys at 3.3 ms whatever the kernel.)
-    for (uint32_t item = blockIdx.x * W + wave; item < a.num_small; item += gridDim.x * W) {
+    for (uint32_t item = fast ? a.num_small : blockIdx.x * W + wave; item < a.num_small;
+         item += gridDim.x * W) {
         const mgpuSegDesc& s = a.segs[a.small_list[item]];
         if (s.n <= 64) wave_bitonic64(a, s, lane);
         else wave_sort<RB, IPT, BLOCK>(a, s, sh, lane, wave);
@@ -531,12 +826,18 @@ __device__ void segsort_body(const mgpuSegArgs& a) {
 // Kernel variants: digit width RB (4..8 bits) x keys per thread IPT (8, 16)
 // x workgroup size BLOCK (128 for digits up to 7 bits, 256, 512), each with
 // the one-workgroup global-memory routine and without it (_ng).
+// 512 threads: at most 96 registers with 8 keys per thread, so that two
+// workgroups of a device-wide pass (80 registers, 42 KB) run beside one of
+// this kernel on a CU instead of one; at most 128 with 16, so that two fit a
+// CU (the LDS allows both).
+#define MGPU_SEG_WAVES(IPT, B) \
+    __attribute__((amdgpu_waves_per_eu(B < 512 ? 1 : IPT == 8 ? 5 : 4)))
 #define MGPU_SEGSORT(RB, IPT, B)                                                                \
     extern "C" __global__ void __launch_bounds__(B)                                            \
         mgpu_segsort_r##RB##_i##IPT##_b##B(mgpuSegArgs a) {                                    \
         segsort_body<RB, IPT, B, true>(a);                                                     \
     }                                                                                          \
-    extern "C" __global__ void __launch_bounds__(B)                                            \
+    extern "C" __global__ void __launch_bounds__(B) MGPU_SEG_WAVES(IPT, B)                        \
         mgpu_segsort_r##RB##_i##IPT##_b##B##_ng(mgpuSegArgs a) {                               \
         segsort_body<RB, IPT, B, false>(a);                                                    \
     }
