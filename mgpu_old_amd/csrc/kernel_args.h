@@ -181,12 +181,17 @@ struct mgpuSegDesc {
     uint32_t pad_;
 };
 
+// Cursors of a persistent launch, a cache line or two apart.
+#define MGPU_SEG_CURSORS 8
+#define MGPU_SEG_CURSOR_WORDS 64
+
 struct mgpuSegArgs {
     const mgpuSegDesc* segs;
     const uint32_t* big_list;    // segments for the workgroup routines, largest first
     const uint32_t* small_list;  // segments for the one-wave routine
-    uint32_t* counters;          // [0] big cursor, [2] finished workgroups ([1],
-                                 // [3] unused): zero on entry, left zero
+    uint32_t* counters;          // [MGPU_SEG_CURSORS][MGPU_SEG_CURSOR_WORDS]: words 0 (cursor
+                                 // into big_list) and 1 (workgroups done); zero on entry,
+                                 // left zero
     uint32_t* error_flag;
     uint32_t num_big;
     uint32_t num_small;

@@ -353,7 +353,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
     const int mixedWgs = mixed_workgroups_per_cu();
 
     // Device arrays: descriptors, then per group [big list | small list],
-    // then 4 counters per group.
+    // then the cursors of each group.
     std::vector<uint32_t> lists;
     for (int v = 0; v < kSegVariants; ++v) {
         Group& g = groups[v];
@@ -578,7 +578,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
     const size_t chBytes = al(sizeof(uint32_t) * chunks.size());
     const size_t tsBytes = al(sizeof(uint32_t) * tileSeg.size());
     const size_t xbBytes = al(sizeof(uint32_t) * P.xcdTileBegin.size());
-    const size_t ctrWords = 4 * std::max<size_t>(1, P.launches.size());
+    const size_t ctrWords = kSegLaunchCounters * std::max<size_t>(1, P.launches.size());
     const size_t payload = descBytes + listBytes + wideBytes + tbBytes + chBytes + tsBytes + xbBytes;
     const size_t total = payload + ctrWords * sizeof(uint32_t);
     char* base = nullptr;
@@ -824,7 +824,7 @@ sortStatus_t mgpu_seg_enqueue(SegPlanData& P, SortLane& lane) {
         a.segs = P.devSegs;
         a.big_list = P.devLists + L.bigOffset;
         a.small_list = P.devLists + L.smallOffset;
-        a.counters = P.devCounters + 4 * li;
+        a.counters = P.devCounters + kSegLaunchCounters * li;
         a.error_flag = lane.errorDev;
         a.num_big = L.numBig;
         a.num_small = L.numSmall;

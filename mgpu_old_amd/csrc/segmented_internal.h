@@ -148,7 +148,8 @@ sortStatus_t mgpu_arena_reserve(SegArena* arena, size_t payload, size_t counterW
 // Upper bound on the plan arrays of a build over `numSegments` segments
 // holding `keys` keys in total, in tiles of at least `minTile` keys.
 size_t mgpu_seg_payload_bound(uint32_t numSegments, uint64_t keys, uint32_t minTile);
-constexpr size_t kSegCounterWords = 4 * kSegVariants;
+constexpr size_t kSegLaunchCounters = MGPU_SEG_CURSORS * MGPU_SEG_CURSOR_WORDS;
+constexpr size_t kSegCounterWords = kSegLaunchCounters * kSegVariants;
 // The lane's side stream and fork/join events, on which the persistent
 // kernels of a plan run beside its device-wide passes.
 sortStatus_t mgpu_lane_ensure_side(SortLane& lane);

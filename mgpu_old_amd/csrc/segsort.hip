@@ -13,10 +13,11 @@
 //   global (larger)          one workgroup runs every pass through global
 //                            memory, tile by tile, with running digit offsets
 //                            (no cross-workgroup lookback needed).
-// Workgroups first drain the block/global list (largest first, from a
-// shared cursor), then their waves take the small list round-robin, one
-// segment per wave at a time.  The last workgroup to finish puts the cursor
-// back to zero, so a captured graph of this launch can be replayed as is.
+// Workgroups first drain the block/global list (largest first, from a cursor
+// per group of workgroups), then their waves take the small list round-robin,
+// one segment per wave at a time.  The last workgroup of a group to finish
+// puts its cursor back to zero, so a captured graph of this launch can be
+// replayed as is.
 //
 // In-LDS routines carry (key, payload) through the passes, one 64-bit LDS
 // word per slot: the payload is the value with one value array, else the
@@ -477,8 +478,8 @@ __device__ __forceinline__ void global_sort(const mgpuSegArgs& a, const mgpuSegD
 // the ranks of all slots are requested before the first is used, keys and
 // payloads lie in 32-bit words of their own, a segment takes no more slots per
 // thread than it fills, and the small list's reads run ahead of the sorts.
-// Plan replays, the routines above -> these, keys only / key + value / two
-// values, us: 60000 segments log-uniform in [1, 512] 109 -> 75 / 123 -> 85 /
+// Plan replays, the routines above -> these (with one cursor for all
+// workgroups), keys only / key + value / two values, us: 60000 segments log-uniform in [1, 512] 109 -> 75 / 123 -> 85 /
 // 135 -> 95; 130000 in [1, 64] 143 -> 85 / 162 -> 98 / 186 -> 112; 20000 in
 // [64, 4096] 297 -> 186 / 357 -> 214 / 411 -> 261; 5000 of 512 105 -> 72 /
 // 125 -> 79 / 134 -> 85.
@@ -742,8 +743,7 @@ __device__ __forceinline__ void wave_phase8(const mgpuSegArgs& a, uint32_t* row,
 
 // GLOBAL: the kernel carries the one-workgroup routine for segments larger
 // than a workgroup's LDS tile.  That routine sets the kernel's register
-// count (r8, 8 keys per thread, 512 threads: 132 VGPRs with it, and half the
-// waves of the 96 that the one without is held to), so
+// count (r8, 8 keys per thread, 512 threads: 149 VGPRs with it, 96 without), so
 // launches whose block-list segments all fit the tile take the kernel
 // without it, which fits more waves per SIMD.
 template <int RB, int IPT, int BLOCK, bool GLOBAL>
@@ -758,19 +758,27 @@ __device__ __forceinline__ void segsort_body(const mgpuSegArgs& a) {
     uint32_t* const words = reinterpret_cast<uint32_t*>(sh.stage);
     const mgpu::LocalMem mem{&sh.count[0][0], sh.tmp, words, words + SegShared<RB, IPT, BLOCK>::TILE};
 
-    // Workgroup phase: block and global segments, largest first, from a
-    // shared cursor.  (Dealt round-robin like the small ones below, they
-    // measured slower where they are many: 20000 segments log-uniform in
-    // [2^6, 2^12] 0.44 -> 0.68 ms, since a workgroup that starts late still
-    // holds a full share; an atomic per segment of this size is cheap.)
-    while (true) {
-        if (tid == 0)
-            sh.item = __hip_atomic_fetch_add(&a.counters[0], 1u, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        const uint32_t item = sh.item;
-        __syncthreads();
-        if (item >= a.num_big) break;
+    // Workgroup phase: block and global segments, largest first.  The first
+    // of a workgroup is its own number; the others it draws from a counter of
+    // its group (workgroups of the same number modulo the groups: with 8, of
+    // one XCD), asked for before the segment at hand is sorted.  One counter
+    // for all served a draw in ~25 ns, so 3000 segments of 4096 keys took the
+    // 75 us of that queue and more, and every launch paid for counting its
+    // workgroups out: plan replays, one counter -> these, keys only / key +
+    // value, us: 3000 of 4096 125 -> 88 / 143 -> 106; 16000 in [1, 8192] 156 ->
+    // 120 / 183 -> 138; 5000 of 512 (nothing drawn) 72 -> 46 / 79 -> 52; 60000
+    // in [1, 512] 76 -> 63 / 85 -> 69.
+    // (Dealt round-robin like the small ones below, they measured slower where
+    // they are many: 20000 segments log-uniform in [2^6, 2^12] 0.44 -> 0.68
+    // ms, since a workgroup that starts late still holds a full share.)
+    const uint32_t groups = gridDim.x % MGPU_SEG_CURSORS == 0 ? MGPU_SEG_CURSORS : 1u;
+    const uint32_t group = blockIdx.x % groups;
+    uint32_t* const cursor = a.counters + group * MGPU_SEG_CURSOR_WORDS;
+    const bool draws = a.num_big > gridDim.x;
+    for (uint32_t item = blockIdx.x; item < a.num_big;) {
+        uint32_t drawn = 0;
+        if (draws && tid == 0)
+            drawn = __hip_atomic_fetch_add(&cursor[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const mgpuSegDesc& s = a.segs[a.big_list[item]];
         if (fast && s.n <= (uint32_t)SegShared<RB, IPT, BLOCK>::TILE) {
             if constexpr (RB == 8) {
@@ -785,6 +793,13 @@ __device__ __forceinline__ void segsort_body(const mgpuSegArgs& a) {
         } else if (tid == 0) {
             mgpu::set_error(a.error_flag, 7u);  // the host never sends one here
         }
+        if (!draws) {
+            __syncthreads();
+            break;
+        }
+        if (tid == 0) sh.item = gridDim.x + drawn * groups + group;
+        __syncthreads();
+        item = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.item);
         __syncthreads();
     }
 
@@ -809,14 +824,13 @@ __device__ __forceinline__ void segsort_body(const mgpuSegArgs& a) {
         else wave_sort<RB, IPT, BLOCK>(a, s, sh, lane, wave);
     }
 
-    __syncthreads();
-    if (tid == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const uint32_t done = __hip_atomic_fetch_add(&a.counters[2], 1u, __ATOMIC_ACQ_REL,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
-        if (done == gridDim.x - 1) {  // every workgroup is past both queues
-            st_agent(&a.counters[0], 0u);
-            st_agent(&a.counters[2], 0u);
+    // The last of the group to be done drawing puts its cursor back.
+    if (draws && tid == 0) {
+        const uint32_t done =
+            __hip_atomic_fetch_add(&cursor[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (done == gridDim.x / groups - 1) {
+            st_agent(&cursor[0], 0u);
+            st_agent(&cursor[1], 0u);
         }
     }
 }

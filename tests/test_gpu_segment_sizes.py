@@ -80,6 +80,17 @@ def test_many_small_segments(engine, oracle, vc):
     _run(engine, oracle, list(rng.integers(1, 90, 9001)), vc, 0, 32, seed=73)
 
 
+@pytest.mark.parametrize("variant", [None, "r8i16", "r7i8"])
+def test_many_workgroup_segments(engine, oracle, variant, monkeypatch):
+    """More workgroup segments than workgroups: drawn from the cursors, which
+    every launch leaves as it found them."""
+    if variant:
+        monkeypatch.setenv("MGPUSORT_SEG_VARIANT", variant)
+    rng = np.random.default_rng(6)
+    for seed in (75, 76):
+        _run(engine, oracle, list(rng.integers(1025, 1200, 2101)), 1, 0, 32, seed=seed)
+
+
 @pytest.mark.parametrize("sizes,device_wide", [
     ([8192, 4097, 100], False),
     ([8192, 8193, 100], True),          # longer segments hold more keys
