@@ -133,6 +133,7 @@ struct sortEngine_d {
     // size).
     hipFunction_t fnLocal = nullptr;
     hipFunction_t fnLocalPay = nullptr;
+    hipFunction_t fnSegSlots[2][2] = {};  // [512, 1024 threads][values]: buckets and segments
     hipFunction_t fnMidCount = nullptr;  // counts of a bucketed sort (null as above)
     hipFunction_t fnIota = nullptr;
     hipFunction_t fnKeyTransform = nullptr;

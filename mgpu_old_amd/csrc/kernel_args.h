@@ -121,7 +121,10 @@ struct mgpuScanArgs {
 #define MGPU_UNSORTED_SLOT (MGPU_FINISHED_SLOT + MGPU_MAX_PASSES)
 // Most frequent digit of each pass (segments per XCD only; digit_scan).
 #define MGPU_MODE_SLOT (MGPU_UNSORTED_SLOT + 8)
-#define MGPU_LANE_COUNTERS (MGPU_MODE_SLOT + MGPU_MAX_PASSES)
+// Segments of the last device-wide count that take every digit pass (not
+// zeroed with the counters before it: the bucket kernel zeroes it).
+#define MGPU_LSD_SLOT (MGPU_MODE_SLOT + MGPU_MAX_PASSES)
+#define MGPU_LANE_COUNTERS (MGPU_LSD_SLOT + 2)
 
 // iota: out[i] = i for i < n (index output of a sort that needs no pass).
 struct mgpuIotaArgs {
@@ -178,7 +181,10 @@ struct mgpuSegDesc {
     uint32_t* keys[2];
     uint32_t* vals[MGPU_MAX_VALUES][2];
     uint32_t n;
-    uint32_t pad_;
+    // Device-wide segments: the field that the bucketed passes scatter by, as
+    // the count kernel chose it (bit 31, shift, width << 8); 0: every digit
+    // pass in turn.
+    uint32_t route;
 };
 
 // Cursors of a persistent launch, a cache line or two apart.
@@ -220,7 +226,7 @@ struct mgpuSegArgs {
 // array `seg`, read from side 0.
 struct mgpuMultiCountArgs {
     const mgpuSegDesc* segs;
-    const uint32_t* chunks;  // [num_chunks][4]: seg, begin, end, unused
+    const uint32_t* chunks;  // [num_chunks][4]: seg, begin, end, bucket size (direct; 0: none)
     uint32_t* hist;          // [num_segs][MGPU_MAX_PASSES][MGPU_RADIX], zero on entry
     uint32_t* clear;         // lookback words to zero
     uint64_t clear_words;    // multiple of 4
@@ -234,6 +240,31 @@ struct mgpuMultiCountArgs {
     uint32_t* digit_start;    // [num_segs][MGPU_MAX_PASSES][MGPU_RADIX]
     uint32_t* tile_counters;  // [MGPU_LANE_COUNTERS]
     uint32_t direct;
+    uint32_t pad_;
+    // Direct counts with a bucket size T: an array whose keys the highest
+    // digit that is not constant spreads into bins small enough gets its route
+    // (mgpuSegDesc), that digit's starts in the first row of its digit_start
+    // block and, in the second, a bucket per T keys (uint4: first key, keys,
+    // bits to sort by, base); any other adds one to *lsd_segments.
+    uint32_t* lsd_segments;
+};
+
+// A workgroup per slot, of 512 threads (up to MGPU_BUCKET_KEYS keys) or 1024: a bucket of a device-wide segment, or
+// a whole segment (MGPU_SLOT_WHOLE: seg indexes segs, else wide).
+#define MGPU_SLOT_WHOLE 0xFFFFFFFFu
+#define MGPU_BUCKET_THREADS 512
+#define MGPU_BUCKET_KEYS 8192
+struct mgpuSegSlotArgs {
+    const mgpuSegDesc* segs;
+    const mgpuSegDesc* wide;
+    const uint32_t* slots;        // [grid][2]: seg, bucket
+    const uint32_t* digit_start;  // blocks of the device-wide segments, as above
+    uint32_t* lsd_segments;       // zeroed
+    uint32_t num_values;
+    uint32_t index_mode;
+    uint32_t result_side;
+    uint32_t first_bit;
+    uint32_t num_bits;
     uint32_t pad_;
 };
 
@@ -285,6 +316,9 @@ struct mgpuMultiPassArgs {
     // bits 16-23: chunks holding keys (the rest are padding), bit 24: the
     // first chunk continues an array begun in an earlier tile.
     const uint32_t* tile_info;
+    // Bucketed batches, passes after the first: the count of segments that
+    // take them (the launch returns at once when it is zero).
+    const uint32_t* lsd_segments;
 };
 
 // Parts (arrays) per packed tile of W waves.

@@ -182,11 +182,10 @@ __device__ __forceinline__ void local_sort_items(const IO& io, const LocalMem& s
     }
 }
 
-// The same with the least IT that holds n <= 16 * kLocalBlock elements.
-template <bool PAY, typename IO>
+// The same with the least IT that holds n <= 16 * B elements.
+template <bool PAY, int B = kLocalBlock, typename IO>
 __device__ __forceinline__ void local_sort(const IO& io, const LocalMem& sh, uint32_t n,
                                            uint32_t base, uint32_t shift, uint32_t bits) {
-    constexpr int B = kLocalBlock;
     if (n <= 1 * B) local_sort_items<B, 1, PAY>(io, sh, n, base, shift, bits);
     else if (n <= 2 * B) local_sort_items<B, 2, PAY>(io, sh, n, base, shift, bits);
     else if (n <= 4 * B) local_sort_items<B, 4, PAY>(io, sh, n, base, shift, bits);

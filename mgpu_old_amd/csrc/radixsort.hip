@@ -624,6 +624,74 @@ __device__ void multi_count_body(const mgpuMultiCountArgs& a) {
     }
 }
 
+// Buckets of an array of n keys whose digit counts the 1024 threads hold
+// (thread (p, d): `sum` keys of digit d of pass p, `ex` before them): bucket j
+// is the bins of the highest digit that is not constant whose first key lies
+// in [j * T, (j + 1) * T), so less than T keys and the rest of its last bin.
+// Where all digits are constant, every T keys as they lie.  False where a
+// bucket is more than a workgroup sorts: the array takes every pass.
+__device__ __forceinline__ bool plan_buckets(const mgpuMultiCountArgs& a, uint32_t sg, uint32_t n,
+                                             uint32_t T, uint32_t p, uint32_t d, uint32_t sum,
+                                             uint32_t ex, uint32_t* starts) {
+    __shared__ uint32_t s_max[16], s_ex[RADIX], s_bin[RADIX + 1];
+    const uint32_t tid = threadIdx.x;
+    uint32_t most = sum;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, o, 64));
+    if ((tid & 63u) == 0) s_max[tid >> 6] = most;
+    __syncthreads();
+    uint32_t pick = MGPU_MAX_PASSES, shift = 0, width = 0;
+#pragma unroll
+    for (int q = 0; q < MGPU_MAX_PASSES; ++q) {
+        const uint32_t m =
+            max(max(s_max[4 * q], s_max[4 * q + 1]), max(s_max[4 * q + 2], s_max[4 * q + 3]));
+        if ((uint32_t)q < a.num_passes && m < n) {
+            pick = (uint32_t)q;
+            shift = a.shift[q];
+            width = (uint32_t)__builtin_popcount(a.mask[q]);
+        }
+    }
+    const bool constant = pick == MGPU_MAX_PASSES;
+    const uint32_t buckets = (n + T - 1) / T;  // at most 64 (the host's choice of T)
+    if (p == pick) s_ex[d] = ex;
+    __syncthreads();
+    if (p == pick) {
+        // First bin of each bucket that starts here (none but this one, or
+        // buckets left empty by a bin of more than T keys).
+        const uint32_t b = ex / T;
+        for (uint32_t j = d == 0 ? 0u : s_ex[d - 1] / T + 1; j <= b; ++j) s_bin[j] = d;
+        if (d == RADIX - 1)
+            for (uint32_t j = b + 1; j <= buckets; ++j) s_bin[j] = RADIX;
+    }
+    __syncthreads();
+    uint4 bucket = make_uint4(0u, 0u, 0u, 0u);
+    if (tid < buckets) {
+        if (constant) {
+            bucket = make_uint4(tid * T, min(T, n - tid * T), 0u, 0u);
+        } else {
+            // (No bins past the digit's own: a bit above it is not sorted by.)
+            const uint32_t end = 1u << width;
+            const uint32_t b0 = min(s_bin[tid], end), b1 = min(s_bin[tid + 1], end);
+            const uint32_t bins = b1 - b0;
+            const uint32_t at = b0 < end ? s_ex[b0] : n, to = b1 < end ? s_ex[b1] : n;
+            const uint32_t more = bins > 1 ? 32u - (uint32_t)__builtin_clz(bins - 1) : 0u;
+            bucket = make_uint4(at, to - at, shift - a.shift[0] + more,
+                                b0 < end ? b0 << shift : 0u);
+        }
+    }
+    const bool fits = __syncthreads_or(bucket.y > MGPU_BUCKET_KEYS) == 0;
+    mgpuSegDesc* const desc = const_cast<mgpuSegDesc*>(a.segs) + sg;
+    if (tid == 0) {
+        desc->route = fits ? 1u << 31 | width << 8 | shift : 0u;
+        if (!fits)
+            __hip_atomic_fetch_add(a.lsd_segments, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!fits) return false;
+    if (p == pick || (constant && tid == 0)) starts[d] = ex;  // (digit 0 for all, from 0)
+    if (tid < buckets) reinterpret_cast<uint4*>(starts + RADIX)[tid] = bucket;
+    return true;
+}
+
 // The same over whole arrays (or 64K-key pieces of larger ones), one
 // 1024-thread workgroup each, with lane-column histograms: per (pass, digit
 // pair) a row of 32 words, word c counting the keys of the lanes with
@@ -728,8 +796,12 @@ __device__ void multi_count_cols_body(const mgpuMultiCountArgs& a) {
         // counters, as that launch would.
         __shared__ uint32_t s_tmp[BLOCK / 64];
         const uint32_t ex = group_exclusive_scan<BLOCK>(sum, s_tmp, tid & 63, tid >> 6);
-        if (p < np) a.digit_start[((size_t)sg * MGPU_MAX_PASSES + p) * RADIX + d] = ex;
-        if (blockIdx.x == 0 && tid < MGPU_LANE_COUNTERS) a.tile_counters[tid] = 0;
+        uint32_t* const starts = a.digit_start + (size_t)sg * MGPU_MAX_PASSES * RADIX;
+        if (blockIdx.x == 0 && tid < MGPU_LSD_SLOT) a.tile_counters[tid] = 0;
+        const uint32_t T = ch[3];
+        if (T == 0 || !plan_buckets(a, sg, end, T, p, d, sum, ex, starts)) {
+            if (p < np) starts[p * RADIX + d] = ex;
+        }
     } else if (sum) {
         __hip_atomic_fetch_add(&a.hist[((size_t)sg * MGPU_MAX_PASSES + p) * RADIX + d], sum,
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -746,7 +818,7 @@ __device__ void multi_scan_body(const mgpuMultiScanArgs& a) {
         a.digit_start[base + p * RADIX + tid] = e;
         a.hist[base + p * RADIX + tid] = 0;
     }
-    if (blockIdx.x == 0 && tid < MGPU_LANE_COUNTERS) a.tile_counters[tid] = 0;
+    if (blockIdx.x == 0 && tid < MGPU_LSD_SLOT) a.tile_counters[tid] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1193,6 +1265,11 @@ __device__ void rank_scatter_body(const Args& a) {
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     uint32_t shift = a.shift, mask = a.mask;
     uint32_t width = (uint32_t)__builtin_popcount(mask);  // mask = 2^width - 1
+    // One tile per workgroup, of several arrays: passes of a bucketed batch.
+    constexpr bool ROUTED = MULTI && RANK == 1 && !XSEG;
+    if constexpr (ROUTED) {
+        if (a.lsd_segments != nullptr && *a.lsd_segments == 0) return;
+    }
     __shared__ uint32_t s_map[MID == 1 ? MGPU_MID_BINS : 1];  // bin (or digit) -> digit
     uint32_t* const row = s_count[wave];  // this wave's digit counts
     const uint32_t gd = tid / G, gk = tid % G;
@@ -1368,6 +1445,23 @@ __device__ void rank_scatter_body(const Args& a) {
         if (tid < RADIX) mid_digit0 = a.mid_hist[MGPU_MID_BINS + tid];
     }
     TileJob job{};
+    // Starts on tile g; ROUTED: false where the first pass scattered its array
+    // into buckets and this is a later one.
+    auto start_tile = [&](uint32_t g) -> bool {
+        job = posted_job(g);
+        if constexpr (ROUTED) {
+            const uint32_t route =
+                ((const __attribute__((address_space(4))) mgpuSegDesc*)job.sd)->route;
+            if (route != 0) {
+                if (a.pass != 0) return false;
+                shift = route & 0xFFu;
+                width = (route >> 8) & 0xFFu;
+                mask = (1u << width) - 1u;
+            }
+        }
+        load_tile(job);
+        return true;
+    };
     uint32_t gtile;
     if constexpr (MID == 3) {
         gtile = take_item(job) ? 0u : seg_tiles;
@@ -1377,10 +1471,7 @@ __device__ void rank_scatter_body(const Args& a) {
         gtile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
         // One tile per workgroup: only a counter left dirty finds none.
         if (!XSEG && gtile >= seg_tiles && tid == 0) set_error(a.error_flag, 2u);
-        if (gtile < seg_tiles) {
-            job = posted_job(gtile);
-            load_tile(job);
-        }
+        if (gtile < seg_tiles && !start_tile(gtile)) gtile = seg_tiles;
     }
     if constexpr (MID == 1)
         mapped = mid_plan_tile<BLOCK>(a, mid_bins, mid_digit0, s_map, s_global, s_tmp, s_stage, shift, width,
@@ -1689,10 +1780,7 @@ __device__ void rank_scatter_body(const Args& a) {
         if (tid == 0) post_tile(take_tile());
         __syncthreads();  // (every read of this tile's stage is done, too)
         gtile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
-        if (gtile < seg_tiles) {
-            job = posted_job(gtile);
-            load_tile(job);
-        }
+        if (gtile < seg_tiles) start_tile(gtile);
         clear_counts();  // (the value stage wrote over the match masks)
     }  // while
 

@@ -33,6 +33,12 @@ constexpr long kTileCounterGroups = 8;
 // its digit starts directly (a 2^18-key segment: 1 MB, a few microseconds).
 constexpr uint32_t kDirectCountMax = 1u << 18;
 
+// Keys of a bucket of a device-wide segment, about (its last bin can make it
+// longer: see plan_buckets), where the batch is large and small, and keys of a
+// batch from which its device-wide segments go through buckets.
+constexpr uint32_t kBucketMaxKeys = 5632, kBucketMinKeys = 4096;
+constexpr uint64_t kBucketedMinTotal = 1u << 18;
+
 // Segments of at least wide.minKeys keys go to the device-wide passes (all
 // of them together, each spread over many workgroups with a lookback chain)
 // instead of one workgroup each.  Above 4096 keys (the largest a 256-thread
@@ -144,6 +150,14 @@ sortStatus_t mgpu_seg_load(sortEngine_d* e) {
         }
     }
 
+    for (int b = 0; b < 2; ++b)
+        for (int v = 0; v < 2; ++v) {
+            const std::string name = std::string("mgpu_seg_slots_b") + (b ? "1024" : "512") + (v ? "_kv" : "_k");
+            if (hipModuleGetFunction(&e->fnSegSlots[b][v], e->segModule, name.c_str()) != hipSuccess)
+                return SORT_STATUS_KERNEL_ERROR;
+            e->kernelNames[e->fnSegSlots[b][v]] = name;
+        }
+
     // Tuning table: kernelPath + "mgpusort_seg_tuning.txt" when present
     // (written by the autotuner), else the built-in default.  Rows
     // "<max ceil(log2 n)> <radix bits> <keys per thread> [<threads>]" pick the
@@ -226,32 +240,45 @@ void pick_variant(const sortEngine_d* e, uint32_t n, int* rb, int* ipt, int* blo
 bool seg_fits_tile(const sortEngine_d* e, uint32_t n) {
     int rb, ipt, block;
     pick_variant(e, n, &rb, &ipt, &block);
-    return rb == 8 && n <= (uint32_t)(block * ipt) && n <= e->segWide.keepKeys;
+    return rb == 8 && n <= (uint32_t)(block * ipt);
 }
 
-// Segments of wide.minKeys keys or more, up to wide.keepKeys, that fit the
-// tile of the kernel the table gives them (the shipped one: 8192 keys with 16
-// keys per thread) stay with one workgroup each, in one launch, while the batch's still longer segments hold
-// at most as many keys as they do.  With more than that the device-wide passes
-// run over most of the keys anyway, and the shorter segments cost less in them
-// than in a kernel beside them that holds 80 KB of LDS on every CU.
-// MGPUSORT_SEG_WIDE_MIN sends all of its segments to the device-wide passes.
-// Plan replays, device-wide -> one workgroup each, keys only / key + value /
-// two values, us: 40 segments in [4097, 8192] 46 -> 30 / 53 -> 29 / 73 -> 33;
-// 3000 in [4097, 9000] 296 -> 254 / 440 -> 308 / 816 -> 415; 16000 log-uniform
-// in [1, 8192] 220 -> 156 / 271 -> 183 / 398 -> 218; 8000 in [64, 10000] 236 ->
-// 196 / 308 -> 235 / 487 -> 315; past the line the two come out alike (6000 in
-// [64, 16384] 272 / 268, 4096 in [1, 2^16] 321 / 333 us, keys only).
-bool keep_in_workgroups(const sortEngine_d* e, const mgpuSegDesc* segs, int numSegments,
-                        uint32_t wideMin) {
-    if (e->segWide.keepKeys < wideMin || std::getenv("MGPUSORT_SEG_WIDE_MIN") != nullptr ||
-        e->rankMethod != 1)
-        return false;
-    uint64_t fit = 0, longer = 0;
-    for (int i = 0; i < numSegments; ++i)
-        if (segs[i].n >= wideMin)
-            (seg_fits_tile(e, segs[i].n) ? fit : longer) += segs[i].n;
-    return longer <= fit;
+// Segments of wide.minKeys keys or more, up to this many, are sorted whole by
+// a workgroup each (0: none).  MGPUSORT_SEG_WIDE_MIN sends all
+// of its segments to the device-wide passes.  A batch with no segment above
+// the persistent kernels' tile (8192 keys) stays with them: 16000 segments
+// log-uniform in [1, 8192] 120 us, key + value 138, against 166 and 163 with
+// those above 4096 in workgroups of 1024 beside them.  Otherwise, plan
+// replays, device-wide passes -> whole, keys only / key + value / two values,
+// us: 2000 segments log-uniform in [2^10, 2^14] 201 -> 100 / 231 -> 111 / 354 ->
+// 144; 3000 in [4097, 9000] 247 -> 116 / 295 -> 154 / 402 -> 199.  Up to 8192
+// keys with 512 threads, two workgroups to a CU, so that one reads or writes
+// while the other sorts: against 1024 threads, one to a CU, those two 125 ->
+// 100 / 133 -> 111 and 161 -> 116 / 191 -> 154.
+uint32_t keep_in_workgroup(const sortEngine_d* e) {
+    if (e->rankMethod != 1 || std::getenv("MGPUSORT_SEG_WIDE_MIN") != nullptr) return 0;
+    return std::min<uint32_t>(e->segWide.keepKeys, MGPU_LOCAL_MAX_KEYS);
+}
+
+// Whether the batch's device-wide segments go through buckets: one scatter by
+// a segment's highest digit, then a workgroup's sort of each bucket, in place
+// of a scatter per digit (plan_buckets says which segments do; the launches of
+// the later digits return at once when all do).  For three digits and more,
+// where the count reads segments whole and one chain per segment with a tile
+// per workgroup serves.  Plan replays, passes -> buckets (with whole segments
+// up to 16384 keys beside them), keys only / key + value / two values, us:
+// 4096 segments log-uniform in [1, 2^16] 318 -> 239 / 528 -> 329 / 904 -> 411;
+// 512 in [2^15, 2^17] 400 -> 316 / 629 -> 452 / 905 -> 543; 32 of 32768 61 ->
+// 51 / 70 -> 58 / 106 -> 64; 8 of 32768 53 -> 44 / 61 -> 48; equal keys 344 ->
+// 172 / 515 -> 235 us (4096 segments).  Keys with two thirds in one digit
+// value, which take every pass, 512 in [2^15, 2^17] 515 -> 548 / 725 -> 787:
+// the chains per XCD that they would take otherwise.  Below 2^18 keys the
+// launches are what counts, and the passes have no more of them.
+bool use_buckets(const sortEngine_d* e, const SegPlanData& P, int packMode, uint64_t wideKeys) {
+    const char* v = std::getenv("MGPUSORT_SEG_XCD");
+    if (v && v[0] == '1' && v[1] == 0) return false;  // chains per XCD were asked for
+    return e->rankMethod == 1 && packMode != 1 && P.sortPasses > 2 &&
+           wideKeys >= kBucketedMinTotal;
 }
 
 }  // namespace
@@ -280,7 +307,8 @@ size_t mgpu_seg_payload_bound(uint32_t numSegments, uint64_t keys, uint32_t minT
     const size_t tiles = keys / std::max(1u, minTile) + segs + MGPU_MAX_SEGS;
     return 2 * al(sizeof(mgpuSegDesc) * segs) + al(sizeof(uint32_t) * segs) +
            al(sizeof(uint32_t) * (segs + 1)) + al(4 * sizeof(uint32_t) * chunks) +
-           al(2 * sizeof(uint32_t) * tiles) + al(sizeof(uint32_t) * (MGPU_MAX_SEGS + 1));
+           al(2 * sizeof(uint32_t) * tiles) + al(sizeof(uint32_t) * (MGPU_MAX_SEGS + 1)) +
+           al(2 * sizeof(uint32_t) * (keys / kBucketMinKeys + segs));
 }
 
 sortStatus_t mgpu_arena_reserve(SegArena* arena, size_t payload, size_t counterWords,
@@ -328,16 +356,26 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
 
     // Group segments by kernel variant; very large ones go device-wide.
     const uint32_t wideMin = device_wide_min(e), chunkKeys = wide_chunk(e);
-    const bool keepFit = keep_in_workgroups(e, segs, numSegments, wideMin);
+    const uint32_t keep = keep_in_workgroup(e);
+    uint32_t longestSeg = 0;
+    for (int i = 0; i < numSegments; ++i) longestSeg = std::max(longestSeg, segs[i].n);
+    const bool noneAboveTile = longestSeg <= keep && seg_fits_tile(e, longestSeg);
     struct Group {
         std::vector<uint32_t> big, small;
     };
     Group groups[kSegVariants];
+    std::vector<uint32_t> slots1024;
     for (int i = 0; i < numSegments; ++i) {
         const uint32_t n = segs[i].n;
         if (n == 0 || P.numBits == 0) continue;
-        if (n >= wideMin && !(keepFit && seg_fits_tile(e, n))) {
-            P.wide.push_back((uint32_t)i);
+        if (n >= wideMin && !noneAboveTile) {
+            if (n <= keep) {
+                auto& list = n <= MGPU_BUCKET_KEYS ? P.slots : slots1024;
+                list.push_back((uint32_t)i);
+                list.push_back(MGPU_SLOT_WHOLE);
+            } else {
+                P.wide.push_back((uint32_t)i);
+            }
             continue;
         }
         int rb, ipt, block;
@@ -420,6 +458,14 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         // barrier per tile), and when no segment outweighs a quarter of an
         // XCD's share (else one XCD would do most of the work).
         // MGPUSORT_SEG_XCD=0|1 forces the choice.
+        // The count reads each segment as one piece and writes its digit
+        // starts itself when no segment is longer than kDirectCountMax keys
+        // (one workgroup per segment stays short) and no piece size was
+        // asked for; else pieces of chunkKeys with a histogram in global
+        // memory and a scan launch after them.
+        P.wideDirectCount = count_cols() && longestSeg <= kDirectCountMax &&
+                            std::getenv("MGPUSORT_SEG_WIDE_CHUNK") == nullptr;
+        P.wideBuckets = P.wideDirectCount && use_buckets(e, P, packMode, wideKeys);
         P.wideXcds = 1;
         P.xcdTileBegin.clear();
         std::vector<size_t> groupEnd(1, P.wide.size());  // end of each XCD's segments
@@ -458,7 +504,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
                 most = std::max(most, t);
             }
             const char* force = std::getenv("MGPUSORT_SEG_XCD");
-            bool use = most * 4 * X <= total && total >= kXcdMinTiles * P.wide.size();
+            bool use = !P.wideBuckets && most * 4 * X <= total && total >= kXcdMinTiles * P.wide.size();
             if (force && (force[0] == '0' || force[0] == '1') && force[1] == 0)
                 use = force[0] == '1' && most * 4 * X <= total;
             if (use) {
@@ -482,29 +528,35 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
             }
         }
         P.widePacked = P.wideVariant->packed[MGPU_VALUES_NONE] != nullptr &&
-                       (packMode == 1 || (packMode == -1 && P.wideXcds == 1));
-        // The count reads each segment as one piece and writes its digit
-        // starts itself when no segment is longer than kDirectCountMax keys
-        // (one workgroup per segment stays short) and no piece size was
-        // asked for; else pieces of chunkKeys with a histogram in global
-        // memory and a scan launch after them.
-        uint32_t longest = 0;
-        for (uint32_t k : P.wide) longest = std::max(longest, segs[k].n);
-        P.wideDirectCount = count_cols() && longest <= kDirectCountMax &&
-                            std::getenv("MGPUSORT_SEG_WIDE_CHUNK") == nullptr;
-        const uint32_t pieceKeys = P.wideDirectCount ? longest : chunkKeys;
+                       (packMode == 1 ||
+                        (packMode == -1 && P.wideXcds == 1 && !P.wideBuckets));
+        const uint32_t pieceKeys = P.wideDirectCount ? longestSeg : chunkKeys;
+        const uint32_t bucketCap = (uint32_t)std::min<uint64_t>(
+            kBucketMaxKeys,
+            std::max<uint64_t>(kBucketMinKeys, wideKeys / (2 * (uint64_t)e->numCUs)));
         // Pieces longest first: workgroups start in about launch order, so
         // the longest counts start first and the short ones fill in behind
         // them (greedy longest-processing-time order).  4096 segments
         // log-uniform in [1, 2^16]: count of the 1,007 device-wide ones
         // 61 -> 51 us alone, replay 0.598 -> 0.586 ms.
-        struct Piece { uint32_t seg, begin, end; };
+        struct Piece { uint32_t seg, begin, end, bucket; };
         std::vector<Piece> pieces;
         for (size_t k = 0; k < P.wide.size(); ++k) {
             const mgpuSegDesc& d = segs[P.wide[k]];
             wideDescs.push_back(d);
+            wideDescs.back().route = 0;
+            uint32_t bucket = 0;
+            if (P.wideBuckets) {
+                const uint32_t want = (d.n + bucketCap - 1) / bucketCap;
+                bucket = (d.n + want - 1) / want;
+                const uint32_t buckets = (d.n + bucket - 1) / bucket;
+                for (uint32_t j = 0; j < buckets; ++j) {
+                    P.slots.push_back((uint32_t)k);
+                    P.slots.push_back(j);
+                }
+            }
             for (uint32_t b = 0; b < d.n; b += pieceKeys)
-                pieces.push_back({(uint32_t)k, b, std::min(d.n, b + pieceKeys)});
+                pieces.push_back({(uint32_t)k, b, std::min(d.n, b + pieceKeys), bucket});
         }
         std::stable_sort(pieces.begin(), pieces.end(), [](const Piece& x, const Piece& y) {
             return x.end - x.begin > y.end - y.begin;
@@ -513,7 +565,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
             chunks.push_back(c.seg);
             chunks.push_back(c.begin);
             chunks.push_back(c.end);
-            chunks.push_back(0);
+            chunks.push_back(c.bucket);
         }
         if (P.widePacked) {
             // Wave chunks back to back, `waves` to a tile.  A segment that
@@ -578,8 +630,12 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
     const size_t chBytes = al(sizeof(uint32_t) * chunks.size());
     const size_t tsBytes = al(sizeof(uint32_t) * tileSeg.size());
     const size_t xbBytes = al(sizeof(uint32_t) * P.xcdTileBegin.size());
+    P.slots1024 = (uint32_t)(P.slots.size() / 2);
+    P.slots.insert(P.slots.end(), slots1024.begin(), slots1024.end());
+    const size_t slBytes = al(sizeof(uint32_t) * P.slots.size());
     const size_t ctrWords = kSegLaunchCounters * std::max<size_t>(1, P.launches.size());
-    const size_t payload = descBytes + listBytes + wideBytes + tbBytes + chBytes + tsBytes + xbBytes;
+    const size_t payload = descBytes + listBytes + wideBytes + tbBytes + chBytes + tsBytes + xbBytes + slBytes;
+    const size_t slOff = payload - slBytes;
     const size_t total = payload + ctrWords * sizeof(uint32_t);
     char* base = nullptr;
     if (!arena) {
@@ -610,6 +666,10 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
             hipMemcpy(base + off + wideBytes + tbBytes + chBytes + tsBytes, P.xcdTileBegin.data(),
                       sizeof(uint32_t) * P.xcdTileBegin.size(), hipMemcpyHostToDevice) != hipSuccess)
             return SORT_STATUS_DEVICE_ERROR;
+        if (!P.slots.empty() && hipMemcpy(base + slOff, P.slots.data(),
+                                          sizeof(uint32_t) * P.slots.size(),
+                                          hipMemcpyHostToDevice) != hipSuccess)
+            return SORT_STATUS_DEVICE_ERROR;
         // Stream-ordered before the launches on the lane's stream (a plain
         // hipMemset would run on the null stream, unordered with a
         // non-blocking lane stream).
@@ -635,6 +695,8 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
                 std::memcpy(h + off + wideBytes + tbBytes + chBytes + tsBytes,
                             P.xcdTileBegin.data(), sizeof(uint32_t) * P.xcdTileBegin.size());
         }
+        if (!P.slots.empty())
+            std::memcpy(h + slOff, P.slots.data(), sizeof(uint32_t) * P.slots.size());
         if (hipMemcpyAsync(base, h, payload, hipMemcpyHostToDevice, lane.stream) != hipSuccess)
             return SORT_STATUS_DEVICE_ERROR;
         P.devCounters = reinterpret_cast<uint32_t*>(base + arena->hostBytes);
@@ -649,6 +711,8 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         reinterpret_cast<uint32_t*>(base + descBytes + listBytes + wideBytes + tbBytes + chBytes);
     P.devXcdTileBegin = reinterpret_cast<uint32_t*>(base + descBytes + listBytes + wideBytes +
                                                     tbBytes + chBytes + tsBytes);
+
+    P.devSlots = reinterpret_cast<uint32_t*>(base + slOff);
 
     // Device-wide segments: lookback words and per-array scratch before any
     // capture.
@@ -674,7 +738,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         if (st) return st;
     }
     // The side stream (before any capture) when there is something to fork.
-    if (!lane.noSide && !P.launches.empty() && !P.wide.empty()) {
+    if (!lane.noSide && !P.launches.empty() && (!P.wide.empty() || !P.slots.empty())) {
         sortStatus_t st = mgpu_lane_ensure_side(lane);
         if (st) return st;
     }
@@ -682,6 +746,11 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
 }
 
 namespace {
+
+uint32_t* wide_digit_start(const SegPlanData& P, const SortLane& lane) {
+    return P.ownMulti ? P.ownMulti + P.wide.size() * MGPU_MAX_PASSES * MGPU_RADIX
+                      : lane.multi + (size_t)lane.multiArrays * MGPU_MAX_PASSES * MGPU_RADIX;
+}
 
 // The device-wide passes over every large segment of the plan at once:
 // digit_count over their chunks, digit_scan per segment, then one
@@ -693,9 +762,7 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
     const uint32_t numWide = (uint32_t)P.wide.size();
     uint32_t* const lookback = P.ownLookback ? P.ownLookback : lane.lookback;
     uint32_t* const hist = P.ownMulti ? P.ownMulti : lane.multi;
-    uint32_t* const digitStart =
-        P.ownMulti ? P.ownMulti + (size_t)numWide * MGPU_MAX_PASSES * MGPU_RADIX
-                   : lane.multi + (size_t)lane.multiArrays * MGPU_MAX_PASSES * MGPU_RADIX;
+    uint32_t* const digitStart = wide_digit_start(P, lane);
 
     mgpuMultiCountArgs ca;
     std::memset(&ca, 0, sizeof(ca));
@@ -725,6 +792,7 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
     ca.digit_start = digitStart;
     ca.tile_counters = lane.tileCounters;
     ca.direct = P.wideDirectCount ? 1u : 0u;
+    ca.lsd_segments = lane.tileCounters + MGPU_LSD_SLOT;
     sortStatus_t st = mgpu_launch(e, lane.stream, cols ? e->fnMultiCountCols : e->fnMultiCount,
                                   grid, threads, &ca);
     if (st) return st;
@@ -760,6 +828,7 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
         pa.shift = ca.shift[p];
         pa.mask = ca.mask[p];
         pa.num_values = (uint32_t)carried;
+        if (P.wideBuckets && p > 0) pa.lsd_segments = lane.tileCounters + MGPU_LSD_SLOT;
         int mode;
         if (P.valueCount == 0) mode = MGPU_VALUES_NONE;
         else if (P.valueCount == -1) mode = p == 0 ? MGPU_VALUES_INDEX : MGPU_VALUES_SINGLE;
@@ -798,6 +867,30 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
 
 }  // namespace
 
+namespace {
+
+// The workgroups' sorts of whole segments with 1024 threads, or the others.
+sortStatus_t mgpu_enqueue_slots(SegPlanData& P, SortLane& lane, hipStream_t s, bool large) {
+    mgpuSegSlotArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.segs = P.devSegs;
+    a.wide = P.devWide;
+    a.slots = P.devSlots + (large ? 2 * P.slots1024 : 0);
+    a.digit_start = wide_digit_start(P, lane);
+    a.lsd_segments = P.wideBuckets && !large ? lane.tileCounters + MGPU_LSD_SLOT : nullptr;
+    a.num_values = P.valueCount == -1 ? 1u : (uint32_t)P.valueCount;
+    a.index_mode = P.valueCount == -1;
+    a.result_side = (uint32_t)P.resultSide;
+    a.first_bit = (uint32_t)P.firstBit;
+    a.num_bits = (uint32_t)P.numBits;
+    const uint32_t count = (uint32_t)(P.slots.size() / 2);
+    return mgpu_launch(P.engine, s, P.engine->fnSegSlots[large][P.valueCount != 0],
+                       large ? count - P.slots1024 : P.slots1024,
+                       large ? MGPU_LOCAL_THREADS : MGPU_BUCKET_THREADS, &a);
+}
+
+}  // namespace
+
 // Queues the launches of a built plan on the lane's stream.
 sortStatus_t mgpu_seg_enqueue(SegPlanData& P, SortLane& lane) {
     sortEngine_d* e = P.engine;
@@ -809,7 +902,7 @@ sortStatus_t mgpu_seg_enqueue(SegPlanData& P, SortLane& lane) {
     // each other, measured no faster: 4096 segments 0.614, 0.613, 0.619 ms
     // with one, two and three.  Forking after the device-wide count, so that
     // the count runs alone, was slower: 0.600 -> 0.639 ms.)
-    const bool fork = !P.launches.empty() && !P.wide.empty() && lane.side;
+    const bool fork = !P.launches.empty() && (!P.wide.empty() || !P.slots.empty()) && lane.side;
     hipStream_t ls = lane.stream;
     if (fork) {
         if (hipEventRecord(lane.fork, lane.stream) != hipSuccess ||
@@ -838,8 +931,16 @@ sortStatus_t mgpu_seg_enqueue(SegPlanData& P, SortLane& lane) {
         sortStatus_t st = mgpu_launch(e, ls, L.fn, L.grid, L.block, &a);
         if (st) return st;
     }
+    if (P.slots.size() / 2 > P.slots1024) {
+        sortStatus_t st = mgpu_enqueue_slots(P, lane, ls, true);
+        if (st) return st;
+    }
     if (!P.wide.empty()) {
         sortStatus_t st = mgpu_enqueue_wide(P, lane);
+        if (st) return st;
+    }
+    if (P.slots1024 != 0) {
+        sortStatus_t st = mgpu_enqueue_slots(P, lane, lane.stream, false);
         if (st) return st;
     }
     if (fork && (hipEventRecord(lane.join, lane.side) != hipSuccess ||

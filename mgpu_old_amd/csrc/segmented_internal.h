@@ -51,8 +51,8 @@ struct SegWideTune {
     uint32_t chunk = 1u << 14;
     int tile = 0;
     int pack = -1;
-    uint32_t keepKeys = 0;  // up to here one workgroup sorts a segment that fits its tile, while
-                            // few keys are in longer ones (0: no segment of minKeys or more)
+    uint32_t keepKeys = 0;  // up to here, and up to MGPU_LOCAL_MAX_KEYS, one workgroup sorts a
+                            // segment (0: none of minKeys or more)
 };
 
 // One persistent launch of one kernel variant.
@@ -101,6 +101,14 @@ struct SegPlanData {
     // The count kernel reads every device-wide segment as one piece and
     // writes its digit starts (no global histogram, no scan launch).
     bool wideDirectCount = false;
+    // A workgroup's sorts of the last launch: (segment, MGPU_SLOT_WHOLE) and,
+    // when the device-wide segments go through one scatter into buckets,
+    // (index in wide, bucket).
+    // (512 threads a workgroup, then from slots1024 on 1024.)
+    std::vector<uint32_t> slots;
+    uint32_t slots1024 = 0;
+    bool wideBuckets = false;
+    uint32_t* devSlots = nullptr;
     mgpuSegDesc* devWide = nullptr;
     uint32_t* devTileBegin = nullptr;  // [segments + 1]: first tile of each (packed: first chunk)
     uint32_t* devTileSeg = nullptr;    // [wideTiles]: the segment of each tile (packed: tile words)

@@ -161,7 +161,7 @@ def main():
             for c in WIDE_CHUNK:
                 for t in WIDE_TILE:
                     for pk in WIDE_PACK:
-                        line = f"wide {m} {c} {t} {pk} 8192"
+                        line = f"wide {m} {c} {t} {pk} 16384"
                         eng = engine_on(torch, tmp, bucket_text + line + "\n")
                         wide[line] = time_plan(torch, eng, keys, vals, starts, args.reps)
                         eng.close()
@@ -201,7 +201,7 @@ def main():
         f.write("# segmented-sort tuning table, written by mgpu_old_amd/tune_segsort.py (key + 1 value,\n"
                 "# bits [0,32)): <max ceil(log2 n)> <radix bits> <keys per thread> <threads> per\n"
                 "# size bucket of the persistent kernel; wide <min keys> <count piece> <tile>\n"
-                "# <packed|unpacked> <keys up to which one workgroup may keep a segment>\n")
+                "# <packed|unpacked> <keys up to which a workgroup sorts a segment whole>\n")
         f.write(bucket_text)
         f.write(best_wide + "\n")
     print(json.dumps({"table": rows, "wide": best_wide, "report": report}), flush=True)

@@ -1,13 +1,13 @@
 """Persistent segmented kernels with 8-bit digits: bit-exact against the oracle
 at the edges of their size classes (one lane per key, one wave with 2, 4, 8
 keys per lane, one workgroup with 2, 4, 6, 8, 12, 16 per thread), for each
-value class, and which kernels take segments between 4097 keys and a
-workgroup's tile."""
+value class; which kernels take segments above 4096 keys; and device-wide
+segments that one scatter sends to buckets."""
 import numpy as np
 import pytest
 
 from mgpu_old_amd import workloads
-from gpu_helpers import GpuSort, make_engine
+from gpu_helpers import GpuSort, make_engine, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -40,6 +40,17 @@ def _keys(starts, seed):
     return keys
 
 
+def _check(oracle, keys, vals, vc, starts, g, fb, eb):
+    out_k, out_v = g.keys(), g.values()
+    for i in range(len(starts) - 1):
+        a, b = int(starts[i]), int(starts[i + 1])
+        rk, rv = oracle.stable_sort(keys[a:b], [v[a:b] for v in vals], value_count=vc,
+                                    first_bit=fb, end_bit=eb)
+        assert np.array_equal(out_k[a:b], rk), f"segment {i} (n={b - a}) keys differ"
+        for j, (o, r) in enumerate(zip(out_v, rv)):
+            assert np.array_equal(o[a:b], r), f"segment {i} (n={b - a}) values[{j}] differ"
+
+
 def _run(engine, oracle, sizes, vc, fb, eb, seed):
     starts = _starts(sizes)
     keys = _keys(starts, seed)
@@ -54,14 +65,7 @@ def _run(engine, oracle, sizes, vc, fb, eb, seed):
     names = set(engine.read_timing())
     engine.enable_timing(False)
     engine.check_device()
-    out_k, out_v = g.keys(), g.values()
-    for i in range(len(sizes)):
-        a, b = int(starts[i]), int(starts[i + 1])
-        rk, rv = oracle.stable_sort(keys[a:b], [v[a:b] for v in vals], value_count=vc,
-                                    first_bit=fb, end_bit=eb)
-        assert np.array_equal(out_k[a:b], rk), f"segment {i} (n={b - a}) keys differ"
-        for j, (o, r) in enumerate(zip(out_v, rv)):
-            assert np.array_equal(o[a:b], r), f"segment {i} (n={b - a}) values[{j}] differ"
+    _check(oracle, keys, vals, vc, starts, g, fb, eb)
     return names
 
 
@@ -91,16 +95,79 @@ def test_many_workgroup_segments(engine, oracle, variant, monkeypatch):
         _run(engine, oracle, list(rng.integers(1025, 1200, 2101)), 1, 0, 32, seed=seed)
 
 
-@pytest.mark.parametrize("sizes,device_wide", [
-    ([8192, 4097, 100], False),
-    ([8192, 8193, 100], True),          # longer segments hold more keys
-    ([8192, 4097, 8193, 100], False),   # and here fewer
-    ([4096, 9000], True),
+@pytest.mark.parametrize("sizes,slots,device_wide", [
+    ([8192, 4097, 100], False, False),  # none above the kernels' tile
+    ([8193, 8192, 4097, 4096], True, False),
+    ([16384, 16385, 4096], True, True),
 ])
-def test_route_above_4096(engine, oracle, sizes, device_wide):
+def test_route_above_4096(engine, oracle, sizes, slots, device_wide):
     names = _run(engine, oracle, sizes, 1, 0, 32, seed=79)
-    wide = 8193 in sizes or 9000 in sizes
-    assert any("mgpu_multi" in k for k in names) == wide, names
-    # 8192 and 4097 keys: a workgroup each (16 keys per thread), or with the rest.
-    in_tile = any("_r8_i16_" in k for k in names)
-    assert in_tile == (not device_wide), names
+    assert any("_slots_" in k for k in names) == slots, names
+    assert any("mgpu_multi" in k for k in names) == device_wide, names
+    assert any("_r8_i16_" in k for k in names) == (not slots), names
+
+
+def _spread(kind, n, seed):
+    u = workloads.uniform_keys(n, seed=seed)
+    if kind == "narrow":  # top digits constant: buckets of a lower digit
+        return u >> np.uint32(11)
+    if kind == "few":  # 16 values, each in more bins than fit a bucket
+        return (u & np.uint32(15)) * np.uint32(0x01010101)
+    if kind == "heavy":  # two thirds in one bin: every pass
+        return np.where(u % np.uint32(3) == 0, u, u & np.uint32(0xFFFFFF))
+    if kind == "equal":
+        return np.full(n, 0xFFFFFFFF, dtype=np.uint32)
+    return u
+
+
+KINDS = ["uniform", "narrow", "few", "heavy", "equal"]
+
+
+@pytest.mark.parametrize("vc", [-1, 0, 1, 2, 6])
+@pytest.mark.parametrize("fb,eb", [(0, 32), (5, 26), (0, 16)])  # 4, 3 and (no buckets) 2 passes
+def test_buckets(engine, oracle, vc, fb, eb):
+    """Device-wide segments of a batch large enough for buckets, each kind of
+    keys in segments of each size: 16385 keys, sizes that divide into buckets
+    evenly and not, and the longest that the count takes whole."""
+    sizes = [16385, 16896, 40000, 65536, 100, 9000] * len(KINDS) + [1 << 18]
+    starts = _starts(sizes)
+    keys = np.concatenate([_spread(KINDS[(i // 6 + i) % len(KINDS)], m, 90 + i)
+                           for i, m in enumerate(sizes)])
+    vals = [workloads.uniform_keys(len(keys), seed=81 + j) for j in range(max(vc, 0))]
+    g = GpuSort(keys, vals, value_count=vc, first_bit=fb, end_bit=eb)
+    import torch
+    torch.cuda.synchronize()
+    engine.enable_timing(True)
+    engine.read_timing()
+    engine.sort_segmented(g.data, starts)
+    torch.cuda.synchronize()
+    names = set(engine.read_timing())
+    engine.enable_timing(False)
+    engine.check_device()
+    _check(oracle, keys, vals, vc, starts, g, fb, eb)
+    assert any("_slots_b512_" in k for k in names) == (eb - fb > 16), names
+
+
+def test_buckets_replayed(engine, oracle):
+    """A captured plan over keys that go through buckets, then keys that take
+    every pass, then both kinds, then buckets again."""
+    import torch
+    sizes = [20000, 30000, 50000, 65536, 100000, 17000]
+    starts = _starts(sizes)
+    n = int(starts[-1])
+    vals = [np.arange(n, dtype=np.uint32)]
+    g = GpuSort(np.zeros(n, dtype=np.uint32), vals, value_count=1)
+    torch.cuda.synchronize()
+    plan = engine.segmented_plan(g.data, starts)
+    for r, kinds in enumerate([["uniform"], ["heavy"], ["uniform", "heavy"], ["narrow"],
+                               ["uniform"]]):
+        keys = np.concatenate([_spread(kinds[i % len(kinds)], m, 200 + 10 * r + i)
+                               for i, m in enumerate(sizes)])
+        g.by_ptr[g.data.keys[0]][:n].copy_(to_dev(keys, n))
+        g.by_ptr[g.data.values[0][0]][:n].copy_(to_dev(vals[0], n))
+        torch.cuda.synchronize()
+        plan.execute(g.data)
+        torch.cuda.synchronize()
+        engine.check_device()
+        _check(oracle, keys, vals, 1, starts, g, 0, 32)
+    plan.close()
