@@ -424,7 +424,10 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
         ma.clear = L.lookback;
         ma.clear_words = (lbWords + 3) & ~uint64_t(3);
         ma.n = n;
-        ma.chunk = std::min(16384u, std::max(4096u, ((n + 63) / 64 + 1023) & ~1023u));
+        // (Smaller pieces pay for more adds to the same words: 1391168 pairs
+        // 49.6 us with up to 12288 keys, 50.1 with 8192, 54.8 with 4096, 50.2
+        // with 16384.)
+        ma.chunk = std::min(12288u, std::max(4096u, ((n + 63) / 64 + 1023) & ~1023u));
         ma.vec_ok = (reinterpret_cast<uintptr_t>(keyBuf[0]) & 15) == 0;
         ma.num_passes = (uint32_t)numPasses;
         ma.bin_shift = (uint32_t)(firstBit + fieldBits - MGPU_MID_BITS);

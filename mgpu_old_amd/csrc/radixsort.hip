@@ -1058,7 +1058,8 @@ __device__ __forceinline__ void load_striped(const uint32_t* src, uint32_t n, ui
 // its input: 20001 pairs 47.4 -> 26.4 us, 150000 51.1 -> 27.7, 2^19 61.0 ->
 // 35.0, 1000003 74.4 -> 46.7, 3000001 96.2 -> 66.8; normal floats 150000
 // 53.3 -> 42.5.  Keys that no grouping spreads: 1.0-1.08x up to 2^20 keys, at
-// 3000001 112 against 108 us (the counts and the empty bucket launch).
+// 1391168 92.4 -> 93.4 us and at 2500001 98.7 -> 100.7 (the counts and the
+// check ahead of each later pass).
 //
 // The digits of a bucketed sort's first scatter, worked out by every workgroup
 // from the counts while its keys load (1024 bins: a few KB from the L2 and a
@@ -1074,7 +1075,7 @@ __device__ __forceinline__ void load_striped(const uint32_t* src, uint32_t n, ui
 // s_start: each digit's first output position; shift, width: the field that is
 // the digit or, when the result is true, the bin whose digit s_map holds; mask:
 // the digit of the padding keys (all ones) of the last tile.  s_work: at least
-// 3 * RADIX words.  c: this thread's bins, digit0: its first-pass digit's count (both read by the
+// 3 * RADIX + 32 words.  c: this thread's bins, digit0: its first-pass digit's count (both read by the
 // caller ahead of the tile's loads, whose return they would otherwise wait
 // for).
 template <int BLOCK>
@@ -1103,9 +1104,34 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
     uint32_t group = sum;
 #pragma unroll
     for (uint32_t off = 1; off < LANES; off <<= 1) group += quad_xor(group, off);
-    uint32_t before = mgpu::block_exclusive_scan_dpp<BLOCK>(sum, s_tmp, lane, wave);
+    // The starts of the bins and of the first pass's digits, and what the
+    // counts allow, behind one barrier: keys that no grouping spreads take no
+    // other here (3 us of the tile's 21 at 1391168 pairs with one for each).
+    constexpr uint32_t W = BLOCK / 64;
+    uint32_t* const s_more = s_work + 3 * RADIX;  // [2][16]
+    const uint32_t inc = mgpu::wave_inclusive_scan_dpp(sum);
+    const uint32_t inc0 = mgpu::wave_inclusive_scan_dpp(digit0);
+    const uint32_t found =
+        (__builtin_amdgcn_ballot_w64(group > MGPU_LOCAL_MAX_KEYS) ? 1u : 0u) |
+        (__builtin_amdgcn_ballot_w64(most > MGPU_LOCAL_MAX_KEYS) ? 2u : 0u) |
+        (__builtin_amdgcn_ballot_w64(group == a.n) ? 4u : 0u);
+    if (lane == 63) {
+        s_tmp[wave] = inc;
+        s_more[wave] = inc0;
+        s_more[16 + wave] = found;
+    }
+    __syncthreads();
+    const bool wave_lane = (lane & 15u) < W;
+    const uint32_t waves = mgpu::row_inclusive_scan_dpp(wave_lane ? s_tmp[lane & 15u] : 0u);
+    const uint32_t waves0 = mgpu::row_inclusive_scan_dpp(wave_lane ? s_more[lane & 15u] : 0u);
+    const uint32_t any = wave_lane ? s_more[16 + (lane & 15u)] : 0u;
+    uint32_t before = inc - sum, start0 = inc0 - digit0;
+    if (wave > 0) {
+        before += (uint32_t)__builtin_amdgcn_readlane((int)waves, (int)(wave - 1));
+        start0 += (uint32_t)__builtin_amdgcn_readlane((int)waves0, (int)(wave - 1));
+    }
     if (last_group && tid == 0) a.mid_plan->start[RADIX] = a.n;
-    if (__syncthreads_and(group <= MGPU_LOCAL_MAX_KEYS)) {
+    if (__builtin_amdgcn_ballot_w64(any & 1u) == 0) {
         const uint32_t g = tid / LANES;
         if (tid % LANES == 0) {
             s_start[g] = before;
@@ -1122,8 +1148,14 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
     uint32_t* const s_keys = s_work;              // keys of each bucket
     uint32_t* const s_first = s_work + RADIX;     // its first bin
     uint32_t* const s_bins = s_work + 2 * RADIX;  // the bin after its last
-    bool fits = __syncthreads_and(most <= MGPU_LOCAL_MAX_KEYS) != 0;
-    bool one = __syncthreads_or(group == a.n) != 0;
+    bool fits = __builtin_amdgcn_ballot_w64(any & 2u) == 0;
+    bool one = __builtin_amdgcn_ballot_w64(any & 4u) != 0;
+    if (!fits && !one) {
+        if (last_group && tid == 0) a.mid_plan->buckets = 0;
+        if (tid < RADIX) s_start[tid] = start0;
+        __syncthreads();
+        return false;
+    }
     int digit = -1;  // the digit whose values are the buckets; -1: bins
     uint32_t digit_shift = a.mid_shift, keys = 0;
     if (fits) {
@@ -1164,8 +1196,9 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
         }
     }
     if (last_group && tid == 0) a.mid_plan->buckets = fits ? 1u : 0u;
-    const uint32_t start =
-        mgpu::block_exclusive_scan_dpp<BLOCK>(fits ? keys : digit0, s_tmp, lane, wave);
+    __syncthreads();  // (every wave has read s_tmp)
+    uint32_t start = mgpu::block_exclusive_scan_dpp<BLOCK>(fits ? keys : 0u, s_tmp, lane, wave);
+    if (!fits) start = start0;
     if (tid < RADIX) {
         s_start[tid] = start;
         if (last_group && fits) {
