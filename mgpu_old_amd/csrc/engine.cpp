@@ -152,8 +152,8 @@ sortStatus_t mgpu_ensure_multi(SortLane& L, uint32_t arrays) {
         L.multi = nullptr;
         L.multiArrays = 0;
         const uint32_t cap = arrays + arrays / 2 + 16;
-        if (hipMalloc(&L.multi, (size_t)cap * 2 * MGPU_MAX_PASSES * MGPU_RADIX * sizeof(uint32_t)) !=
-            hipSuccess) {
+        if (hipMalloc(&L.multi, ((size_t)cap * 2 * MGPU_MAX_PASSES * MGPU_RADIX +
+                                 MGPU_MULTI_DONE_WORDS(cap)) * sizeof(uint32_t)) != hipSuccess) {
             L.multi = nullptr;
             return SORT_STATUS_DEVICE_ALLOC_FAILED;
         }
@@ -162,7 +162,8 @@ sortStatus_t mgpu_ensure_multi(SortLane& L, uint32_t arrays) {
     // Stream-ordered: a plain hipMemset runs on the null stream, which a
     // non-blocking lane stream does not wait for.
     if (hipMemsetAsync(L.multi, 0,
-                       (size_t)L.multiArrays * MGPU_MAX_PASSES * MGPU_RADIX * sizeof(uint32_t),
+                       ((size_t)L.multiArrays * MGPU_MAX_PASSES * MGPU_RADIX +
+                        MGPU_MULTI_DONE_WORDS(L.multiArrays)) * sizeof(uint32_t),
                        L.stream) != hipSuccess)
         return SORT_STATUS_DEVICE_ERROR;
     L.multiDirty = false;

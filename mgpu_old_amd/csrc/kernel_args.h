@@ -226,7 +226,8 @@ struct mgpuSegArgs {
 // array `seg`, read from side 0.
 struct mgpuMultiCountArgs {
     const mgpuSegDesc* segs;
-    const uint32_t* chunks;  // [num_chunks][4]: seg, begin, end, bucket size (direct; 0: none)
+    const uint32_t* chunks;  // [num_chunks][4]: seg, begin, end, (direct) bucket size, 0: none,
+                             // | pieces of the array << 16
     uint32_t* hist;          // [num_segs][MGPU_MAX_PASSES][MGPU_RADIX], zero on entry
     uint32_t* clear;         // lookback words to zero
     uint64_t clear_words;    // multiple of 4
@@ -234,13 +235,14 @@ struct mgpuMultiCountArgs {
     uint32_t num_passes;
     uint32_t shift[MGPU_MAX_PASSES];
     uint32_t mask[MGPU_MAX_PASSES];
-    // Lane-column kernel only: every chunk is a whole array (direct != 0),
-    // so the kernel writes the digit starts and zeroes the tile counters
-    // itself, in place of multi_scan; hist is not used.
+    // Lane-column kernel only (direct != 0): the last of an array's workgroups
+    // writes its digit starts in place of multi_scan, which leaves hist and done as they
+    // were; the tile counters are zeroed too.
     uint32_t* digit_start;    // [num_segs][MGPU_MAX_PASSES][MGPU_RADIX]
     uint32_t* tile_counters;  // [MGPU_LANE_COUNTERS]
     uint32_t direct;
     uint32_t pad_;
+    uint32_t* done;  // [num_segs]: pieces counted, zero on entry
     // Direct counts with a bucket size T: an array whose keys the highest
     // digit that is not constant spreads into bins small enough gets its route
     // (mgpuSegDesc), that digit's starts in the first row of its digit_start
@@ -267,6 +269,9 @@ struct mgpuSegSlotArgs {
     uint32_t num_bits;
     uint32_t pad_;
 };
+
+// Words of `done` counters for so many arrays, between hist and digit_start.
+#define MGPU_MULTI_DONE_WORDS(arrays) (((size_t)(arrays) + 63) & ~(size_t)63)
 
 // digit_scan, one workgroup per array; zeroes hist and the tile counters.
 struct mgpuMultiScanArgs {

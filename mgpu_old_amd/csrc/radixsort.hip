@@ -718,7 +718,9 @@ __device__ void multi_count_cols_body(const mgpuMultiCountArgs& a) {
     __syncthreads();
     const uint32_t* ch = a.chunks + 4 * blockIdx.x;
     const uint32_t sg = ch[0], begin = ch[1], end = ch[2];
+    const uint32_t T = ch[3] & 0xFFFFu, pieces = ch[3] >> 16;
     const uint32_t* kp = a.segs[sg].keys[0];
+    const uint32_t n = a.segs[sg].n;
     const auto keys = mgpu::to_global(kp);
     const uint32_t np = a.num_passes;
     // Pass p's word for key k: row d / 2 of the pass's RADIX / 2 (digit d =
@@ -788,18 +790,38 @@ __device__ void multi_count_cols_body(const mgpuMultiCountArgs& a) {
             hi += w >> 16;
         }
     }
-    const uint32_t sum = (h ? hi : lo) + (uint32_t)__shfl_xor((int)(h ? lo : hi), 1, 64);
+    uint32_t sum = (h ? hi : lo) + (uint32_t)__shfl_xor((int)(h ? lo : hi), 1, 64);
     if (a.direct) {
-        // The piece is the whole array: its digit starts, pass by pass (a
-        // scan per group of 256 threads), with no global histogram and no
-        // separate scan launch.  Workgroup 0 zeroes the passes' tile
-        // counters, as that launch would.
-        __shared__ uint32_t s_tmp[BLOCK / 64];
+        // The array's digit starts, pass by pass (a scan per group of 256
+        // threads), by the workgroup whose piece is the last to be counted:
+        // no separate scan launch, and none waits for another.  An array of
+        // one piece needs no global histogram.  Workgroup 0 zeroes the
+        // passes' tile counters, as that launch would.
+        // (With every array one piece, the longest set the time of a small
+        // batch: 4 of 200000 keys, key + value, 80 -> 54 us.)
+        __shared__ uint32_t s_tmp[BLOCK / 64], s_last;
+        if (blockIdx.x == 0 && tid < MGPU_LSD_SLOT) a.tile_counters[tid] = 0;
+        if (pieces > 1) {
+            uint32_t* const word = &a.hist[((size_t)sg * MGPU_MAX_PASSES + p) * RADIX + d];
+            if (sum)
+                __hip_atomic_fetch_add(word, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // The adds of every thread are in before the piece counts as done.
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (tid == 0)
+                s_last = __hip_atomic_fetch_add(&a.done[sg], 1u, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            if (s_last != pieces - 1) return;
+            if (p < np) {
+                sum = ld_agent(word);
+                st_agent(word, 0u);
+            }
+            if (tid == 0) st_agent(&a.done[sg], 0u);
+        }
         const uint32_t ex = group_exclusive_scan<BLOCK>(sum, s_tmp, tid & 63, tid >> 6);
         uint32_t* const starts = a.digit_start + (size_t)sg * MGPU_MAX_PASSES * RADIX;
-        if (blockIdx.x == 0 && tid < MGPU_LSD_SLOT) a.tile_counters[tid] = 0;
-        const uint32_t T = ch[3];
-        if (T == 0 || !plan_buckets(a, sg, end, T, p, d, sum, ex, starts)) {
+        if (T == 0 || !plan_buckets(a, sg, n, T, p, d, sum, ex, starts)) {
             if (p < np) starts[p * RADIX + d] = ex;
         }
     } else if (sum) {

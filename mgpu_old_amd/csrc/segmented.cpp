@@ -29,9 +29,14 @@ constexpr uint64_t kXcdMinTiles = 4;
 // Tile counters of a one-chain-per-segment launch (groups of segments).
 constexpr long kTileCounterGroups = 8;
 
-// Longest segment the device-wide count reads with one workgroup, writing
-// its digit starts directly (a 2^18-key segment: 1 MB, a few microseconds).
+// Longest segment whose digit starts the device-wide count writes itself.
 constexpr uint32_t kDirectCountMax = 1u << 18;
+
+// Keys of a piece of that count: a workgroup per CU, where that leaves pieces
+// worth their 1024 adds to the segment's histogram.  100 segments of 20000
+// keys 62 us in pieces of 8192, 58 whole; 4 of 200000 47 in pieces of up to
+// 32768, 73 whole (keys only; one workgroup counts 200000 keys in 43 us).
+constexpr uint32_t kCountPieceMin = 32768, kCountPieceMax = 1u << 18;
 
 // Keys of a bucket of a device-wide segment, about (its last bin can make it
 // longer: see plan_buckets), where the batch is large and small, and keys of a
@@ -458,11 +463,9 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         // barrier per tile), and when no segment outweighs a quarter of an
         // XCD's share (else one XCD would do most of the work).
         // MGPUSORT_SEG_XCD=0|1 forces the choice.
-        // The count reads each segment as one piece and writes its digit
-        // starts itself when no segment is longer than kDirectCountMax keys
-        // (one workgroup per segment stays short) and no piece size was
-        // asked for; else pieces of chunkKeys with a histogram in global
-        // memory and a scan launch after them.
+        // The count writes the digit starts itself when no segment is longer
+        // than kDirectCountMax keys and no piece size was asked for; else
+        // pieces of chunkKeys and a scan launch after them.
         P.wideDirectCount = count_cols() && longestSeg <= kDirectCountMax &&
                             std::getenv("MGPUSORT_SEG_WIDE_CHUNK") == nullptr;
         P.wideBuckets = P.wideDirectCount && use_buckets(e, P, packMode, wideKeys);
@@ -530,7 +533,11 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         P.widePacked = P.wideVariant->packed[MGPU_VALUES_NONE] != nullptr &&
                        (packMode == 1 ||
                         (packMode == -1 && P.wideXcds == 1 && !P.wideBuckets));
-        const uint32_t pieceKeys = P.wideDirectCount ? longestSeg : chunkKeys;
+        const uint32_t pieceKeys =
+            P.wideDirectCount
+                ? (uint32_t)std::min<uint64_t>(
+                      kCountPieceMax, std::max<uint64_t>(kCountPieceMin, wideKeys / e->numCUs))
+                : chunkKeys;
         const uint32_t bucketCap = (uint32_t)std::min<uint64_t>(
             kBucketMaxKeys,
             std::max<uint64_t>(kBucketMinKeys, wideKeys / (2 * (uint64_t)e->numCUs)));
@@ -565,7 +572,8 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
             chunks.push_back(c.seg);
             chunks.push_back(c.begin);
             chunks.push_back(c.end);
-            chunks.push_back(c.bucket);
+            const uint32_t n = segs[P.wide[c.seg]].n;
+            chunks.push_back(P.wideDirectCount ? c.bucket | (n + pieceKeys - 1) / pieceKeys << 16 : 0u);
         }
         if (P.widePacked) {
             // Wave chunks back to back, `waves` to a tile.  A segment that
@@ -722,12 +730,13 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         if (ownScratch) {
             // Histograms must start at zero (the scan leaves them zero after
             // every run); lookback words are zeroed by the count kernel.
-            const size_t multiWords = (size_t)2 * P.wide.size() * MGPU_MAX_PASSES * MGPU_RADIX;
+            const size_t histWords = P.wide.size() * MGPU_MAX_PASSES * MGPU_RADIX;
+            const size_t zeroWords = histWords + MGPU_MULTI_DONE_WORDS(P.wide.size());
             if (hipMalloc(&P.ownLookback, ((lbWords + 3) & ~uint64_t(3)) * sizeof(uint32_t)) !=
                     hipSuccess ||
-                hipMalloc(&P.ownMulti, multiWords * sizeof(uint32_t)) != hipSuccess)
+                hipMalloc(&P.ownMulti, (zeroWords + histWords) * sizeof(uint32_t)) != hipSuccess)
                 return SORT_STATUS_DEVICE_ALLOC_FAILED;
-            if (hipMemsetAsync(P.ownMulti, 0, multiWords * sizeof(uint32_t) / 2, lane.stream) !=
+            if (hipMemsetAsync(P.ownMulti, 0, zeroWords * sizeof(uint32_t), lane.stream) !=
                     hipSuccess ||
                 hipStreamSynchronize(lane.stream) != hipSuccess)
                 return SORT_STATUS_DEVICE_ERROR;
@@ -747,9 +756,14 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
 
 namespace {
 
-uint32_t* wide_digit_start(const SegPlanData& P, const SortLane& lane) {
+// The per-array scratch of the device-wide passes: hist, done, digit starts.
+uint32_t* wide_done(const SegPlanData& P, const SortLane& lane) {
     return P.ownMulti ? P.ownMulti + P.wide.size() * MGPU_MAX_PASSES * MGPU_RADIX
                       : lane.multi + (size_t)lane.multiArrays * MGPU_MAX_PASSES * MGPU_RADIX;
+}
+uint32_t* wide_digit_start(const SegPlanData& P, const SortLane& lane) {
+    return wide_done(P, lane) +
+           MGPU_MULTI_DONE_WORDS(P.ownMulti ? P.wide.size() : (size_t)lane.multiArrays);
 }
 
 // The device-wide passes over every large segment of the plan at once:
@@ -792,6 +806,7 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
     ca.digit_start = digitStart;
     ca.tile_counters = lane.tileCounters;
     ca.direct = P.wideDirectCount ? 1u : 0u;
+    ca.done = wide_done(P, lane);
     ca.lsd_segments = lane.tileCounters + MGPU_LSD_SLOT;
     sortStatus_t st = mgpu_launch(e, lane.stream, cols ? e->fnMultiCountCols : e->fnMultiCount,
                                   grid, threads, &ca);

@@ -98,8 +98,8 @@ struct SegPlanData {
     // devTileSeg two words per tile (its first segment; part starts, chunks
     // holding keys and whether it continues a segment).
     bool widePacked = false;
-    // The count kernel reads every device-wide segment as one piece and
-    // writes its digit starts (no global histogram, no scan launch).
+    // The count kernel writes the digit starts of the device-wide segments
+    // (no scan launch).
     bool wideDirectCount = false;
     // A workgroup's sorts of the last launch: (segment, MGPU_SLOT_WHOLE) and,
     // when the device-wide segments go through one scatter into buckets,
