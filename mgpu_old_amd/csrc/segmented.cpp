@@ -361,9 +361,27 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
 
     // Group segments by kernel variant; very large ones go device-wide.
     const uint32_t wideMin = device_wide_min(e), chunkKeys = wide_chunk(e);
-    const uint32_t keep = keep_in_workgroup(e);
-    uint32_t longestSeg = 0;
-    for (int i = 0; i < numSegments; ++i) longestSeg = std::max(longestSeg, segs[i].n);
+    uint32_t keep = keep_in_workgroup(e), longestSeg = 0, numSmall = 0;
+    uint64_t longKeys = 0;  // in segments above a bucket's size
+    for (int i = 0; i < numSegments; ++i) {
+        longestSeg = std::max(longestSeg, segs[i].n);
+        if (segs[i].n < wideMin) ++numSmall;
+        if (segs[i].n > MGPU_BUCKET_KEYS) longKeys += segs[i].n;
+    }
+    const bool directCount = count_cols() && longestSeg <= kDirectCountMax &&
+                             std::getenv("MGPUSORT_SEG_WIDE_CHUNK") == nullptr;
+    // A batch on one stream (the server's) runs its launches one after
+    // another, and a dozen workgroups' launch costs what a full one does:
+    // where there are buckets, the segments between a bucket's size and 16384
+    // keys go through them as well, and few small ones join the whole
+    // segments of the last launch.  Batches of 27 requests log-uniform in
+    // [2^10, 2^18] ran 14 and 25 us longer with a launch for each of the two.
+    bool smallInSlots = false;
+    if (lane.noSide && keep > MGPU_BUCKET_KEYS && directCount &&
+        use_buckets(e, P, pack_mode(e), longKeys)) {
+        keep = MGPU_BUCKET_KEYS;
+        smallInSlots = numSmall <= (uint32_t)e->numCUs;
+    }
     const bool noneAboveTile = longestSeg <= keep && seg_fits_tile(e, longestSeg);
     struct Group {
         std::vector<uint32_t> big, small;
@@ -373,7 +391,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
     for (int i = 0; i < numSegments; ++i) {
         const uint32_t n = segs[i].n;
         if (n == 0 || P.numBits == 0) continue;
-        if (n >= wideMin && !noneAboveTile) {
+        if ((n >= wideMin && !noneAboveTile) || smallInSlots) {
             if (n <= keep) {
                 auto& list = n <= MGPU_BUCKET_KEYS ? P.slots : slots1024;
                 list.push_back((uint32_t)i);
@@ -466,8 +484,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         // The count writes the digit starts itself when no segment is longer
         // than kDirectCountMax keys and no piece size was asked for; else
         // pieces of chunkKeys and a scan launch after them.
-        P.wideDirectCount = count_cols() && longestSeg <= kDirectCountMax &&
-                            std::getenv("MGPUSORT_SEG_WIDE_CHUNK") == nullptr;
+        P.wideDirectCount = directCount;
         P.wideBuckets = P.wideDirectCount && use_buckets(e, P, packMode, wideKeys);
         P.wideXcds = 1;
         P.xcdTileBegin.clear();

@@ -171,3 +171,36 @@ def test_buckets_replayed(engine, oracle):
         engine.check_device()
         _check(oracle, keys, vals, 1, starts, g, 0, 32)
     plan.close()
+
+
+@pytest.mark.parametrize("vc,width", [(0, 32), (1, 32), (2, 24), (1, 16)])
+def test_served_batch(engine, oracle, vc, width):
+    """Requests of every class at once: on the server's one stream small ones
+    and those between 8193 and 16384 keys join the buckets' launches (not with
+    the two passes of 16 bits)."""
+    import torch
+    import mgpu_old_amd as mg
+    from gpu_helpers import to_host
+    sizes = [100, 1, 4096, 4097, 8192, 8193, 16384, 16385, 40000, 100000, 200000, 1 << 18]
+    reqs, host = [], []
+    for i, n in enumerate(sizes):
+        keys = _spread(KINDS[i % len(KINDS)], n, 300 + i)
+        vals = [workloads.uniform_keys(n, seed=400 + 10 * i + j) for j in range(vc)]
+        tk, tv = to_dev(keys), [to_dev(v) for v in vals]
+        r = mg.SortRequest()
+        r.keys = tk.data_ptr()
+        for j, t in enumerate(tv):
+            r.values[j] = t.data_ptr()
+        r.numElements, r.valueCount, r.firstBit, r.endBit = n, vc, 0, width
+        reqs.append(r)
+        host.append((keys, vals, tk, tv))
+    torch.cuda.synchronize()
+    with mg.Server(engine, 1 << 30, max_in_flight=2, max_elements=1 << 18) as srv:
+        comps = srv.replay(reqs, np.zeros(len(reqs)))
+    torch.cuda.synchronize()
+    for i, (c, (keys, vals, tk, tv)) in enumerate(zip(comps, host)):
+        assert c.status == 0, f"request {i} failed: {mg.status_string(c.status)}"
+        rk, rv = oracle.stable_sort(keys, vals, first_bit=0, end_bit=width)
+        assert np.array_equal(to_host(tk, keys.size), rk), f"request {i} keys differ"
+        for j, t in enumerate(tv):
+            assert np.array_equal(to_host(t, keys.size), rv[j]), f"request {i} values[{j}] differ"
