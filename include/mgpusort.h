@@ -324,13 +324,13 @@ sortStatus_t SORTAPI sortServerDestroy(sortServer_t server);
  * XCD) that no call has reported yet; SUCCESS otherwise. */
 sortStatus_t SORTAPI sortCheckDevice(sortEngine_t engine);
 
-/* What the engine chose at creation, and the last device inconsistency code
- * (0 none; 1 a lookback wait gave up; 2 a tile counter left dirty; 4 a
- * scatter offset out of range; 5 a segment with no workgroup on its XCD;
- * 6 a packed tile with more segments than it can hold; 7 a segment larger
- * than the tile of a kernel built without the global-memory routine: both
- * only from a broken plan) without clearing it.  No counterpart in the
- * reference. */
+/* What the engine chose at creation, and the first device inconsistency code
+ * that no call has reported yet (0 none; 1 a lookback wait gave up; 2 a tile
+ * counter left dirty; 4 a scatter offset out of range; 5 a segment with no
+ * workgroup on its XCD; 6 a packed tile with more segments than it can hold;
+ * 7 a segment larger than the tile of a kernel built without the global-memory
+ * routine: both only from a broken plan) without clearing it.  No counterpart
+ * in the reference. */
 typedef struct {
     int device;
     int numCUs;

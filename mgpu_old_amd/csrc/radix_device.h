@@ -35,9 +35,14 @@ __device__ __forceinline__ __attribute__((address_space(1))) T* to_global(T* p) 
 }
 
 // Records a failed self-check in the launch's error word, which lives in
-// host memory mapped into the device (system scope: the host reads it).
+// host memory mapped into the device (system scope: the host reads it).  The
+// first code stays: a pass after one that failed reads keys it left unwritten
+// and can find offsets out of range, which says nothing of the cause.  (A
+// plain read and write: the word has no atomics over the bus, and codes of
+// one pass have one cause.)
 __device__ __forceinline__ void set_error(uint32_t* flag, uint32_t code) {
-    __hip_atomic_store(flag, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0)
+        __hip_atomic_store(flag, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Inclusive scan over the 64 lanes of a wave.

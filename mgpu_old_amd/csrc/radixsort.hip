@@ -37,6 +37,8 @@ namespace {
 
 constexpr uint32_t RADIX = MGPU_RADIX;
 
+using mgpu::set_error;
+
 __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -48,12 +50,6 @@ __device__ __forceinline__ uint32_t ld_agent(const uint32_t* p) {
 
 __device__ __forceinline__ void st_agent(uint32_t* p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Records a failed self-check in the launch's error word, which lives in
-// host memory mapped into the device (system scope: the host reads it).
-__device__ __forceinline__ void set_error(uint32_t* flag, uint32_t code) {
-    __hip_atomic_store(flag, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Lane i gets v of lane i - 1, lane 0 gets lane0 (DPP wave_shr:1).
