@@ -74,7 +74,8 @@ typedef struct sortEngine_d* sortEngine_t;
  * kernelPath + "<name>.hsaco" (prefix concatenation, as the reference does
  * with cubins).  A NULL or empty kernelPath means the directory holding
  * libmgpusort.so; the environment variable MGPUSORT_KERNEL_PATH, when set,
- * overrides both. */
+ * overrides both.  Code objects built with other argument layouts than the
+ * library's are refused with SORT_STATUS_KERNEL_ERROR before any launch. */
 sortStatus_t SORTAPI sortCreateEngine(const char* kernelPath, sortEngine_t* engine);
 
 /* Replaces inc/mgpusort.h:54-55.  Validates the arguments as the reference

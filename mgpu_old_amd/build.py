@@ -7,6 +7,7 @@ Outputs go to mgpu_old_amd/lib/ (git-ignored, shipped with the tree):
 python -m mgpu_old_amd.build --ubsan DIR builds DIR/libmgpusort.so with the
 host code under UndefinedBehaviorSanitizer (load it with MGPUSORT_LIBRARY).
 """
+import hashlib
 import os
 import subprocess
 import sys
@@ -37,6 +38,21 @@ HOST_SOURCES = ["engine.cpp", "loader.cpp", "segmented.cpp", "server.cpp"]
 HIP_HOST_SOURCES = ["noalloc.hip"]
 
 
+def args_layout(text=None):
+    """Number of the argument layouts in kernel_args.h (`text`, or the file):
+    host library and code objects carry it, and an engine refuses code objects
+    of another number.  Any change of the file changes it, so that nothing has
+    to be raised by hand where sizes stay and meanings change."""
+    if text is None:
+        with open(os.path.join(CSRC, "kernel_args.h"), "rb") as f:
+            text = f.read()
+    return int.from_bytes(hashlib.sha256(text).digest()[:4], "little") | 1
+
+
+def layout_flag():
+    return [f"-DMGPU_ARGS_LAYOUT={args_layout():#x}u"]
+
+
 def _run(cmd):
     print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
@@ -47,14 +63,14 @@ def build(verbose=True):
     for obj, srcs in CODE_OBJECTS.items():
         # A plain gfx950 ELF code object (no offload bundle) for hipModuleLoad.
         _run([HIPCC, f"--offload-arch={ARCH}", "-O3", "-std=c++17", "--offload-device-only",
-              "--no-gpu-bundle-output", *DEVICE_FLAGS,
+              "--no-gpu-bundle-output", *DEVICE_FLAGS, *layout_flag(),
               "-I", CSRC, *[os.path.join(CSRC, s) for s in srcs],
               "-o", os.path.join(LIB, obj)])
     objects = []
     for src in HIP_HOST_SOURCES:
         obj = os.path.join(LIB, os.path.splitext(src)[0] + ".o")
         _run([HIPCC, f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-c",
-              "-fvisibility=hidden", *DEVICE_FLAGS,
+              "-fvisibility=hidden", *DEVICE_FLAGS, *layout_flag(),
               "-I", CSRC, "-I", INCLUDE, os.path.join(CSRC, src), "-o", obj])
         objects.append(obj)
     # Host code only: plain g++ against the HIP runtime, no device pass.
@@ -63,7 +79,7 @@ def build(verbose=True):
 
 def _link_host(out, objects, flags):
     _run([CXX, *flags, "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wextra",
-          "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+          "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", *layout_flag(),
           "-I", CSRC, "-I", INCLUDE, "-I", os.path.join(ROCM, "include"),
           *[os.path.join(CSRC, s) for s in HOST_SOURCES], *objects,
           "-o", out,

@@ -201,6 +201,9 @@ bool mgpu_noalloc_setup(int device);
 // Loads the code objects named from e->kernelPath and allocates the fixed
 // scratch.  On failure the engine is left for mgpu_engine_destroy.
 sortStatus_t mgpu_engine_load(sortEngine_d* e);
+// SORT_STATUS_KERNEL_ERROR unless the code object was built with this library's
+// argument layouts.
+sortStatus_t mgpu_check_layout(hipModule_t module, hipStream_t stream);
 void mgpu_engine_destroy(sortEngine_d* e);
 
 // Pass split of numBits into passes of at most maxWidth bits; returns the

@@ -5,6 +5,17 @@
 #pragma once
 #include <stdint.h>
 
+// Number of these layouts, made from this file by the build: each code object
+// exports it as mgpu_args_layout, and an engine compares it with its own
+// before any launch (kernels given another layout's arguments would follow
+// whatever pointers they found).
+#ifndef MGPU_ARGS_LAYOUT
+#define MGPU_ARGS_LAYOUT 0u
+#endif
+#define MGPU_ARGS_LAYOUT_NAME "mgpu_args_layout"
+#define MGPU_EXPORT_ARGS_LAYOUT \
+    extern "C" __device__ __attribute__((used)) uint32_t mgpu_args_layout = MGPU_ARGS_LAYOUT;
+
 #define MGPU_RADIX_BITS 8
 #define MGPU_RADIX 256
 #define MGPU_MAX_PASSES 4

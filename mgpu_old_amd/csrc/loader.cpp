@@ -219,13 +219,29 @@ bool lds_add_in_lane_order(sortEngine_d* e) {
 
 }  // namespace
 
+sortStatus_t mgpu_check_layout(hipModule_t module, hipStream_t stream) {
+    hipDeviceptr_t at = nullptr;
+    size_t bytes = 0;
+    uint32_t layout = 0;
+    if (hipModuleGetGlobal(&at, &bytes, module, MGPU_ARGS_LAYOUT_NAME) != hipSuccess ||
+        bytes != sizeof(layout)) {
+        (void)hipGetLastError();
+        return SORT_STATUS_KERNEL_ERROR;
+    }
+    if (hipMemcpyAsync(&layout, at, sizeof(layout), hipMemcpyDeviceToHost, stream) != hipSuccess ||
+        hipStreamSynchronize(stream) != hipSuccess)
+        return SORT_STATUS_DEVICE_ERROR;
+    return layout == MGPU_ARGS_LAYOUT ? SORT_STATUS_SUCCESS : SORT_STATUS_KERNEL_ERROR;
+}
+
 sortStatus_t mgpu_engine_load(sortEngine_d* e) {
     std::string path = e->kernelPath + kRadixObject;
     if (hipModuleLoad(&e->radixModule, path.c_str()) != hipSuccess) {
         e->radixModule = nullptr;
         return SORT_STATUS_KERNEL_NOT_FOUND;
     }
-    sortStatus_t st = get_fn(e, e->radixModule, "mgpu_digit_count", &e->fnCount);
+    sortStatus_t st = mgpu_check_layout(e->radixModule, e->lane.stream);
+    if (!st) st = get_fn(e, e->radixModule, "mgpu_digit_count", &e->fnCount);
     if (!st) st = get_fn(e, e->radixModule, "mgpu_digit_count_cols", &e->fnCountCols);
     // Counts of typed keys: without them (an older code object) typed sorts
     // map the keys in place around the sort.

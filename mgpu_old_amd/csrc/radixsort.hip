@@ -33,6 +33,8 @@
 #include "localsort.h"
 #include "radix_device.h"
 
+MGPU_EXPORT_ARGS_LAYOUT
+
 namespace {
 
 constexpr uint32_t RADIX = MGPU_RADIX;

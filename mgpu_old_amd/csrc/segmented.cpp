@@ -135,6 +135,7 @@ sortStatus_t mgpu_seg_load(sortEngine_d* e) {
         e->segModule = nullptr;
         return SORT_STATUS_KERNEL_NOT_FOUND;
     }
+    if (const sortStatus_t st = mgpu_check_layout(e->segModule, e->lane.stream)) return st;
     for (int v = 0; v < kSegVariants; ++v) {
         const int rb = seg_variant_bits(v), ipt = seg_variant_ipt(v), block = seg_variant_block(v);
         if (!seg_variant_valid(rb, ipt, block)) continue;

@@ -31,6 +31,8 @@
 #include "localsort.h"
 #include "radix_device.h"
 
+MGPU_EXPORT_ARGS_LAYOUT
+
 namespace {
 
 using mgpu::block_exclusive_scan;
