@@ -977,7 +977,8 @@ sortStatus_t SORTAPI sortArrayTyped(sortEngine_t engine, sortData_t data, int ke
 // the split, so as few passes as 8-bit digits need run instead where they end
 // on the same side (one more when the parities differ; 500000 pairs by 6-bit
 // digits 60.1 -> 31.7 us).  Early exit keeps the caller's passes: which of
-// them are skipped shows in the parity.
+// them are skipped shows in the parity.  What the caller's passes need is asked
+// for also where fewer run: the index output's other side for a second pass.
 sortStatus_t SORTAPI sortArrayEx(sortEngine_t engine, sortData_t data, int numSortThreads,
                                  int valuesPerThread, int bitPass, bool useTransList) {
     (void)useTransList;
@@ -998,6 +999,8 @@ sortStatus_t SORTAPI sortArrayEx(sortEngine_t engine, sortData_t data, int numSo
         int fewest = mgpu_plan_passes(numBits, MGPU_RADIX_BITS, nullptr);
         fewest += (passes ^ fewest) & 1;
         if (fewest < passes && fewest <= MGPU_MAX_PASSES) {
+            if (data->valueCount == -1 && data->numElements > 0 && !data->values[0][0])
+                return SORT_STATUS_INVALID_VALUE;
             passes = fewest;
             for (int p = 0; p < passes; ++p)
                 widths[p] = numBits / passes + (p >= passes - numBits % passes ? 1 : 0);
