@@ -330,7 +330,8 @@ sortStatus_t SORTAPI sortCheckDevice(sortEngine_t engine);
  * counter left dirty; 4 a scatter offset out of range; 5 a segment with no
  * workgroup on its XCD; 6 a packed tile with more segments than it can hold;
  * 7 a segment larger than the tile of a kernel built without the global-memory
- * routine: both only from a broken plan) without clearing it.  No counterpart
+ * routine; 8 a bucket or segment larger than its workgroup sorts: 6 to 8 only
+ * from a broken plan) without clearing it.  No counterpart
  * in the reference. */
 typedef struct {
     int device;

@@ -357,6 +357,7 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
         // flips the words whose top bit the mapping cleared.
         la.out_lo = toHi;
         la.out_hi = toLo;
+        la.error_flag = L.errorDev;
         return la;
     };
     hipFunction_t localFn = valueCount ? e->fnLocalPay : e->fnLocal;

@@ -279,6 +279,7 @@ struct mgpuSegSlotArgs {
     uint32_t first_bit;
     uint32_t num_bits;
     uint32_t pad_;
+    uint32_t* error_flag;
 };
 
 // Words of `done` counters for so many arrays, between hist and digit_start.
@@ -427,6 +428,7 @@ struct mgpuLocalArgs {
     uint32_t* starts;        // [MGPU_MAX_PASSES][MGPU_RADIX]
     uint32_t num_passes;
     uint32_t last_width;     // of the last pass's digit
+    uint32_t* error_flag;
 };
 
 // Bucketed sort of mid-sized arrays: mid_count counts the top MGPU_MID_BITS

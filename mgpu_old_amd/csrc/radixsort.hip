@@ -2441,7 +2441,11 @@ __device__ __forceinline__ void local_sort_array(const mgpuLocalArgs& a) {
     }
     if (!a.plan->buckets) return;
     const uint32_t begin = a.plan->start[b], n = a.plan->start[b + 1] - begin;
-    if (n == 0 || n > MGPU_LOCAL_MAX_KEYS) return;
+    if (n == 0) return;
+    if (n > MGPU_LOCAL_MAX_KEYS || begin > a.n || n > a.n - begin) {  // only from a broken count
+        if (threadIdx.x == 0) set_error(a.error_flag, 8u);
+        return;
+    }
     mgpu::local_sort<PAY>(mgpu::LocalArrays{a, begin}, local_mem(sh), n, a.plan->base[b],
                           a.first_bit, a.plan->bits[b]);
 }

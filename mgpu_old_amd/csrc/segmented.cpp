@@ -916,6 +916,7 @@ sortStatus_t mgpu_enqueue_slots(SegPlanData& P, SortLane& lane, hipStream_t s, b
     a.result_side = (uint32_t)P.resultSide;
     a.first_bit = (uint32_t)P.firstBit;
     a.num_bits = (uint32_t)P.numBits;
+    a.error_flag = lane.errorDev;
     const uint32_t count = (uint32_t)(P.slots.size() / 2);
     return mgpu_launch(P.engine, s, P.engine->fnSegSlots[large][P.valueCount != 0],
                        large ? count - P.slots1024 : P.slots1024,

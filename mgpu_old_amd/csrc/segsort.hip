@@ -882,6 +882,10 @@ __device__ __forceinline__ void slot_body(const mgpuSegSlotArgs& a) {
         base = at[3];
         if (n == 0) return;
     }
+    if (n > TILE || io.begin > io.d->n || n > io.d->n - io.begin) {  // only from a broken plan
+        if (threadIdx.x == 0) mgpu::set_error(a.error_flag, 8u);
+        return;
+    }
     mgpu::local_sort<PAY, BLOCK>(io, mgpu::local_mem(sh), n, base, a.first_bit, bits);
 }
 
