@@ -162,21 +162,38 @@ __device__ __forceinline__ void local_sort_items(const IO& io, const LocalMem& s
             for (int j = 0; j < IT; ++j)
                 __builtin_amdgcn_raw_buffer_store_b32(pay[j], rv, (int)(off + j * 256u), 0, 0);
         } else {
-            // Two or more arrays: gathered through the source index.
-            for (uint32_t v = 0; v < io.num_values(); ++v) {
+            // Two or more arrays, each through a stage in LDS: read in order,
+            // taken in the keys' order, written in order, so that every global
+            // access is whole lines.  Against a gather from global memory through
+            // the source index, 16384 keys with six arrays: by 8 bits 50.9 -> 20.5
+            // us (device-wide pass 23.0), by 32 bits 63.7 -> 33.4; 3 * 2^20 keys
+            // with six in buckets 143.6 -> 120.3.  The two stages alternate:
+            // one barrier an array, as a wave that writes a stage again has
+            // passed the barrier that follows all reads of it.
+            uint32_t val[IT];
+            auto load = [&](uint32_t v) {
                 const __amdgpu_buffer_rsrc_t rv = words_rsrc(io.vals_in(v), n);
-                const __amdgpu_buffer_rsrc_t ro = words_rsrc(io.vals_out(v), n);
-                uint32_t val[IT];
 #pragma unroll
                 for (int j = 0; j < IT; ++j)
-                    val[j] = __builtin_amdgcn_raw_buffer_load_b32(rv, (int)(pay[j] * 4u), 0, 0);
-                // Every gather of the workgroup has its data before the
-                // first store (the two sides may be one buffer).
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    val[j] = __builtin_amdgcn_raw_buffer_load_b32(rv, (int)(off + j * 256u), 0, 0);
+            };
+            load(0);
+            __syncthreads();  // the last pass's reads of the stages
+            for (uint32_t v = 0; v < io.num_values(); ++v) {
+                uint32_t* const stage = v & 1 ? sh.pay : sh.key;
+#pragma unroll
+                for (int j = 0; j < IT; ++j) stage[first + j * 64] = val[j];
+                if (v + 1 < io.num_values()) load(v + 1);
+                // Every wave has read this array before any writes it (the two
+                // sides may be one buffer).
                 __syncthreads();
+                const __amdgpu_buffer_rsrc_t ro = words_rsrc(io.vals_out(v), n);
+                uint32_t out[IT];
+#pragma unroll
+                for (int j = 0; j < IT; ++j) out[j] = stage[pay[j]];
 #pragma unroll
                 for (int j = 0; j < IT; ++j)
-                    __builtin_amdgcn_raw_buffer_store_b32(val[j], ro, (int)(off + j * 256u), 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b32(out[j], ro, (int)(off + j * 256u), 0, 0);
             }
         }
     }
