@@ -466,7 +466,8 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
                                                  : MGPU_VALUES_MULTI;
         const int laterMode = valueCount == -1 ? MGPU_VALUES_SINGLE : firstMode;
         const bool oneLaunch = n <= kMidOneLaunchMaxKeys && var.midRest[laterMode];
-        auto pass = [&](int p, hipFunction_t f) {
+        const bool merged = !oneLaunch && var.midLocal[laterMode];
+        auto pass = [&](int p, hipFunction_t f, uint32_t grid) {
             const int in = p & 1;
             pa.keys_in = keyBuf[in];
             pa.keys_out = keyBuf[in ^ 1];
@@ -482,26 +483,29 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
             pa.mask = (1u << widths[p]) - 1u;
             pa.key_types = p == 0 ? kernelKeyType
                            : p == numPasses - 1 || oneLaunch ? kernelKeyType << 8
+                           : p == 1 && merged                ? kernelKeyType << 16
                                                              : 0u;
-            return mgpu_launch(e, L.stream, f, numTiles, var.blockThreads, &pa, timed);
+            return mgpu_launch(e, L.stream, f, grid, var.blockThreads, &pa, timed);
         };
-        st = pass(0, var.mid[firstMode]);
+        st = pass(0, var.mid[firstMode], numTiles + 1);  // one for the plan
         if (st) return st;
-        mgpuLocalArgs la = local_args(1);
-        la.plan = L.midPlan;
-        la.hist = L.hist;
-        la.starts = L.digitStart;
-        la.num_passes = (uint32_t)numPasses;
-        la.last_width = (uint32_t)widths[numPasses - 1];
-        st = mgpu_launch(e, L.stream, localFn, MGPU_RADIX, MGPU_LOCAL_THREADS, &la, timed);
+        int next = 1;
+        if (merged) {
+            st = pass(next++, var.midLocal[laterMode], std::max<uint32_t>(MGPU_RADIX, numTiles));
+        } else {
+            mgpuLocalArgs la = local_args(1);
+            la.plan = L.midPlan;
+            la.hist = L.hist;
+            st = mgpu_launch(e, L.stream, localFn, MGPU_RADIX, MGPU_LOCAL_THREADS, &la, timed);
+        }
         if (st) return st;
         L.histDirty = false;
         if (oneLaunch) {
-            st = pass(1, var.midRest[laterMode]);
+            st = pass(next, var.midRest[laterMode], numTiles);
             if (st) return st;
         } else {
-            for (int p = 1; p < numPasses; ++p) {
-                st = pass(p, var.midPass[laterMode]);
+            for (; next < numPasses; ++next) {
+                st = pass(next, var.midPass[laterMode], numTiles);
                 if (st) return st;
             }
         }

@@ -37,10 +37,12 @@ struct PassVariant {
     hipFunction_t passKM[4] = {};
     hipFunction_t xsegKM[4] = {};
     // Bucketed sorts: the first scatter by value mode, and a pass after it when
-    // the buckets do not fit, or all of them in one launch (no index form: they
+    // the buckets do not fit, the first of those that also sorts the buckets
+    // when they do, or all of the passes in one launch (no index form: they
     // read the indices); null where not built.
     hipFunction_t mid[4] = {};
     hipFunction_t midPass[4] = {};
+    hipFunction_t midLocal[4] = {};
     hipFunction_t midRest[4] = {};
     uint32_t xsegGrid = 0;        // workgroups of an xseg launch: all that fit on the device
     uint32_t tile() const { return blockThreads * itemsPerThread; }

@@ -382,7 +382,8 @@ struct mgpuPassArgs {
     // left as they are): bits 0-7, the type of the keys the pass reads, which
     // it maps to their unsigned order (the sort's first pass); bits 8-15, the
     // type the keys it writes go back to (its last pass, which counts nothing
-    // for a next one).  One word: the kernels run short of scalar registers.
+    // for a next one); bits 16-23, the same for a launch that sorts buckets
+    // where they are used.  One word: the kernels run short of scalar registers.
     uint32_t key_types;
     uint32_t pad_;
     // Bucketed sort: the plan (its first scatter writes it, the launches of
@@ -393,8 +394,9 @@ struct mgpuPassArgs {
     // tile_counter is the counter of its items and finished[p - 1] counts the
     // tiles done of pass p.
     mgpuMidPlan* mid_plan;
-    const uint32_t* mid_hist;
-    const uint32_t* mid_starts;   // [MGPU_MAX_PASSES][MGPU_RADIX]: digit starts, for one launch of all
+    uint32_t* mid_hist;
+    uint32_t* mid_starts;         // [MGPU_MAX_PASSES][MGPU_RADIX]: digit starts of the passes after
+                                  // the first scatter, which writes them
     uint32_t mid_shift;           // of the bins
     uint32_t mid_target;
     uint32_t mid_passes;
@@ -421,13 +423,9 @@ struct mgpuLocalArgs {
     uint32_t in_lo, in_hi, out_lo, out_hi;
     uint32_t pad_;
     // Bucketed sort: workgroup b sorts bucket b of the plan (nothing when the
-    // plan does not use buckets), and workgroup p < num_passes makes pass p's
-    // digit starts of mid_count's histogram and zeroes it.
+    // plan does not use buckets), and the first one zeroes mid_count's histogram.
     const mgpuMidPlan* plan;
     uint32_t* hist;
-    uint32_t* starts;        // [MGPU_MAX_PASSES][MGPU_RADIX]
-    uint32_t num_passes;
-    uint32_t last_width;     // of the last pass's digit
     uint32_t* error_flag;
 };
 

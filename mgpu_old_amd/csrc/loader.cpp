@@ -95,6 +95,11 @@ sortStatus_t load_variant(sortEngine_d* e, uint32_t threads, uint32_t items, uin
         }
         v->midPass[m] = f;
         e->kernelNames[f] = name;
+        std::snprintf(name, sizeof(name), "mgpu_rank_scatter_b%u_i%u_r1_l_v%d", threads, items, m);
+        if (hipModuleGetFunction(&f, e->radixModule, name) == hipSuccess) {
+            v->midLocal[m] = f;
+            e->kernelNames[f] = name;
+        }
         std::snprintf(name, sizeof(name), "mgpu_rank_scatter_b%u_i%u_r1_f_v%d", threads, items, m);
         if (hipModuleGetFunction(&f, e->radixModule, name) != hipSuccess) continue;
         v->midRest[m] = f;

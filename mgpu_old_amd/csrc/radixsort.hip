@@ -1076,10 +1076,10 @@ __device__ __forceinline__ void load_striped(const uint32_t* src, uint32_t n, ui
 // digit passes take a scatter each, all of them bound by latency at these
 // sizes (10-12 us a launch).  Digit passes -> buckets, a sort with the fill of
 // its input: 20001 pairs 47.4 -> 26.4 us, 150000 51.1 -> 27.7, 2^19 61.0 ->
-// 35.0, 1000003 74.4 -> 46.7, 3000001 96.2 -> 66.8; normal floats 150000
-// 53.3 -> 42.5.  Keys that no grouping spreads: 1.0-1.08x up to 2^20 keys, at
-// 1391168 92.4 -> 93.4 us and at 2500001 98.7 -> 100.7 (the counts and the
-// check ahead of each later pass).
+// 35.0, 900001 68.8 -> 42.1, 3145728 96.1 -> 68.5; normal floats 150000
+// 53.3 -> 42.5.  Keys that no grouping spreads (low-entropy pairs), digit passes
+// -> the same behind these counts: 65536 56.6 -> 50.4 us, 400001 66.7 -> 60.9,
+// 1391168 94.0 -> 93.0, 2500001 103.2 -> 103.8, 3145728 107.8 -> 109.1.
 //
 // The digits of a bucketed sort's first scatter, worked out by every workgroup
 // from the counts while its keys load (1024 bins: a few KB from the L2 and a
@@ -1109,7 +1109,7 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
     static_assert(LANES == 2 || LANES == 4, "a group of bins is held by neighbouring lanes");
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const bool last_group = blockIdx.x + 1 == gridDim.x;
+    const bool writes = blockIdx.x == a.num_tiles;  // the workgroup without a tile
     const uint32_t field_shift = a.mid_field[0] & 0xFFu;
     auto put_plan = [&](uint32_t b, uint32_t start, uint32_t base, uint32_t bits) {
         a.mid_plan->start[b] = start;
@@ -1151,15 +1151,15 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
         before += (uint32_t)__builtin_amdgcn_readlane((int)waves, (int)(wave - 1));
         start0 += (uint32_t)__builtin_amdgcn_readlane((int)waves0, (int)(wave - 1));
     }
-    if (last_group && tid == 0) a.mid_plan->start[RADIX] = a.n;
+    if (writes && tid == 0) a.mid_plan->start[RADIX] = a.n;
     if (__builtin_amdgcn_ballot_w64(any & 1u) == 0) {
         const uint32_t g = tid / LANES;
         if (tid % LANES == 0) {
             s_start[g] = before;
-            if (last_group)
+            if (writes)
                 put_plan(g, before, g * GROUP << a.mid_shift, a.mid_shift - field_shift + 2);
         }
-        if (last_group && tid == 0) a.mid_plan->buckets = 1;
+        if (writes && tid == 0) a.mid_plan->buckets = 1;
         shift = a.mid_shift + MGPU_MID_BITS - MGPU_RADIX_BITS;
         width = MGPU_RADIX_BITS;
         mask = RADIX - 1;
@@ -1172,7 +1172,7 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
     bool fits = __builtin_amdgcn_ballot_w64(any & 2u) == 0;
     bool one = __builtin_amdgcn_ballot_w64(any & 4u) != 0;
     if (!fits && !one) {
-        if (last_group && tid == 0) a.mid_plan->buckets = 0;
+        if (writes && tid == 0) a.mid_plan->buckets = 0;
         if (tid < RADIX) s_start[tid] = start0;
         __syncthreads();
         return false;
@@ -1246,20 +1246,20 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
             const uint32_t piece = (a.n + RADIX - 1) / RADIX;
             if (tid < RADIX) {
                 s_start[tid] = start0;
-                if (last_group) put_plan(tid, min(a.n, tid * piece), 0u, 0u);
+                if (writes) put_plan(tid, min(a.n, tid * piece), 0u, 0u);
             }
-            if (last_group && tid == 0) a.mid_plan->buckets = 1;
+            if (writes && tid == 0) a.mid_plan->buckets = 1;
             __syncthreads();
             return false;
         }
     }
-    if (last_group && tid == 0) a.mid_plan->buckets = fits ? 1u : 0u;
+    if (writes && tid == 0) a.mid_plan->buckets = fits ? 1u : 0u;
     __syncthreads();  // (every wave has read s_tmp)
     uint32_t start = mgpu::block_exclusive_scan_dpp<BLOCK>(fits ? keys : 0u, s_tmp, lane, wave);
     if (!fits) start = start0;
     if (tid < RADIX) {
         s_start[tid] = start;
-        if (last_group && fits) {
+        if (writes && fits) {
             // The keys of a bucket of bins lie above its first bin, and the
             // bits that number its bins are left to sort by; the keys of a
             // digit's bucket differ below the digit only.
@@ -1277,6 +1277,50 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
     }
     return fits && digit < 0;
 }
+
+// The digit starts of the passes after the first scatter, by its workgroup
+// without a tile: the last digits are the bins' top bits.
+template <int BLOCK>
+__device__ void mid_later_starts(const mgpuPassArgs& a, uint32_t* s_tmp) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    for (uint32_t p = 1; p < a.mid_passes; ++p) {
+        const uint32_t width = a.mid_field[p] >> 8;
+        uint32_t c = 0;
+        if (p + 1 < a.mid_passes) {
+            if (tid < RADIX) c = a.mid_hist[MGPU_MID_BINS + p * RADIX + tid];
+        } else if (tid < 1u << width) {
+            const uint32_t per = MGPU_MID_BINS >> width;
+            for (uint32_t i = 0; i < per; ++i) c += a.mid_hist[tid * per + i];
+        }
+        __syncthreads();  // (s_tmp was read)
+        const uint32_t start = mgpu::block_exclusive_scan_dpp<BLOCK>(c, s_tmp, lane, wave);
+        if (tid < RADIX) a.mid_starts[p * RADIX + tid] = start;
+    }
+}
+
+// A bucket's elements for local_sort: from side 1, which the scatter filled
+// and a later pass reads, to the side that all passes would end on.
+template <int VMODE>
+struct MidBucket {
+    const mgpuPassArgs& a;
+    uint32_t begin;
+    __device__ __forceinline__ const uint32_t* keys_in() const { return a.keys_in + begin; }
+    __device__ __forceinline__ uint32_t* keys_out() const {
+        return (a.mid_passes & 1 ? const_cast<uint32_t*>(a.keys_in) : a.keys_out) + begin;
+    }
+    __device__ __forceinline__ const uint32_t* vals_in(uint32_t v) const { return a.vals_in[v] + begin; }
+    __device__ __forceinline__ uint32_t* vals_out(uint32_t v) const {
+        return (a.mid_passes & 1 ? const_cast<uint32_t*>(a.vals_in[v]) : a.vals_out[v]) + begin;
+    }
+    __device__ __forceinline__ uint32_t mode() const { return VMODE; }
+    __device__ __forceinline__ uint32_t num_values() const { return a.num_values; }
+    __device__ __forceinline__ uint32_t read(uint32_t k) const { return k; }
+    __device__ __forceinline__ uint32_t write(uint32_t k) const {
+        const uint32_t type = a.key_types >> 16;
+        return type ? mgpu_key_from_radix(k, type) : k;
+    }
+};
 
 // RANK 0: in-wave ranking by LDS match masks (documented behaviour only).
 // RANK 1: one LDS atomic add per key on the wave's count of its digit: the
@@ -1299,7 +1343,9 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
 // buckets looked up by the key's bin when the counts allow it, else the first
 // pass's digits; 2 is a pass after it, which returns at once when buckets were
 // used; 3 is all of those passes in one launch (returning at once costs ~3 us a
-// launch).  Its work items, (pass, tile) in order, come from one counter; an item waits
+// launch); 4 is the pass after the scatter and, where buckets were used, the
+// sort of each of them: the launch of that sort alone costs 5 us, which keys
+// that no grouping spreads paid for nothing.  MID 3's work items, (pass, tile) in order, come from one counter; an item waits
 // for the pass before it to be complete, that is for items handed out earlier
 // to workgroups that run, so no number of resident workgroups is needed.  Data
 // goes between XCDs inside the launch: loads and stores are coherent ones.
@@ -1307,6 +1353,7 @@ template <int BLOCK, int IPT, int RANK, int VMODE, bool MULTI, bool XSEG, bool E
           int MID, typename Args>
 __device__ void rank_scatter_body(const Args& a) {
     static_assert(MID == 0 || (RANK == 1 && !MULTI && !XSEG && !EE), "one array, one chain");
+    static_assert(MID != 4 || BLOCK * IPT == MGPU_LOCAL_MAX_KEYS, "a workgroup sorts a bucket");
     if constexpr (MID == 2 || MID == 3) {
         if (a.mid_plan->buckets) return;
     }
@@ -1333,7 +1380,8 @@ __device__ void rank_scatter_body(const Args& a) {
     // staged, so they share the value stage's memory.
     constexpr bool JOINT = VMODE == MGPU_VALUES_SINGLE || VMODE == MGPU_VALUES_INDEX;
     constexpr uint32_t MATCH_WORDS = RANK == 0 ? (uint32_t)W * RADIX * 2 : 0;
-    constexpr uint32_t AUX_WORDS0 = JOINT && TILE > MATCH_WORDS ? TILE : MATCH_WORDS;
+    constexpr uint32_t AUX_WORDS0 =
+        (JOINT || (MID == 4 && VMODE == MGPU_VALUES_MULTI)) && TILE > MATCH_WORDS ? TILE : MATCH_WORDS;
     constexpr uint32_t AUX_WORDS = AUX_WORDS0 > 0 ? AUX_WORDS0 : 2;
     __shared__ uint32_t s_stage[TILE];
     __shared__ __attribute__((aligned(16))) uint32_t s_aux[AUX_WORDS];
@@ -1363,6 +1411,26 @@ __device__ void rank_scatter_body(const Args& a) {
     }
     __shared__ uint32_t s_map[MID == 1 ? MGPU_MID_BINS : 1];  // bin (or digit) -> digit
     uint32_t* const row = s_count[wave];  // this wave's digit counts
+    if constexpr (MID == 4) {
+        if (blockIdx.x == 0)
+            for (uint32_t i = tid; i < MGPU_MID_HIST_WORDS; i += BLOCK) a.mid_hist[i] = 0;
+        if (a.mid_plan->buckets) {
+            if (blockIdx.x >= RADIX) return;
+            const mgpuMidPlan& plan = *a.mid_plan;
+            const uint32_t begin = plan.start[blockIdx.x], n = plan.start[blockIdx.x + 1] - begin;
+            if (n == 0) return;
+            if (n > MGPU_LOCAL_MAX_KEYS || begin > a.n || n > a.n - begin) {
+                if (tid == 0) set_error(a.error_flag, 8u);  // only from a broken count
+                return;
+            }
+            const mgpu::LocalMem mem{&s_count[0][0], s_tmp, s_stage, s_aux};
+            mgpu::local_sort<VMODE != MGPU_VALUES_NONE>(MidBucket<VMODE>{a, begin}, mem, n,
+                                                        plan.base[blockIdx.x], a.mid_field[0] & 0xFFu,
+                                                        plan.bits[blockIdx.x]);
+            return;
+        }
+        if (blockIdx.x >= a.num_tiles) return;
+    }
     const uint32_t gd = tid / G, gk = tid % G;
     uint32_t* const col = &s_count[gk * R][gd];
 
@@ -1434,6 +1502,8 @@ __device__ void rank_scatter_body(const Args& a) {
     // take in order (thread 0; seg_tiles when there is none left).
     auto take_tile = [&]() {
         uint32_t t = seg_tiles;  // a workgroup of an XCD without a segment takes none
+        if constexpr (MID == 1)
+            if (blockIdx.x == a.num_tiles) return t;
         bool grouped = false;
         if constexpr (MULTI && !XSEG) grouped = a.num_xcds > 1;
         if (grouped) {
@@ -1481,7 +1551,7 @@ __device__ void rank_scatter_body(const Args& a) {
             load_striped<IPT, LAUX>(vals_in(job, 0), job.n, wave_base, lane, val);
     };
     uint32_t key_types = 0;
-    if constexpr (KMAP) key_types = a.key_types;
+    if constexpr (KMAP && MID != 4) key_types = a.key_types;  // (4: neither first nor last)
     // MID 3: the next item, once the pass before its own is complete.
     auto take_item = [&](TileJob& job) -> bool {
         if constexpr (MID == 3) {
@@ -1561,12 +1631,19 @@ __device__ void rank_scatter_body(const Args& a) {
         __syncthreads();
         gtile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
         // One tile per workgroup: only a counter left dirty finds none.
-        if (!XSEG && gtile >= seg_tiles && tid == 0) set_error(a.error_flag, 2u);
+        if (!XSEG && gtile >= seg_tiles && tid == 0 && (MID != 1 || blockIdx.x < a.num_tiles))
+            set_error(a.error_flag, 2u);
         if (gtile < seg_tiles && !start_tile(gtile)) gtile = seg_tiles;
     }
     if constexpr (MID == 1)
+    {
         mapped = mid_plan_tile<BLOCK>(a, mid_bins, mid_digit0, s_map, s_global, s_tmp, s_stage, shift, width,
                              mask);
+        if (blockIdx.x == a.num_tiles) {
+            mid_later_starts<BLOCK>(a, s_tmp);
+            return;
+        }
+    }
     while (gtile < seg_tiles) {
         const uint32_t n = job.n, tile = job.tile;
         const uint32_t base = (job.first + tile) * TILE;
@@ -2417,8 +2494,8 @@ MGPU_RANK_SCATTER(256, 16, 1)
 MGPU_RANK_SCATTER(512, 16, 1)
 MGPU_RANK_SCATTER(1024, 16, 1)
 // A bucketed sort's first scatter (_m_) and the passes after it when buckets
-// do not fit: each a launch (_c_), or all in one (_f_); they read no generated
-// indices.
+// do not fit: each a launch (_c_; _l_ is the first of them and sorts the
+// buckets where they fit), or all in one (_f_); they read no generated indices.
 #define MGPU_RANK_SCATTER_MID_MODE(B, I, T, M, V, MODE)                                       \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_##T##_v##V(mgpuPassArgs a) {                       \
@@ -2432,6 +2509,9 @@ MGPU_RANK_SCATTER(1024, 16, 1)
     MGPU_RANK_SCATTER_MID_MODE(B, I, c, 2, 0, MGPU_VALUES_NONE)                               \
     MGPU_RANK_SCATTER_MID_MODE(B, I, c, 2, 2, MGPU_VALUES_SINGLE)                             \
     MGPU_RANK_SCATTER_MID_MODE(B, I, c, 2, 3, MGPU_VALUES_MULTI)
+MGPU_RANK_SCATTER_MID_MODE(1024, 16, l, 4, 0, MGPU_VALUES_NONE)
+MGPU_RANK_SCATTER_MID_MODE(1024, 16, l, 4, 2, MGPU_VALUES_SINGLE)
+MGPU_RANK_SCATTER_MID_MODE(1024, 16, l, 4, 3, MGPU_VALUES_MULTI)
 MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 0, MGPU_VALUES_NONE)
 MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 2, MGPU_VALUES_SINGLE)
 MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 3, MGPU_VALUES_MULTI)
@@ -2456,27 +2536,9 @@ __device__ __forceinline__ void local_sort_array(const mgpuLocalArgs& a) {
                               a.num_bits);
         return;
     }
-    // The counts go back to zero; when the digit passes go on, workgroup p first
-    // makes pass p's digit starts of them (the last digits are the bins' top
-    // bits).
     const uint32_t b = blockIdx.x;
-    if (b < a.num_passes) {
-        const uint32_t tid = threadIdx.x, first = b + 1 == a.num_passes ? 0u : MGPU_MID_BINS + b * RADIX;
-        uint32_t* const h = a.hist + first;
-        uint32_t cnt = 0;
-        if (first == 0) {
-            const uint32_t per = MGPU_MID_BINS >> a.last_width;
-            if (tid < (1u << a.last_width))
-                for (uint32_t i = 0; i < per; ++i) cnt += h[tid * per + i];
-        } else if (tid < RADIX) {
-            cnt = h[tid];
-        }
-        const uint32_t st = mgpu::block_exclusive_scan_dpp<MGPU_LOCAL_THREADS>(
-            cnt, sh.tmp, tid & 63, (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)));
-        if (tid < RADIX) a.starts[b * RADIX + tid] = st;
-        __syncthreads();
-        if (first == 0 || tid < RADIX) h[tid] = 0;
-    }
+    if (b == 0)
+        for (uint32_t i = threadIdx.x; i < MGPU_MID_HIST_WORDS; i += MGPU_LOCAL_THREADS) a.hist[i] = 0;
     if (!a.plan->buckets) return;
     const uint32_t begin = a.plan->start[b], n = a.plan->start[b + 1] - begin;
     if (n == 0) return;
