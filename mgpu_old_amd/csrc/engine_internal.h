@@ -21,6 +21,9 @@ struct PassVariant {
     hipFunction_t xseg[4] = {};   // mgpu_rank_scatter_b*_i*_r*_x_v<mode>: a chain per XCD segment
     hipFunction_t multi[4] = {};  // mgpu_multi_scatter_b*_i*_r*_v<mode>
     hipFunction_t multiX[4] = {}; // mgpu_multi_scatter_b*_i*_r*_x_v<mode>: chains per XCD
+    // The second pass of a bucketed batch, whose first workgroups sort its slots
+    // (atomic-add ranking, 512 x 16, no index form; null elsewhere).
+    hipFunction_t multiSlots[4] = {};
     uint32_t multiXGrid = 0;      // workgroups of a multiX launch: all that fit
     // Packed tiles of several arrays (atomic-add ranking only; null when not
     // built for the shape): mgpu_multi_packed_b*_i*_v<mode> and ..._x_v<mode>.

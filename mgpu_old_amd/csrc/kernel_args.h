@@ -132,8 +132,8 @@ struct mgpuScanArgs {
 #define MGPU_UNSORTED_SLOT (MGPU_FINISHED_SLOT + MGPU_MAX_PASSES)
 // Most frequent digit of each pass (segments per XCD only; digit_scan).
 #define MGPU_MODE_SLOT (MGPU_UNSORTED_SLOT + 8)
-// Segments of the last device-wide count that take every digit pass (not
-// zeroed with the counters before it: the bucket kernel zeroes it).
+// Segments that take every digit pass: as the device-wide count adds them up
+// (the first pass zeroes it), then as the passes after the first find them.
 #define MGPU_LSD_SLOT (MGPU_MODE_SLOT + MGPU_MAX_PASSES)
 #define MGPU_LANE_COUNTERS (MGPU_LSD_SLOT + 2)
 
@@ -262,26 +262,6 @@ struct mgpuMultiCountArgs {
     uint32_t* lsd_segments;
 };
 
-// A workgroup per slot, of 512 threads (up to MGPU_BUCKET_KEYS keys) or 1024: a bucket of a device-wide segment, or
-// a whole segment (MGPU_SLOT_WHOLE: seg indexes segs, else wide).
-#define MGPU_SLOT_WHOLE 0xFFFFFFFFu
-#define MGPU_BUCKET_THREADS 512
-#define MGPU_BUCKET_KEYS 8192
-struct mgpuSegSlotArgs {
-    const mgpuSegDesc* segs;
-    const mgpuSegDesc* wide;
-    const uint32_t* slots;        // [grid][2]: seg, bucket
-    const uint32_t* digit_start;  // blocks of the device-wide segments, as above
-    uint32_t* lsd_segments;       // zeroed
-    uint32_t num_values;
-    uint32_t index_mode;
-    uint32_t result_side;
-    uint32_t first_bit;
-    uint32_t num_bits;
-    uint32_t pad_;
-    uint32_t* error_flag;
-};
-
 // Words of `done` counters for so many arrays, between hist and digit_start.
 #define MGPU_MULTI_DONE_WORDS(arrays) (((size_t)(arrays) + 63) & ~(size_t)63)
 
@@ -292,6 +272,25 @@ struct mgpuMultiScanArgs {
     uint32_t* tile_counters;  // [MGPU_LANE_COUNTERS]
     uint32_t num_passes;
     uint32_t pad_;
+};
+
+// A workgroup per slot, of 512 threads (up to MGPU_BUCKET_KEYS keys) or 1024: a bucket of a device-wide segment, or
+// a whole segment (MGPU_SLOT_WHOLE: seg indexes segs, else wide).
+#define MGPU_SLOT_WHOLE 0xFFFFFFFFu
+#define MGPU_BUCKET_THREADS 512
+#define MGPU_BUCKET_KEYS 8192
+struct mgpuSegSlotArgs {
+    const mgpuSegDesc* segs;
+    const mgpuSegDesc* wide;
+    const uint32_t* slots;        // [grid][2]: seg, bucket
+    const uint32_t* digit_start;  // blocks of the device-wide segments, as above
+    uint32_t num_values;
+    uint32_t index_mode;
+    uint32_t result_side;
+    uint32_t first_bit;
+    uint32_t num_bits;
+    uint32_t pad_;
+    uint32_t* error_flag;
 };
 
 // rank_scatter over the tiles of all arrays.
@@ -333,9 +332,14 @@ struct mgpuMultiPassArgs {
     // bits 16-23: chunks holding keys (the rest are padding), bit 24: the
     // first chunk continues an array begun in an earlier tile.
     const uint32_t* tile_info;
-    // Bucketed batches, passes after the first: the count of segments that
-    // take them (the launch returns at once when it is zero).
-    const uint32_t* lsd_segments;
+    // Bucketed batches (else null): the two words at MGPU_LSD_SLOT.  The first
+    // pass moves the count to the second word, and a launch of a later pass
+    // returns at once when that is zero.
+    uint32_t* lsd_segments;
+    // Launches that sort slots as well (their first num_slots workgroups).
+    mgpuSegSlotArgs slot;
+    uint32_t num_slots;
+    uint32_t pad2_;
 };
 
 // Parts (arrays) per packed tile of W waves.

@@ -107,6 +107,18 @@ sortStatus_t load_variant(sortEngine_d* e, uint32_t threads, uint32_t items, uin
     }
     if (!v->mid[MGPU_VALUES_MULTI])
         for (int m = 0; m < 4; ++m) v->mid[m] = v->midPass[m] = nullptr;
+    for (int m = 0; m < 4 && rank == 1; ++m) {
+        char name[96];
+        hipFunction_t f = nullptr;
+        if (m == MGPU_VALUES_INDEX) continue;
+        std::snprintf(name, sizeof(name), "mgpu_multi_scatter_slots_b%u_i%u_v%d", threads, items, m);
+        if (hipModuleGetFunction(&f, e->radixModule, name) != hipSuccess) {
+            for (int k = 0; k < 4; ++k) v->multiSlots[k] = nullptr;
+            break;
+        }
+        v->multiSlots[m] = f;
+        e->kernelNames[f] = name;
+    }
     // Packed multi-array forms, likewise.
     bool packed = rank == 1;
     for (int m = 0; m < 4 && packed; ++m) {

@@ -211,4 +211,59 @@ __device__ __forceinline__ void local_sort(const IO& io, const LocalMem& sh, uin
     else local_sort_items<B, 16, PAY>(io, sh, n, base, shift, bits);
 }
 
+// A segment's descriptor does not change while a kernel that sorts it runs, so
+// it is read through the constant address space: scalar loads, once a wave.
+typedef const __attribute__((address_space(4))) mgpuSegDesc* ConstDesc;
+typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
+
+// A slot's elements for local_sort_items.
+struct SlotIO {
+    ConstDesc d;
+    uint32_t begin, in, out, fill, values;
+    __device__ __forceinline__ const uint32_t* keys_in() const { return d->keys[in] + begin; }
+    __device__ __forceinline__ uint32_t* keys_out() const { return d->keys[out] + begin; }
+    __device__ __forceinline__ const uint32_t* vals_in(uint32_t v) const { return d->vals[v][in] + begin; }
+    __device__ __forceinline__ uint32_t* vals_out(uint32_t v) const { return d->vals[v][out] + begin; }
+    __device__ __forceinline__ uint32_t mode() const { return fill; }
+    __device__ __forceinline__ uint32_t num_values() const { return values; }
+    __device__ __forceinline__ uint32_t read(uint32_t k) const { return k; }
+    __device__ __forceinline__ uint32_t write(uint32_t k) const { return k; }
+};
+
+// A workgroup per bucket (read from side
+// 1, where the one scatter left it) or whole segment.  Bound by LDS round trips
+// and barriers as local_sort_items is (4096 segments log-uniform in [1, 2^16]:
+// 23 M pairs at ~150 keys a nanosecond, 2.4 TB/s), so buckets are of a size
+// that fits two workgroups on a CU: with 1024 threads and 11520 keys, one on a
+// CU, that batch took 371 us in all instead of 329, keys only 298 instead of
+// 239.
+template <int BLOCK, uint32_t TILE, bool PAY>
+__device__ __forceinline__ void sort_slot(const mgpuSegSlotArgs& a, const LocalMem& mem, uint32_t slot) {
+    const uint32_t seg = a.slots[2 * slot], bucket = a.slots[2 * slot + 1];
+    const uint32_t moved = a.num_values > 1 ? MGPU_VALUES_MULTI : MGPU_VALUES_SINGLE;
+    SlotIO io{(ConstDesc)(a.segs + seg), 0u, 0u, a.result_side,
+              a.index_mode ? MGPU_VALUES_INDEX : moved, a.num_values};
+    uint32_t n, base = 0, bits = a.num_bits;
+    if (bucket == MGPU_SLOT_WHOLE) {
+        n = io.d->n;
+    } else {
+        io.d = (ConstDesc)(a.wide + seg);
+        if (io.d->route == 0) return;
+        const ConstWords at = (ConstWords)(a.digit_start + (size_t)seg * (MGPU_MAX_PASSES * MGPU_RADIX) +
+                                           MGPU_RADIX + 4 * bucket);
+        io.begin = at[0];
+        io.in = 1;
+        io.fill = moved;
+        n = at[1];
+        bits = at[2];
+        base = at[3];
+        if (n == 0) return;
+    }
+    if (n > TILE || io.begin > io.d->n || n > io.d->n - io.begin) {  // only from a broken plan
+        if (threadIdx.x == 0) set_error(a.error_flag, 8u);
+        return;
+    }
+    local_sort<PAY, BLOCK>(io, mem, n, base, a.first_bit, bits);
+}
+
 }  // namespace mgpu

@@ -1345,14 +1345,19 @@ struct MidBucket {
 // used; 3 is all of those passes in one launch (returning at once costs ~3 us a
 // launch); 4 is the pass after the scatter and, where buckets were used, the
 // sort of each of them: the launch of that sort alone costs 5 us, which keys
-// that no grouping spreads paid for nothing.  MID 3's work items, (pass, tile) in order, come from one counter; an item waits
+// that no grouping spreads paid for nothing.  5 is the second pass over several
+// arrays, whose first workgroups sort the batch's slots.  MID 3's work items, (pass, tile) in order, come from one counter; an item waits
 // for the pass before it to be complete, that is for items handed out earlier
 // to workgroups that run, so no number of resident workgroups is needed.  Data
 // goes between XCDs inside the launch: loads and stores are coherent ones.
 template <int BLOCK, int IPT, int RANK, int VMODE, bool MULTI, bool XSEG, bool EE, bool KMAP,
           int MID, typename Args>
 __device__ void rank_scatter_body(const Args& a) {
-    static_assert(MID == 0 || (RANK == 1 && !MULTI && !XSEG && !EE), "one array, one chain");
+    static_assert(MID == 0 || MID == 5 || (RANK == 1 && !MULTI && !XSEG && !EE),
+                  "one array, one chain");
+    static_assert(MID != 5 || (RANK == 1 && MULTI && !XSEG && BLOCK == MGPU_BUCKET_THREADS &&
+                               BLOCK * IPT == MGPU_BUCKET_KEYS),
+                  "a workgroup sorts a slot");
     static_assert(MID != 4 || BLOCK * IPT == MGPU_LOCAL_MAX_KEYS, "a workgroup sorts a bucket");
     if constexpr (MID == 2 || MID == 3) {
         if (a.mid_plan->buckets) return;
@@ -1381,7 +1386,7 @@ __device__ void rank_scatter_body(const Args& a) {
     constexpr bool JOINT = VMODE == MGPU_VALUES_SINGLE || VMODE == MGPU_VALUES_INDEX;
     constexpr uint32_t MATCH_WORDS = RANK == 0 ? (uint32_t)W * RADIX * 2 : 0;
     constexpr uint32_t AUX_WORDS0 =
-        (JOINT || (MID == 4 && VMODE == MGPU_VALUES_MULTI)) && TILE > MATCH_WORDS ? TILE : MATCH_WORDS;
+        (JOINT || (MID >= 4 && VMODE == MGPU_VALUES_MULTI)) && TILE > MATCH_WORDS ? TILE : MATCH_WORDS;
     constexpr uint32_t AUX_WORDS = AUX_WORDS0 > 0 ? AUX_WORDS0 : 2;
     __shared__ uint32_t s_stage[TILE];
     __shared__ __attribute__((aligned(16))) uint32_t s_aux[AUX_WORDS];
@@ -1406,8 +1411,22 @@ __device__ void rank_scatter_body(const Args& a) {
     uint32_t width = (uint32_t)__builtin_popcount(mask);  // mask = 2^width - 1
     // One tile per workgroup, of several arrays: passes of a bucketed batch.
     constexpr bool ROUTED = MULTI && RANK == 1 && !XSEG;
+    if constexpr (MID == 5) {
+        if (blockIdx.x < a.num_slots) {
+            mgpu::sort_slot<BLOCK, TILE, VMODE != MGPU_VALUES_NONE>(
+                a.slot, mgpu::LocalMem{&s_count[0][0], s_tmp, s_stage, s_aux}, blockIdx.x);
+            return;
+        }
+    }
     if constexpr (ROUTED) {
-        if (a.lsd_segments != nullptr && *a.lsd_segments == 0) return;
+        if (a.lsd_segments != nullptr) {
+            if (a.pass != 0) {
+                if (a.lsd_segments[1] == 0) return;
+            } else if (blockIdx.x == 0 && tid == 0) {
+                a.lsd_segments[1] = a.lsd_segments[0];
+                a.lsd_segments[0] = 0;
+            }
+        }
     }
     __shared__ uint32_t s_map[MID == 1 ? MGPU_MID_BINS : 1];  // bin (or digit) -> digit
     uint32_t* const row = s_count[wave];  // this wave's digit counts
@@ -2512,6 +2531,15 @@ MGPU_RANK_SCATTER(1024, 16, 1)
 MGPU_RANK_SCATTER_MID_MODE(1024, 16, l, 4, 0, MGPU_VALUES_NONE)
 MGPU_RANK_SCATTER_MID_MODE(1024, 16, l, 4, 2, MGPU_VALUES_SINGLE)
 MGPU_RANK_SCATTER_MID_MODE(1024, 16, l, 4, 3, MGPU_VALUES_MULTI)
+// The second pass of a bucketed batch, which sorts the buckets as well.
+#define MGPU_MULTI_SLOTS(V, MODE)                                                             \
+    extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) \
+        mgpu_multi_scatter_slots_b512_i16_v##V(mgpuMultiPassArgs a) {                          \
+        rank_scatter_body<512, 16, 1, MODE, true, false, false, false, 5>(a);                 \
+    }
+MGPU_MULTI_SLOTS(0, MGPU_VALUES_NONE)
+MGPU_MULTI_SLOTS(2, MGPU_VALUES_SINGLE)
+MGPU_MULTI_SLOTS(3, MGPU_VALUES_MULTI)
 MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 0, MGPU_VALUES_NONE)
 MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 2, MGPU_VALUES_SINGLE)
 MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 3, MGPU_VALUES_MULTI)

@@ -362,11 +362,12 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
 
     // Group segments by kernel variant; very large ones go device-wide.
     const uint32_t wideMin = device_wide_min(e), chunkKeys = wide_chunk(e);
-    uint32_t keep = keep_in_workgroup(e), longestSeg = 0, numSmall = 0;
+    uint32_t keep = keep_in_workgroup(e), longestSeg = 0, numSmall = 0, numWhole = 0;
     uint64_t longKeys = 0;  // in segments above a bucket's size
     for (int i = 0; i < numSegments; ++i) {
         longestSeg = std::max(longestSeg, segs[i].n);
         if (segs[i].n < wideMin) ++numSmall;
+        else if (segs[i].n <= keep) ++numWhole;
         if (segs[i].n > MGPU_BUCKET_KEYS) longKeys += segs[i].n;
     }
     const bool directCount = count_cols() && longestSeg <= kDirectCountMax &&
@@ -384,6 +385,9 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         smallInSlots = numSmall <= (uint32_t)e->numCUs;
     }
     const bool noneAboveTile = longestSeg <= keep && seg_fits_tile(e, longestSeg);
+    // Beside the side stream: where the segments that a workgroup sorts whole
+    // are no more than the CUs, one launch sorts them all there.
+    const bool few = !lane.noSide && numWhole <= (uint32_t)e->numCUs;
     struct Group {
         std::vector<uint32_t> big, small;
     };
@@ -394,7 +398,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         if (n == 0 || P.numBits == 0) continue;
         if ((n >= wideMin && !noneAboveTile) || smallInSlots) {
             if (n <= keep) {
-                auto& list = n <= MGPU_BUCKET_KEYS ? P.slots : slots1024;
+                auto& list = n <= MGPU_BUCKET_KEYS && !few ? P.slots : slots1024;
                 list.push_back((uint32_t)i);
                 list.push_back(MGPU_SLOT_WHOLE);
             } else {
@@ -764,8 +768,9 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         }
         if (st) return st;
     }
-    // The side stream (before any capture) when there is something to fork.
-    if (!lane.noSide && !P.launches.empty() && (!P.wide.empty() || !P.slots.empty())) {
+    // The side stream (before any capture) when there may be something to fork.
+    if (!lane.noSide && ((!P.launches.empty() && (!P.wide.empty() || !P.slots.empty())) ||
+                         (!P.wide.empty() && !P.slots.empty()))) {
         sortStatus_t st = mgpu_lane_ensure_side(lane);
         if (st) return st;
     }
@@ -784,9 +789,40 @@ uint32_t* wide_digit_start(const SegPlanData& P, const SortLane& lane) {
            MGPU_MULTI_DONE_WORDS(P.ownMulti ? P.wide.size() : (size_t)lane.multiArrays);
 }
 
+// The workgroups' sorts of whole segments with 1024 threads (large), or the
+// others.
+mgpuSegSlotArgs slot_args(const SegPlanData& P, const SortLane& lane, bool large) {
+    mgpuSegSlotArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.segs = P.devSegs;
+    a.wide = P.devWide;
+    a.slots = P.devSlots + (large ? 2 * P.slots1024 : 0);
+    a.digit_start = wide_digit_start(P, lane);
+    a.num_values = P.valueCount == -1 ? 1u : (uint32_t)P.valueCount;
+    a.index_mode = P.valueCount == -1;
+    a.result_side = (uint32_t)P.resultSide;
+    a.first_bit = (uint32_t)P.firstBit;
+    a.num_bits = (uint32_t)P.numBits;
+    a.error_flag = lane.errorDev;
+    return a;
+}
+
+sortStatus_t mgpu_enqueue_slots(SegPlanData& P, SortLane& lane, hipStream_t s, bool large) {
+    mgpuSegSlotArgs a = slot_args(P, lane, large);
+    const uint32_t count = (uint32_t)(P.slots.size() / 2);
+    return mgpu_launch(P.engine, s, P.engine->fnSegSlots[large][P.valueCount != 0],
+                       large ? count - P.slots1024 : P.slots1024,
+                       large ? MGPU_LOCAL_THREADS : MGPU_BUCKET_THREADS, &a);
+}
+
 // The device-wide passes over every large segment of the plan at once:
 // digit_count over their chunks, digit_scan per segment, then one
 // rank_scatter launch per pass over the tiles of all of them.
+// Where the segments go through buckets, these (and the segments sorted whole
+// with them) are sorted in the launch of the second pass, or before it where
+// the tile shape has no such form.  (The passes after the first on the side
+// stream instead, beside the buckets' sorts: every join of two branches of a
+// graph costs ~15 us, 8 segments of 32768 keys 56 -> 79 us.)
 sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
     sortEngine_d* e = P.engine;
     const uint32_t np = (uint32_t)P.sortPasses;
@@ -844,6 +880,12 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
 
     const int carried = P.valueCount == -1 ? 1 : P.valueCount;
     for (uint32_t p = 0; p < np; ++p) {
+        const bool slots = P.wideBuckets && p == 1;
+        const bool merged = slots && P.wideVariant->multiSlots[MGPU_VALUES_NONE] != nullptr;
+        if (slots && !merged) {
+            st = mgpu_enqueue_slots(P, lane, lane.stream, false);
+            if (st) return st;
+        }
         mgpuMultiPassArgs pa;
         std::memset(&pa, 0, sizeof(pa));
         pa.segs = P.devWide;
@@ -861,7 +903,7 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
         pa.shift = ca.shift[p];
         pa.mask = ca.mask[p];
         pa.num_values = (uint32_t)carried;
-        if (P.wideBuckets && p > 0) pa.lsd_segments = lane.tileCounters + MGPU_LSD_SLOT;
+        if (P.wideBuckets) pa.lsd_segments = lane.tileCounters + MGPU_LSD_SLOT;
         int mode;
         if (P.valueCount == 0) mode = MGPU_VALUES_NONE;
         else if (P.valueCount == -1) mode = p == 0 ? MGPU_VALUES_INDEX : MGPU_VALUES_SINGLE;
@@ -889,38 +931,19 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
                 pa.xcd_tile_begin = P.devXcdTileBegin;
                 pa.num_xcds = P.wideGroups;
             }
+            if (merged) {
+                pa.slot = slot_args(P, lane, false);
+                pa.num_slots = P.slots1024;
+            }
             st = mgpu_launch(e, lane.stream,
-                             P.widePacked ? P.wideVariant->packed[mode] : P.wideVariant->multi[mode],
-                             P.wideTiles, P.wideVariant->blockThreads, &pa);
+                             P.widePacked ? P.wideVariant->packed[mode]
+                             : merged     ? P.wideVariant->multiSlots[mode]
+                                          : P.wideVariant->multi[mode],
+                             P.wideTiles + pa.num_slots, P.wideVariant->blockThreads, &pa);
         }
         if (st) return st;
     }
     return SORT_STATUS_SUCCESS;
-}
-
-}  // namespace
-
-namespace {
-
-// The workgroups' sorts of whole segments with 1024 threads, or the others.
-sortStatus_t mgpu_enqueue_slots(SegPlanData& P, SortLane& lane, hipStream_t s, bool large) {
-    mgpuSegSlotArgs a;
-    std::memset(&a, 0, sizeof(a));
-    a.segs = P.devSegs;
-    a.wide = P.devWide;
-    a.slots = P.devSlots + (large ? 2 * P.slots1024 : 0);
-    a.digit_start = wide_digit_start(P, lane);
-    a.lsd_segments = P.wideBuckets && !large ? lane.tileCounters + MGPU_LSD_SLOT : nullptr;
-    a.num_values = P.valueCount == -1 ? 1u : (uint32_t)P.valueCount;
-    a.index_mode = P.valueCount == -1;
-    a.result_side = (uint32_t)P.resultSide;
-    a.first_bit = (uint32_t)P.firstBit;
-    a.num_bits = (uint32_t)P.numBits;
-    a.error_flag = lane.errorDev;
-    const uint32_t count = (uint32_t)(P.slots.size() / 2);
-    return mgpu_launch(P.engine, s, P.engine->fnSegSlots[large][P.valueCount != 0],
-                       large ? count - P.slots1024 : P.slots1024,
-                       large ? MGPU_LOCAL_THREADS : MGPU_BUCKET_THREADS, &a);
 }
 
 }  // namespace
@@ -936,7 +959,15 @@ sortStatus_t mgpu_seg_enqueue(SegPlanData& P, SortLane& lane) {
     // each other, measured no faster: 4096 segments 0.614, 0.613, 0.619 ms
     // with one, two and three.  Forking after the device-wide count, so that
     // the count runs alone, was slower: 0.600 -> 0.639 ms.)
-    const bool fork = !P.launches.empty() && (!P.wide.empty() || !P.slots.empty()) && lane.side;
+    // Segments sorted whole by a workgroup each go beside the device-wide passes
+    // too (unless they share a launch with buckets).  After the passes they held
+    // a small batch up: 40 segments log-uniform in [1, 2^16], key + value, 107
+    // us, with one launch for all of those beside the passes 95.
+    const bool large = P.slots.size() / 2 > P.slots1024;
+    const bool whole = P.slots1024 != 0 && !P.wideBuckets;
+    const bool fork = lane.side && !lane.noSide &&
+                      (P.wide.empty() ? !P.launches.empty() && (large || whole)
+                                      : !P.launches.empty() || large || whole);
     hipStream_t ls = lane.stream;
     if (fork) {
         if (hipEventRecord(lane.fork, lane.stream) != hipSuccess ||
@@ -965,16 +996,16 @@ sortStatus_t mgpu_seg_enqueue(SegPlanData& P, SortLane& lane) {
         sortStatus_t st = mgpu_launch(e, ls, L.fn, L.grid, L.block, &a);
         if (st) return st;
     }
-    if (P.slots.size() / 2 > P.slots1024) {
+    if (large) {
         sortStatus_t st = mgpu_enqueue_slots(P, lane, ls, true);
+        if (st) return st;
+    }
+    if (whole) {
+        sortStatus_t st = mgpu_enqueue_slots(P, lane, P.wide.empty() ? lane.stream : ls, false);
         if (st) return st;
     }
     if (!P.wide.empty()) {
         sortStatus_t st = mgpu_enqueue_wide(P, lane);
-        if (st) return st;
-    }
-    if (P.slots1024 != 0) {
-        sortStatus_t st = mgpu_enqueue_slots(P, lane, lane.stream, false);
         if (st) return st;
     }
     if (fork && (hipEventRecord(lane.join, lane.side) != hipSuccess ||

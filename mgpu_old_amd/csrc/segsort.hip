@@ -486,16 +486,15 @@ __device__ __forceinline__ void global_sort(const mgpuSegArgs& a, const mgpuSegD
 // [64, 4096] 297 -> 186 / 357 -> 214 / 411 -> 261; 5000 of 512 105 -> 72 /
 // 125 -> 79 / 134 -> 85.
 
-// A segment's arrays.  Its descriptor does not change while the kernel runs,
-// so it is read through the constant address space: scalar loads, once a wave.
+using mgpu::ConstDesc;
+using mgpu::ConstWords;
+
+// A segment's arrays, read through the constant address space.
 struct SegArrays {
     const uint32_t *ki, *vi;  // keys and the first values, input side
     uint32_t *ko, *vo;        // result side
     uint32_t seg, n;
 };
-
-typedef const __attribute__((address_space(4))) mgpuSegDesc* ConstDesc;
-typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
 
 __device__ __forceinline__ SegArrays seg_arrays(const mgpuSegArgs& a, uint32_t seg) {
     const ConstDesc d = (ConstDesc)(a.segs + seg);
@@ -837,68 +836,18 @@ __device__ __forceinline__ void segsort_body(const mgpuSegArgs& a) {
     }
 }
 
-// A slot's elements for local_sort_items.
-struct SlotIO {
-    ConstDesc d;
-    uint32_t begin, in, out, fill, values;
-    __device__ __forceinline__ const uint32_t* keys_in() const { return d->keys[in] + begin; }
-    __device__ __forceinline__ uint32_t* keys_out() const { return d->keys[out] + begin; }
-    __device__ __forceinline__ const uint32_t* vals_in(uint32_t v) const { return d->vals[v][in] + begin; }
-    __device__ __forceinline__ uint32_t* vals_out(uint32_t v) const { return d->vals[v][out] + begin; }
-    __device__ __forceinline__ uint32_t mode() const { return fill; }
-    __device__ __forceinline__ uint32_t num_values() const { return values; }
-    __device__ __forceinline__ uint32_t read(uint32_t k) const { return k; }
-    __device__ __forceinline__ uint32_t write(uint32_t k) const { return k; }
-};
-
-// The last launch of a batch with such: a workgroup per bucket (read from side
-// 1, where the one scatter left it) or whole segment.  Bound by LDS round trips
-// and barriers as local_sort_items is (4096 segments log-uniform in [1, 2^16]:
-// 23 M pairs at ~150 keys a nanosecond, 2.4 TB/s), so buckets are of a size
-// that fits two workgroups on a CU: with 1024 threads and 11520 keys, one on a
-// CU, that batch took 371 us in all instead of 329, keys only 298 instead of
-// 239.
-template <int BLOCK, uint32_t TILE, bool PAY>
-__device__ __forceinline__ void slot_body(const mgpuSegSlotArgs& a) {
-    __shared__ mgpu::LocalShared<BLOCK, TILE, PAY> sh;
-    if (a.lsd_segments != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *a.lsd_segments = 0;
-    const uint32_t seg = a.slots[2 * blockIdx.x], bucket = a.slots[2 * blockIdx.x + 1];
-    const uint32_t moved = a.num_values > 1 ? MGPU_VALUES_MULTI : MGPU_VALUES_SINGLE;
-    SlotIO io{(ConstDesc)(a.segs + seg), 0u, 0u, a.result_side,
-              a.index_mode ? MGPU_VALUES_INDEX : moved, a.num_values};
-    uint32_t n, base = 0, bits = a.num_bits;
-    if (bucket == MGPU_SLOT_WHOLE) {
-        n = io.d->n;
-    } else {
-        io.d = (ConstDesc)(a.wide + seg);
-        if (io.d->route == 0) return;
-        const ConstWords at = (ConstWords)(a.digit_start + (size_t)seg * (MGPU_MAX_PASSES * MGPU_RADIX) +
-                                           MGPU_RADIX + 4 * bucket);
-        io.begin = at[0];
-        io.in = 1;
-        io.fill = moved;
-        n = at[1];
-        bits = at[2];
-        base = at[3];
-        if (n == 0) return;
-    }
-    if (n > TILE || io.begin > io.d->n || n > io.d->n - io.begin) {  // only from a broken plan
-        if (threadIdx.x == 0) mgpu::set_error(a.error_flag, 8u);
-        return;
-    }
-    mgpu::local_sort<PAY, BLOCK>(io, mgpu::local_mem(sh), n, base, a.first_bit, bits);
-}
-
 }  // namespace
 
 #define MGPU_SEG_SLOTS(B, TILE)                                                                \
     extern "C" __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(4)))    \
         mgpu_seg_slots_b##B##_k(mgpuSegSlotArgs a) {                                            \
-        slot_body<B, TILE, false>(a);                                                          \
+        __shared__ mgpu::LocalShared<B, TILE, false> sh;                                        \
+        mgpu::sort_slot<B, TILE, false>(a, mgpu::local_mem(sh), blockIdx.x);                    \
     }                                                                                          \
     extern "C" __global__ void __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(4)))    \
         mgpu_seg_slots_b##B##_kv(mgpuSegSlotArgs a) {                                           \
-        slot_body<B, TILE, true>(a);                                                           \
+        __shared__ mgpu::LocalShared<B, TILE, true> sh;                                         \
+        mgpu::sort_slot<B, TILE, true>(a, mgpu::local_mem(sh), blockIdx.x);                     \
     }
 MGPU_SEG_SLOTS(512, 8192)
 MGPU_SEG_SLOTS(1024, 16384)

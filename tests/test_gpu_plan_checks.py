@@ -35,7 +35,7 @@ class Desc(ctypes.Structure):  # mgpuSegDesc
 
 
 class SlotArgs(ctypes.Structure):  # mgpuSegSlotArgs
-    _fields_ = [("segs", P), ("wide", P), ("slots", P), ("digit_start", P), ("lsd_segments", P),
+    _fields_ = [("segs", P), ("wide", P), ("slots", P), ("digit_start", P),
                 ("num_values", U), ("index_mode", U), ("result_side", U), ("first_bit", U),
                 ("num_bits", U), ("pad", U), ("error_flag", P)]
 
@@ -90,7 +90,7 @@ def test_slots(threads, most, begin, past):
     code = 8 if past or begin == 1000 else 0
     keys = np.random.default_rng(n).integers(0, 1 << 32, n, dtype=np.uint32)
     sides = [to_dev(keys), to_dev(keys)]
-    flag, lsd = to_dev(np.zeros(1, np.uint32)), to_dev(np.ones(1, np.uint32))
+    flag = to_dev(np.zeros(1, np.uint32))
     d = Desc(n=n, route=1 << 31)
     for s in (0, 1):
         d.keys[s] = sides[s].data_ptr()
@@ -100,7 +100,7 @@ def test_slots(threads, most, begin, past):
     dev_starts = to_dev(starts)
     slots = to_dev(np.array([0, 0xFFFFFFFF if begin is None else 0], np.uint32))
     a = SlotArgs(segs=seg.data_ptr(), wide=seg.data_ptr(), slots=slots.data_ptr(),
-                 digit_start=dev_starts.data_ptr(), lsd_segments=lsd.data_ptr(),
+                 digit_start=dev_starts.data_ptr(),
                  result_side=1 if begin is None else 0, num_bits=32, error_flag=flag.data_ptr())
     _launch("mgpusort_seg.hsaco", f"mgpu_seg_slots_b{threads}_k", 1, threads, a)
     assert to_host(flag, 1)[0] == code
