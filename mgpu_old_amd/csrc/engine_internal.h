@@ -21,6 +21,12 @@ struct PassVariant {
     hipFunction_t xseg[4] = {};   // mgpu_rank_scatter_b*_i*_r*_x_v<mode>: a chain per XCD segment
     hipFunction_t multi[4] = {};  // mgpu_multi_scatter_b*_i*_r*_v<mode>
     hipFunction_t multiX[4] = {}; // mgpu_multi_scatter_b*_i*_r*_x_v<mode>: chains per XCD
+    // The passes of a bucketed batch (atomic-add ranking only): one chain a
+    // segment, and chains per XCD for those after the first (1024 x 16, no index
+    // form; null elsewhere).
+    hipFunction_t multiRouted[4] = {};
+    hipFunction_t multiRoutedX[4] = {};
+    uint32_t multiRoutedXGrid = 0;
     // The second pass of a bucketed batch, whose first workgroups sort its slots
     // (atomic-add ranking, 512 x 16, no index form; null elsewhere).
     hipFunction_t multiSlots[4] = {};

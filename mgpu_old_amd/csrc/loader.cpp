@@ -107,6 +107,15 @@ sortStatus_t load_variant(sortEngine_d* e, uint32_t threads, uint32_t items, uin
     }
     if (!v->mid[MGPU_VALUES_MULTI])
         for (int m = 0; m < 4; ++m) v->mid[m] = v->midPass[m] = nullptr;
+    for (int m = 0; m < 4 && rank == 1 && !st; ++m) {
+        char name[96];
+        std::snprintf(name, sizeof(name), "mgpu_multi_scatter_b%u_i%u_r1_r_v%d", threads, items, m);
+        st = get_fn(e, e->radixModule, name, &v->multiRouted[m]);
+        if (m == MGPU_VALUES_INDEX) continue;
+        std::snprintf(name, sizeof(name), "mgpu_multi_scatter_b%u_i%u_r1_xr_v%d", threads, items, m);
+        if (get_fn(e, e->radixModule, name, &v->multiRoutedX[m])) v->multiRoutedX[m] = nullptr;
+    }
+    if (st) return st;
     for (int m = 0; m < 4 && rank == 1; ++m) {
         char name[96];
         hipFunction_t f = nullptr;
@@ -153,6 +162,14 @@ sortStatus_t load_variant(sortEngine_d* e, uint32_t threads, uint32_t items, uin
         perCU < 1)
         perCU = 1;
     v->multiXGrid = (uint32_t)perCU * (uint32_t)e->numCUs;
+    if (v->multiRoutedX[MGPU_VALUES_SINGLE]) {
+        perCU = 0;
+        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(
+                &perCU, v->multiRoutedX[MGPU_VALUES_SINGLE], (int)threads, 0) != hipSuccess ||
+            perCU < 1)
+            perCU = 1;
+        v->multiRoutedXGrid = (uint32_t)perCU * (uint32_t)e->numCUs;
+    }
     if (v->packedX[MGPU_VALUES_SINGLE]) {
         perCU = 0;
         if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(

@@ -1351,8 +1351,9 @@ struct MidBucket {
 // to workgroups that run, so no number of resident workgroups is needed.  Data
 // goes between XCDs inside the launch: loads and stores are coherent ones.
 template <int BLOCK, int IPT, int RANK, int VMODE, bool MULTI, bool XSEG, bool EE, bool KMAP,
-          int MID, typename Args>
+          int MID, bool ROUTED, typename Args>
 __device__ void rank_scatter_body(const Args& a) {
+    static_assert(!ROUTED || (MULTI && RANK == 1), "passes of a bucketed batch");
     static_assert(MID == 0 || MID == 5 || (RANK == 1 && !MULTI && !XSEG && !EE),
                   "one array, one chain");
     static_assert(MID != 5 || (RANK == 1 && MULTI && !XSEG && BLOCK == MGPU_BUCKET_THREADS &&
@@ -1409,8 +1410,6 @@ __device__ void rank_scatter_body(const Args& a) {
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     uint32_t shift = a.shift, mask = a.mask;
     uint32_t width = (uint32_t)__builtin_popcount(mask);  // mask = 2^width - 1
-    // One tile per workgroup, of several arrays: passes of a bucketed batch.
-    constexpr bool ROUTED = MULTI && RANK == 1 && !XSEG;
     if constexpr (MID == 5) {
         if (blockIdx.x < a.num_slots) {
             mgpu::sort_slot<BLOCK, TILE, VMODE != MGPU_VALUES_NONE>(
@@ -1419,13 +1418,11 @@ __device__ void rank_scatter_body(const Args& a) {
         }
     }
     if constexpr (ROUTED) {
-        if (a.lsd_segments != nullptr) {
-            if (a.pass != 0) {
-                if (a.lsd_segments[1] == 0) return;
-            } else if (blockIdx.x == 0 && tid == 0) {
-                a.lsd_segments[1] = a.lsd_segments[0];
-                a.lsd_segments[0] = 0;
-            }
+        if (XSEG || a.pass != 0) {
+            if (a.lsd_segments[1] == 0) return;
+        } else if (blockIdx.x == 0 && tid == 0) {
+            a.lsd_segments[1] = a.lsd_segments[0];
+            a.lsd_segments[0] = 0;
         }
     }
     __shared__ uint32_t s_map[MID == 1 ? MGPU_MID_BINS : 1];  // bin (or digit) -> digit
@@ -1633,7 +1630,7 @@ __device__ void rank_scatter_body(const Args& a) {
             const uint32_t route =
                 ((const __attribute__((address_space(4))) mgpuSegDesc*)job.sd)->route;
             if (route != 0) {
-                if (a.pass != 0) return false;
+                if (XSEG || a.pass != 0) return false;
                 shift = route & 0xFFu;
                 width = (route >> 8) & 0xFFu;
                 mask = (1u << width) - 1u;
@@ -1643,6 +1640,20 @@ __device__ void rank_scatter_body(const Args& a) {
         return true;
     };
     uint32_t gtile;
+    // On to a tile that this pass takes (ROUTED with XSEG: the workgroup's next
+    // ones; one tile per workgroup: none).
+    auto skip_tiles = [&]() {
+        if constexpr (ROUTED && XSEG) {
+            do {
+                __syncthreads();  // (every wave has read the tile's number)
+                if (tid == 0) post_tile(take_tile());
+                __syncthreads();
+                gtile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
+            } while (gtile < seg_tiles && !start_tile(gtile));
+        } else {
+            gtile = seg_tiles;
+        }
+    };
     if constexpr (MID == 3) {
         gtile = take_item(job) ? 0u : seg_tiles;
     } else {
@@ -1652,7 +1663,7 @@ __device__ void rank_scatter_body(const Args& a) {
         // One tile per workgroup: only a counter left dirty finds none.
         if (!XSEG && gtile >= seg_tiles && tid == 0 && (MID != 1 || blockIdx.x < a.num_tiles))
             set_error(a.error_flag, 2u);
-        if (gtile < seg_tiles && !start_tile(gtile)) gtile = seg_tiles;
+        if (gtile < seg_tiles && !start_tile(gtile)) skip_tiles();
     }
     if constexpr (MID == 1)
     {
@@ -1967,7 +1978,7 @@ __device__ void rank_scatter_body(const Args& a) {
         if (tid == 0) post_tile(take_tile());
         __syncthreads();  // (every read of this tile's stage is done, too)
         gtile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile[0]);
-        if (gtile < seg_tiles) start_tile(gtile);
+        if (gtile < seg_tiles && !start_tile(gtile)) skip_tiles();
         clear_counts();  // (the value stage wrote over the match masks)
     }  // while
 
@@ -2433,29 +2444,43 @@ extern "C" __global__ void __launch_bounds__(256) mgpu_multi_scan(mgpuMultiScanA
 #define MGPU_RANK_SCATTER_MODE(B, I, R, V, MODE)                                             \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r##R##_v##V(mgpuPassArgs a) {                         \
-        rank_scatter_body<B, I, R, MODE, false, false, false, false, 0>(a);                      \
+        rank_scatter_body<B, I, R, MODE, false, false, false, false, 0, false>(a);                      \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r##R##_x_v##V(mgpuPassArgs a) {                       \
-        rank_scatter_body<B, I, R, MODE, false, true, false, false, 0>(a);                       \
+        rank_scatter_body<B, I, R, MODE, false, true, false, false, 0, false>(a);                       \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_multi_scatter_b##B##_i##I##_r##R##_v##V(mgpuMultiPassArgs a) {                   \
-        rank_scatter_body<B, I, R, MODE, true, false, false, false, 0>(a);                       \
+        rank_scatter_body<B, I, R, MODE, true, false, false, false, 0, false>(a);                       \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_multi_scatter_b##B##_i##I##_r##R##_x_v##V(mgpuMultiPassArgs a) {                 \
-        rank_scatter_body<B, I, R, MODE, true, true, false, false, 0>(a);                        \
+        rank_scatter_body<B, I, R, MODE, true, true, false, false, 0, false>(a);                        \
     }
+// Forms for the passes of a bucketed batch (atomic-add ranking only): a
+// segment's route read with its descriptor, and return at once when no segment
+// takes the pass.  With a chain per XCD for the passes after the first only,
+// whose field does not vary (it would cost them registers: 6 spilled).
+#define MGPU_RANK_SCATTER_ROUTED_MODE(B, I, FORM, XCDS, V, MODE)                              \
+    extern "C" __global__ void __launch_bounds__(B)                                           \
+        mgpu_multi_scatter_b##B##_i##I##_r1_##FORM##_v##V(mgpuMultiPassArgs a) {              \
+        rank_scatter_body<B, I, 1, MODE, true, XCDS, false, false, 0, true>(a);               \
+    }
+#define MGPU_RANK_SCATTER_ROUTED(B, I)                                                        \
+    MGPU_RANK_SCATTER_ROUTED_MODE(B, I, r, false, 0, MGPU_VALUES_NONE)                        \
+    MGPU_RANK_SCATTER_ROUTED_MODE(B, I, r, false, 1, MGPU_VALUES_INDEX)                       \
+    MGPU_RANK_SCATTER_ROUTED_MODE(B, I, r, false, 2, MGPU_VALUES_SINGLE)                      \
+    MGPU_RANK_SCATTER_ROUTED_MODE(B, I, r, false, 3, MGPU_VALUES_MULTI)
 // Early-exit forms (atomic-add ranking only): one chain, and a chain per XCD.
 #define MGPU_RANK_SCATTER_EE_MODE(B, I, V, MODE)                                              \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_ee_v##V(mgpuPassArgs a) {                          \
-        rank_scatter_body<B, I, 1, MODE, false, false, true, false, 0>(a);                       \
+        rank_scatter_body<B, I, 1, MODE, false, false, true, false, 0, false>(a);                       \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_x_ee_v##V(mgpuPassArgs a) {                        \
-        rank_scatter_body<B, I, 1, MODE, false, true, true, false, 0>(a);                        \
+        rank_scatter_body<B, I, 1, MODE, false, true, true, false, 0, false>(a);                        \
     }
 // Forms that map signed or float keys to their unsigned order as they read
 // them, or back as they write them (atomic-add ranking only): the first and
@@ -2463,11 +2488,11 @@ extern "C" __global__ void __launch_bounds__(256) mgpu_multi_scan(mgpuMultiScanA
 #define MGPU_RANK_SCATTER_KM_MODE(B, I, V, MODE)                                              \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_km_v##V(mgpuPassArgs a) {                          \
-        rank_scatter_body<B, I, 1, MODE, false, false, false, true, 0>(a);                       \
+        rank_scatter_body<B, I, 1, MODE, false, false, false, true, 0, false>(a);                       \
     }                                                                                         \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_x_km_v##V(mgpuPassArgs a) {                        \
-        rank_scatter_body<B, I, 1, MODE, false, true, false, true, 0>(a);                        \
+        rank_scatter_body<B, I, 1, MODE, false, true, false, true, 0, false>(a);                        \
     }
 #define MGPU_RANK_SCATTER_KM(B, I)                                                            \
     MGPU_RANK_SCATTER_KM_MODE(B, I, 0, MGPU_VALUES_NONE)                                      \
@@ -2518,7 +2543,7 @@ MGPU_RANK_SCATTER(1024, 16, 1)
 #define MGPU_RANK_SCATTER_MID_MODE(B, I, T, M, V, MODE)                                       \
     extern "C" __global__ void __launch_bounds__(B)                                           \
         mgpu_rank_scatter_b##B##_i##I##_r1_##T##_v##V(mgpuPassArgs a) {                       \
-        rank_scatter_body<B, I, 1, MODE, false, false, false, true, M>(a);                    \
+        rank_scatter_body<B, I, 1, MODE, false, false, false, true, M, false>(a);                    \
     }
 #define MGPU_RANK_SCATTER_MID(B, I)                                                           \
     MGPU_RANK_SCATTER_MID_MODE(B, I, m, 1, 0, MGPU_VALUES_NONE)                               \
@@ -2535,7 +2560,7 @@ MGPU_RANK_SCATTER_MID_MODE(1024, 16, l, 4, 3, MGPU_VALUES_MULTI)
 #define MGPU_MULTI_SLOTS(V, MODE)                                                             \
     extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) \
         mgpu_multi_scatter_slots_b512_i16_v##V(mgpuMultiPassArgs a) {                          \
-        rank_scatter_body<512, 16, 1, MODE, true, false, false, false, 5>(a);                 \
+        rank_scatter_body<512, 16, 1, MODE, true, false, false, false, 5, true>(a);                 \
     }
 MGPU_MULTI_SLOTS(0, MGPU_VALUES_NONE)
 MGPU_MULTI_SLOTS(2, MGPU_VALUES_SINGLE)
@@ -2545,6 +2570,12 @@ MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 2, MGPU_VALUES_SINGLE)
 MGPU_RANK_SCATTER_MID_MODE(512, 16, f, 3, 3, MGPU_VALUES_MULTI)
 MGPU_RANK_SCATTER_MID(512, 16)
 MGPU_RANK_SCATTER_MID(1024, 16)
+MGPU_RANK_SCATTER_ROUTED(256, 16)
+MGPU_RANK_SCATTER_ROUTED(512, 16)
+MGPU_RANK_SCATTER_ROUTED(1024, 16)
+MGPU_RANK_SCATTER_ROUTED_MODE(1024, 16, xr, true, 0, MGPU_VALUES_NONE)
+MGPU_RANK_SCATTER_ROUTED_MODE(1024, 16, xr, true, 2, MGPU_VALUES_SINGLE)
+MGPU_RANK_SCATTER_ROUTED_MODE(1024, 16, xr, true, 3, MGPU_VALUES_MULTI)
 MGPU_RANK_SCATTER_EE(512, 16)
 MGPU_RANK_SCATTER_EE(1024, 16)
 MGPU_RANK_SCATTER_KM(512, 16)

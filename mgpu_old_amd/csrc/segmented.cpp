@@ -529,7 +529,10 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
                 most = std::max(most, t);
             }
             const char* force = std::getenv("MGPUSORT_SEG_XCD");
-            bool use = !P.wideBuckets && most * 4 * X <= total && total >= kXcdMinTiles * P.wide.size();
+            // (Bucketed batches: for the passes after the first, which only
+            // segments that have no buckets take.)
+            bool use = most * 4 * X <= total && total >= kXcdMinTiles * P.wide.size() &&
+                       (!P.wideBuckets || P.wideVariant->multiRoutedX[MGPU_VALUES_NONE] != nullptr);
             if (force && (force[0] == '0' || force[0] == '1') && force[1] == 0)
                 use = force[0] == '1' && most * 4 * X <= total;
             if (use) {
@@ -881,7 +884,8 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
     const int carried = P.valueCount == -1 ? 1 : P.valueCount;
     for (uint32_t p = 0; p < np; ++p) {
         const bool slots = P.wideBuckets && p == 1;
-        const bool merged = slots && P.wideVariant->multiSlots[MGPU_VALUES_NONE] != nullptr;
+        const bool merged = slots && P.wideXcds == 1 &&
+                            P.wideVariant->multiSlots[MGPU_VALUES_NONE] != nullptr;
         if (slots && !merged) {
             st = mgpu_enqueue_slots(P, lane, lane.stream, false);
             if (st) return st;
@@ -915,30 +919,35 @@ sortStatus_t mgpu_enqueue_wide(SegPlanData& P, SortLane& lane) {
             pa.tile_begin = nullptr;
             pa.tile_seg = nullptr;
         }
-        if (P.wideXcds > 1) {
+        if (P.wideXcds > 1 && !(P.wideBuckets && p == 0)) {
             // Workgroups that loop over their XCD's tiles: as many as fit.
             pa.xcd_tile_begin = P.devXcdTileBegin;
             pa.num_xcds = P.wideXcds;
             pa.finished = lane.tileCounters + MGPU_FINISHED_SLOT + p;
-            const uint32_t fit =
-                P.widePacked ? P.wideVariant->packedXGrid : P.wideVariant->multiXGrid;
+            const uint32_t fit = P.widePacked    ? P.wideVariant->packedXGrid
+                                 : P.wideBuckets ? P.wideVariant->multiRoutedXGrid
+                                                 : P.wideVariant->multiXGrid;
             const uint32_t g = std::max(P.wideXcds, std::min(P.wideTiles, fit));
             st = mgpu_launch(e, lane.stream,
-                             P.widePacked ? P.wideVariant->packedX[mode] : P.wideVariant->multiX[mode],
+                             P.widePacked    ? P.wideVariant->packedX[mode]
+                             : P.wideBuckets ? P.wideVariant->multiRoutedX[mode]
+                                             : P.wideVariant->multiX[mode],
                              g, P.wideVariant->blockThreads, &pa);
         } else {
-            if (P.wideGroups > 1) {
+            const uint32_t groups = std::max(P.wideGroups, P.wideXcds);
+            if (groups > 1) {
                 pa.xcd_tile_begin = P.devXcdTileBegin;
-                pa.num_xcds = P.wideGroups;
+                pa.num_xcds = groups;
             }
             if (merged) {
                 pa.slot = slot_args(P, lane, false);
                 pa.num_slots = P.slots1024;
             }
             st = mgpu_launch(e, lane.stream,
-                             P.widePacked ? P.wideVariant->packed[mode]
-                             : merged     ? P.wideVariant->multiSlots[mode]
-                                          : P.wideVariant->multi[mode],
+                             P.widePacked    ? P.wideVariant->packed[mode]
+                             : merged        ? P.wideVariant->multiSlots[mode]
+                             : P.wideBuckets ? P.wideVariant->multiRouted[mode]
+                                             : P.wideVariant->multi[mode],
                              P.wideTiles + pa.num_slots, P.wideVariant->blockThreads, &pa);
         }
         if (st) return st;

@@ -63,9 +63,10 @@ SIZES = [16385, 20_000, 40_000, 70_001, 131_072, LONGEST, 5000, 300, 12_000]
 @pytest.mark.parametrize("kinds", [["even"], ["twothird"], ["sorted"], ["equal"], ["tiny"],
                                    ["even", "twothird"], ["narrow", "twothird", "equal", "sorted"]])
 @pytest.mark.parametrize("vc", [-1, 0, 1, 3])
-@pytest.mark.parametrize("repeat", [1, 4, 12])
+# (0: long ones only and many, so that whole segments are dealt to XCDs.)
+@pytest.mark.parametrize("repeat", [1, 4, 12, 0])
 def test_routes(engine, oracle, kinds, vc, repeat):
-    sizes = SIZES * repeat if repeat > 1 else SIZES[3:7]
+    sizes = SIZES * repeat if repeat > 1 else SIZES[3:7] if repeat else SIZES[2:6] * 20
     starts = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
     n = int(starts[-1])
     parts = [_keys(kinds[i % len(kinds)], s, seed=i) for i, s in enumerate(sizes)]
@@ -73,8 +74,14 @@ def test_routes(engine, oracle, kinds, vc, repeat):
     vals = [workloads.uniform_keys(n, seed=70 + j) for j in range(max(vc, 0))]
     g = GpuSort(keys, vals, value_count=vc)
     plan = engine.segmented_plan(g.data, starts)
+    engine.enable_timing(True)  # (the plan's launches one by one, by name)
+    engine.read_timing()
     plan.execute(g.data)
     engine.check_device()
+    names = set(engine.read_timing())
+    engine.enable_timing(False)
+    if engine.info()["xcdSegments"] > 1:
+        assert any("_xr_" in k for k in names) == (repeat == 0), names
     side1 = to_host(g.by_ptr[g.data.keys[1]], n)
     out, outs = g.keys(), g.values()
     wide = sum(s for s in sizes if s > WHOLE)
