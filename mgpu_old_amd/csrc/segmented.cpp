@@ -363,31 +363,45 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
     // Group segments by kernel variant; very large ones go device-wide.
     const uint32_t wideMin = device_wide_min(e), chunkKeys = wide_chunk(e);
     uint32_t keep = keep_in_workgroup(e), longestSeg = 0, numSmall = 0, numWhole = 0;
-    uint64_t longKeys = 0;  // in segments above a bucket's size
+    uint64_t longKeys = 0, wholeKeys = 0;  // in segments above a bucket's size, and above `keep`
     for (int i = 0; i < numSegments; ++i) {
-        longestSeg = std::max(longestSeg, segs[i].n);
-        if (segs[i].n < wideMin) ++numSmall;
-        else if (segs[i].n <= keep) ++numWhole;
-        if (segs[i].n > MGPU_BUCKET_KEYS) longKeys += segs[i].n;
+        const uint32_t n = segs[i].n;
+        longestSeg = std::max(longestSeg, n);
+        if (n != 0 && n < wideMin) ++numSmall;
+        else if (n != 0 && n <= keep) ++numWhole;
+        if (n > MGPU_BUCKET_KEYS) longKeys += n;
+        if (n > keep) wholeKeys += n;
     }
     const bool directCount = count_cols() && longestSeg <= kDirectCountMax &&
                              std::getenv("MGPUSORT_SEG_WIDE_CHUNK") == nullptr;
-    // A batch on one stream (the server's) runs its launches one after
-    // another, and a dozen workgroups' launch costs what a full one does:
-    // where there are buckets, the segments between a bucket's size and 16384
-    // keys go through them as well, and few small ones join the whole
-    // segments of the last launch.  Batches of 27 requests log-uniform in
+    // Beside device-wide passes, a launch that sorts no more whole segments than
+    // there are CUs costs what a full one does, and the passes would take those
+    // segments along for nothing.  So few of them
+    // * are sorted in one launch on the side stream where small ones are there
+    //   anyway and the passes are more than two (40 segments log-uniform in [1,
+    //   2^16], key + value, 97 -> 92 us);
+    // * else go through buckets above a bucket's size and are sorted with these
+    //   up to it, where there are buckets (20 in [4097, 40000] 63 us by passes
+    //   alone, 50 so, 96 with the two branches of a side stream in the graph);
+    // * else take the passes (300 in [1, 2^16] by 16 bits 82 us, 98 with a launch
+    //   on the side stream).
+    // A batch on one stream (the server's) has no side, and its few small
+    // segments join the buckets' launch as well: 27 requests log-uniform in
     // [2^10, 2^18] ran 14 and 25 us longer with a launch for each of the two.
-    bool smallInSlots = false;
-    if (lane.noSide && keep > MGPU_BUCKET_KEYS && directCount &&
-        use_buckets(e, P, pack_mode(e), longKeys)) {
-        keep = MGPU_BUCKET_KEYS;
-        smallInSlots = numSmall <= (uint32_t)e->numCUs;
+    const bool few = numWhole <= (uint32_t)e->numCUs;
+    bool smallInSlots = false, withBuckets = !few;
+    const uint64_t bucketedKeys = lane.noSide ? longKeys : wholeKeys;
+    const bool buckets = keep != 0 && directCount && use_buckets(e, P, pack_mode(e), bucketedKeys);
+    if (lane.noSide ? buckets && keep > MGPU_BUCKET_KEYS
+                    : buckets && few && (numSmall == 0 || P.sortPasses <= 2)) {
+        keep = std::min<uint32_t>(keep, MGPU_BUCKET_KEYS);
+        withBuckets = true;
+        smallInSlots = lane.noSide && numSmall <= (uint32_t)e->numCUs;
+    } else if (few && longestSeg > keep &&
+               (lane.noSide || numSmall == 0 || P.sortPasses <= 2)) {
+        keep = 0;
     }
     const bool noneAboveTile = longestSeg <= keep && seg_fits_tile(e, longestSeg);
-    // Beside the side stream: where the segments that a workgroup sorts whole
-    // are no more than the CUs, one launch sorts them all there.
-    const bool few = !lane.noSide && numWhole <= (uint32_t)e->numCUs;
     struct Group {
         std::vector<uint32_t> big, small;
     };
@@ -398,7 +412,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         if (n == 0 || P.numBits == 0) continue;
         if ((n >= wideMin && !noneAboveTile) || smallInSlots) {
             if (n <= keep) {
-                auto& list = n <= MGPU_BUCKET_KEYS && !few ? P.slots : slots1024;
+                auto& list = n <= MGPU_BUCKET_KEYS && withBuckets ? P.slots : slots1024;
                 list.push_back((uint32_t)i);
                 list.push_back(MGPU_SLOT_WHOLE);
             } else {
@@ -772,8 +786,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         if (st) return st;
     }
     // The side stream (before any capture) when there may be something to fork.
-    if (!lane.noSide && ((!P.launches.empty() && (!P.wide.empty() || !P.slots.empty())) ||
-                         (!P.wide.empty() && !P.slots.empty()))) {
+    if (!lane.noSide && !P.launches.empty() && (!P.wide.empty() || !P.slots.empty())) {
         sortStatus_t st = mgpu_lane_ensure_side(lane);
         if (st) return st;
     }
@@ -968,15 +981,14 @@ sortStatus_t mgpu_seg_enqueue(SegPlanData& P, SortLane& lane) {
     // each other, measured no faster: 4096 segments 0.614, 0.613, 0.619 ms
     // with one, two and three.  Forking after the device-wide count, so that
     // the count runs alone, was slower: 0.600 -> 0.639 ms.)
-    // Segments sorted whole by a workgroup each go beside the device-wide passes
-    // too (unless they share a launch with buckets).  After the passes they held
-    // a small batch up: 40 segments log-uniform in [1, 2^16], key + value, 107
-    // us, with one launch for all of those beside the passes 95.
+    // Segments sorted whole by a workgroup each go with them (unless they share
+    // a launch with buckets): after the passes they held a small batch up, 40
+    // segments log-uniform in [1, 2^16], key + value, 107 us, so 94.  Without
+    // device-wide passes, those of up to 8192 keys beside the others.
     const bool large = P.slots.size() / 2 > P.slots1024;
     const bool whole = P.slots1024 != 0 && !P.wideBuckets;
-    const bool fork = lane.side && !lane.noSide &&
-                      (P.wide.empty() ? !P.launches.empty() && (large || whole)
-                                      : !P.launches.empty() || large || whole);
+    const bool fork =
+        !P.launches.empty() && lane.side && !lane.noSide && (!P.wide.empty() || whole);
     hipStream_t ls = lane.stream;
     if (fork) {
         if (hipEventRecord(lane.fork, lane.stream) != hipSuccess ||
