@@ -7,9 +7,10 @@ creation (kernelPath + "mgpusort_seg_tuning.txt"):
      with every segment kept in the persistent kernel;
   2. the device-wide passes, on the batch they serve (4096 segments with
      sizes log-uniform in [1, 2^16], key + one value): the size from which a
-     segment takes them, the tile shape and whether tiles are packed
-     (segments back to back) or one segment's own, timed with the bucket
-     rows of step 1 in force (the count piece size only matters for segments
+     segment takes them, the tile shape, whether tiles are packed (segments
+     back to back) or one segment's own, and the keys up to which a workgroup
+     sorts a segment whole instead, timed with the bucket rows of step 1 in
+     force (the count piece size only matters for segments
      above 2^18 keys, which this batch does not have: it stays at 2^16, the
      better of 2^14 and 2^16 on the sort server's batches);
   3. on the same batch, for each threshold of step 2, one variant for every
@@ -49,6 +50,13 @@ WIDE_CHUNK = [1 << 16]
 # Gkeys/s); "large" is the alternative measured here.
 WIDE_TILE = ["auto", "large"]
 WIDE_PACK = ["packed", "unpacked"]
+WIDE_KEEP = [0, 8192, 16384]  # 0: none above the persistent kernels' threshold
+
+
+def wide_lines():
+    """The candidates of the table's wide row."""
+    return [f"wide {m} {c} {t} {pk} {keep}" for m in WIDE_MIN for c in WIDE_CHUNK
+            for t in WIDE_TILE for pk in WIDE_PACK for keep in WIDE_KEEP]
 
 
 def bucket_sizes(lo, hi, total, seed):
@@ -157,16 +165,11 @@ def main():
         keys = workloads.uniform_keys_torch(n, 44, "cuda", torch=torch)
         vals = torch.arange(n, dtype=torch.int32, device="cuda")
         wide = {}
-        for m in WIDE_MIN:
-            for c in WIDE_CHUNK:
-                for t in WIDE_TILE:
-                    for pk in WIDE_PACK:
-                        line = f"wide {m} {c} {t} {pk} 16384"
-                        eng = engine_on(torch, tmp, bucket_text + line + "\n")
-                        wide[line] = time_plan(torch, eng, keys, vals, starts, args.reps)
-                        eng.close()
-                        print(f"[tune] 4096 segments ({n} keys) {line}: {wide[line] * 1e3:.3f} ms",
-                              flush=True)
+        for line in wide_lines():
+            eng = engine_on(torch, tmp, bucket_text + line + "\n")
+            wide[line] = time_plan(torch, eng, keys, vals, starts, args.reps)
+            eng.close()
+            print(f"[tune] 4096 segments ({n} keys) {line}: {wide[line] * 1e3:.3f} ms", flush=True)
         best_wide = min(wide, key=wide.get)
         report["wide"] = {"best": best_wide, "keys": n, "ms": {k: t * 1e3 for k, t in wide.items()}}
 

@@ -8,21 +8,27 @@ It plays the role of the reference's pass tables (sort/src/mgpusort/
 sorttables.cpp:16-1465, generated offline by sort/src/tablegen/tablegen.cpp:
 9-64 from measured rates), but times every candidate directly on the GPU.
 A candidate replaces the engine's built-in choice only when it is faster by
-more than --margin, so timing noise does not flip choices.
+more than --margin, so timing noise does not flip choices.  A candidate is
+asked for by a table of its own, as the one written here asks for it: sorts
+that take other routes at a size (one workgroup, buckets) are timed on those.
 
 Usage (on a gfx950 box):  python -m mgpu_old_amd.tune_sort [--out PATH]
 """
 import argparse
 import json
 import os
+import shutil
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CLASSES = {"keys": 0, "index": -1, "kv": 1, "multi": 2}  # value class -> valueCount
-CANDIDATES = {("small", "one"): {"MGPUSORT_TILE": "512x16", "MGPUSORT_XCD": "0"},
-              ("large", "one"): {"MGPUSORT_TILE": "1024x16", "MGPUSORT_XCD": "0"},
-              ("small", "xcd"): {"MGPUSORT_TILE": "512x16", "MGPUSORT_XCD": "1"},
-              ("large", "xcd"): {"MGPUSORT_TILE": "1024x16", "MGPUSORT_XCD": "1"}}
+CANDIDATES = [(tile, chains) for chains in ("one", "xcd") for tile in ("small", "large")]
+
+
+def candidate_table(tile, chains):
+    """The table that asks for one choice at every size."""
+    return "".join(f"31 {cls} {tile} {chains}\n" for cls in CLASSES)
 
 
 def choose(times, builtin, margin):
@@ -45,17 +51,16 @@ def table_rows(choices):
     return rows
 
 
-def make_engine(mg, torch, env):
-    saved = {k: os.environ.get(k) for k in env}
-    os.environ.update(env)
-    try:
-        eng = mg.Engine()
-    finally:
-        for k, v in saved.items():
-            if v is None:
-                os.environ.pop(k, None)
-            else:
-                os.environ[k] = v
+def make_engine(mg, torch, dirpath, table):
+    """An engine over a copy of the code objects in `dirpath` with this table
+    (None: none, the built-in rules)."""
+    os.makedirs(dirpath, exist_ok=True)
+    for name in ("mgpusort_radix.hsaco", "mgpusort_seg.hsaco"):
+        shutil.copy(os.path.join(mg.LIB_DIR, name), os.path.join(dirpath, name))
+    if table is not None:
+        with open(os.path.join(dirpath, "mgpusort_sort_tuning.txt"), "w") as f:
+            f.write(table)
+    eng = mg.Engine(dirpath + os.sep)
     eng.set_stream(torch.cuda.current_stream().cuda_stream)
     return eng
 
@@ -114,11 +119,14 @@ def main():
     import mgpu_old_amd as mg
     from mgpu_old_amd import workloads
 
-    # The table being written must not steer the measurement.
-    if os.path.exists(args.out):
-        os.remove(args.out)
-    engines = {c: make_engine(mg, torch, env) for c, env in CANDIDATES.items()}
-    engines["builtin"] = make_engine(mg, torch, {})
+    # (In folders of their own: the table being written steers none of them.)
+    tmp = tempfile.mkdtemp(prefix="sorttune")
+    try:
+        engines = {c: make_engine(mg, torch, os.path.join(tmp, "_".join(c)), candidate_table(*c))
+                   for c in CANDIDATES}
+        engines["builtin"] = make_engine(mg, torch, os.path.join(tmp, "builtin"), None)
+    finally:
+        shutil.rmtree(tmp, ignore_errors=True)  # (the engines have loaded what they need)
     choices = {cls: [] for cls in CLASSES}
     report = {}
     for lg in range(args.min_log2, args.max_log2 + 1):
