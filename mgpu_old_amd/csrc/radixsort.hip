@@ -1959,15 +1959,23 @@ __device__ void rank_scatter_body(const Args& a) {
         if constexpr (VMODE == MGPU_VALUES_MULTI) {
             for (uint32_t v = 0; v < a.num_values; ++v) {
                 load_striped<IPT, LAUX>(vals_in(job, v), n, wave_base, lane, val);
-                const __amdgpu_buffer_rsrc_t ro = array_rsrc(vals_out(job, v), n);
+                uint32_t* const dstv = vals_out(job, v);
+                const __amdgpu_buffer_rsrc_t ro = array_rsrc(dstv, n);
                 __syncthreads();
 #pragma unroll
                 for (int j = 0; j < IPT; ++j) s_stage[pos[j]] = val[j];
                 __syncthreads();
 #pragma unroll
-                for (int i = 0; i < IPT; ++i)
-                    __builtin_amdgcn_raw_buffer_store_b32(s_stage[i * BLOCK + tid], ro,
-                                                          (int)(dest[i] * 4u), 0, SAUX);
+                for (int i = 0; i < IPT; ++i) {
+                    // (Several arrays with a chain per XCD, two values: with a
+                    // branch a slot 64 segments in [2^18, 2^20] 1115 us, range
+                    // checked 1082; one array the other way round, 2^24 keys 467
+                    // and 478.)
+                    if constexpr (MULTI || MID == 3)
+                        __builtin_amdgcn_raw_buffer_store_b32(s_stage[i * BLOCK + tid], ro,
+                                                              (int)(dest[i] * 4u), 0, SAUX);
+                    else if (dest[i] < n) dstv[dest[i]] = s_stage[i * BLOCK + tid];
+                }
             }
         }
 
