@@ -1091,7 +1091,8 @@ __device__ __forceinline__ void load_striped(const uint32_t* src, uint32_t n, ui
 // 35.0, 900001 68.8 -> 42.1, 3145728 96.1 -> 68.5; normal floats 150000
 // 53.3 -> 42.5.  Keys that no grouping spreads (low-entropy pairs), digit passes
 // -> the same behind these counts: 65536 56.6 -> 50.4 us, 400001 66.7 -> 60.9,
-// 1391168 94.0 -> 93.0, 2500001 103.2 -> 103.8, 3145728 107.8 -> 109.1.
+// 1391168 94.0 -> 92.5, 2500001 103.2 -> 103.2, 3145728 107.8 -> 108.5 (by 24
+// bits 86.9 -> 88.1).
 //
 // The digits of a bucketed sort's first scatter, worked out by every workgroup
 // from the counts while its keys load (1024 bins: a few KB from the L2 and a
@@ -1712,16 +1713,16 @@ __device__ void rank_scatter_body(const Args& a) {
         }
         uint32_t dig[MID == 1 ? IPT : 1];
         if constexpr (MID == 1) {
-#pragma unroll
-            for (int j = 0; j < IPT; ++j) dig[j] = __builtin_amdgcn_ubfe(key[j], shift, width);
             if (mapped) {
 #pragma unroll
-                for (int j = 0; j < IPT; ++j) dig[j] = s_map[dig[j]];
+                for (int j = 0; j < IPT; ++j)
+                    dig[j] = s_map[__builtin_amdgcn_ubfe(key[j], shift, width)];
             }
         }
         auto digit_of = [&](int j) -> uint32_t {
-            if constexpr (MID == 1) return dig[j];
-            else return __builtin_amdgcn_ubfe(key[j], shift, width);
+            const uint32_t d = __builtin_amdgcn_ubfe(key[j], shift, width);
+            if constexpr (MID == 1) return mapped ? dig[j] : d;
+            else return d;
         };
 
         // Rank within the wave: pos[j] = earlier same-digit keys of this wave.
