@@ -360,7 +360,7 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
         la.error_flag = L.errorDev;
         return la;
     };
-    hipFunction_t localFn = valueCount ? e->fnLocalPay : e->fnLocal;
+    hipFunction_t localFn = valueCount == 0 ? e->fnLocal : valueCount > 1 ? e->fnLocalMany : e->fnLocalPay;
     if (n <= kLocalSortMaxKeys && localFn && !earlyExit) {
         mgpuLocalArgs la = local_args(0);
         la.in_lo = toLo;
@@ -487,7 +487,9 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
                                                              : 0u;
             return mgpu_launch(e, L.stream, f, grid, var.blockThreads, &pa, timed);
         };
-        st = pass(0, var.mid[firstMode], numTiles + 1);  // one for the plan
+        // (In tiles of a workgroup's sort, one more for the plan and the later
+        // passes' digit starts.)
+        st = pass(0, var.mid[firstMode], numTiles + (tile == MGPU_LOCAL_MAX_KEYS ? 1u : 0u));
         if (st) return st;
         int next = 1;
         if (merged) {
@@ -496,6 +498,9 @@ sortStatus_t mgpu_sort_passes(sortEngine_d* e, SortLane& L, uint32_t n, int firs
             mgpuLocalArgs la = local_args(1);
             la.plan = L.midPlan;
             la.hist = L.hist;
+            la.starts = L.digitStart;
+            la.num_passes = (uint32_t)numPasses;
+            la.last_width = (uint32_t)widths[numPasses - 1];
             st = mgpu_launch(e, L.stream, localFn, MGPU_RADIX, MGPU_LOCAL_THREADS, &la, timed);
         }
         if (st) return st;

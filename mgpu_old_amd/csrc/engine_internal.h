@@ -138,12 +138,14 @@ struct sortEngine_d {
     hipFunction_t fnCountKM = nullptr;    // the two over signed or float keys
     hipFunction_t fnCountColsKM = nullptr;
     hipFunction_t fnScan = nullptr;
-    // One workgroup, every pass in LDS: keys only, and with a payload.  Null
+    // One workgroup, every pass in LDS: keys only, with a payload, and with
+    // several values.  Null
     // where the atomic-add ranking is off, or where a tile shape or a chain
     // per XCD was asked for by name (the device-wide passes then run at every
     // size).
     hipFunction_t fnLocal = nullptr;
     hipFunction_t fnLocalPay = nullptr;
+    hipFunction_t fnLocalMany = nullptr;
     hipFunction_t fnSegSlots[2][2] = {};  // [512, 1024 threads][values]: buckets and segments
     hipFunction_t fnMidCount = nullptr;  // counts of a bucketed sort (null as above)
     hipFunction_t fnIota = nullptr;

@@ -400,7 +400,7 @@ struct mgpuPassArgs {
     mgpuMidPlan* mid_plan;
     uint32_t* mid_hist;
     uint32_t* mid_starts;         // [MGPU_MAX_PASSES][MGPU_RADIX]: digit starts of the passes after
-                                  // the first scatter, which writes them
+                                  // the first scatter
     uint32_t mid_shift;           // of the bins
     uint32_t mid_target;
     uint32_t mid_passes;
@@ -427,9 +427,13 @@ struct mgpuLocalArgs {
     uint32_t in_lo, in_hi, out_lo, out_hi;
     uint32_t pad_;
     // Bucketed sort: workgroup b sorts bucket b of the plan (nothing when the
-    // plan does not use buckets), and the first one zeroes mid_count's histogram.
+    // plan does not use buckets), and workgroup p < num_passes makes pass p's
+    // digit starts of mid_count's histogram and zeroes it.
     const mgpuMidPlan* plan;
     uint32_t* hist;
+    uint32_t* starts;        // [MGPU_MAX_PASSES][MGPU_RADIX]
+    uint32_t num_passes;
+    uint32_t last_width;     // of the last pass's digit
     uint32_t* error_flag;
 };
 

@@ -317,6 +317,7 @@ sortStatus_t mgpu_engine_load(sortEngine_d* e) {
     if (e->rankMethod == 1 && !e->xcdForce && !(t && *t)) {
         st = get_fn(e, e->radixModule, "mgpu_local_sort_k", &e->fnLocal);
         if (!st) st = get_fn(e, e->radixModule, "mgpu_local_sort_kv", &e->fnLocalPay);
+        if (!st) st = get_fn(e, e->radixModule, "mgpu_local_sort_kvs", &e->fnLocalMany);
         if (!st) st = get_fn(e, e->radixModule, "mgpu_mid_count", &e->fnMidCount);
         if (st) return st;
     }

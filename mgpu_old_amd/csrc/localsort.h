@@ -66,8 +66,9 @@ struct LocalArrays {
 // Sorts the n elements of `io`, 0 < n <= IT * BLOCK, by bits [shift0, shift0 +
 // bits) of (key - base).  IT keys per thread: wave w holds keys w * 64 * IT +
 // j * 64 + lane.  Slots past n hold all ones in every digit, so they stay
-// behind every key.
-template <int BLOCK, int IT, bool PAY, typename IO>
+// behind every key.  MANY: whether io carries two or more values (-1: io.mode()
+// says so).
+template <int BLOCK, int IT, bool PAY, int MANY = -1, typename IO>
 __device__ __forceinline__ void local_sort_items(const IO& io, const LocalMem& sh, uint32_t n, uint32_t base,
                                  uint32_t shift0, uint32_t bits) {
     constexpr uint32_t G = BLOCK / MGPU_RADIX;  // threads per digit in the scan
@@ -85,7 +86,7 @@ __device__ __forceinline__ void local_sort_items(const IO& io, const LocalMem& s
         for (int j = 0; j < IT; ++j)
             key[j] = __builtin_amdgcn_raw_buffer_load_b32(rk, (int)(off + j * 256u), 0, 0);
         if constexpr (PAY) {
-            if (fill == MGPU_VALUES_SINGLE) {
+            if (MANY != 1 && fill == MGPU_VALUES_SINGLE) {
                 const __amdgpu_buffer_rsrc_t rv = words_rsrc(io.vals_in(0), n);
 #pragma unroll
                 for (int j = 0; j < IT; ++j)
@@ -156,12 +157,12 @@ __device__ __forceinline__ void local_sort_items(const IO& io, const LocalMem& s
                                                   (int)(off + j * 256u), 0, 0);
     }
     if constexpr (PAY) {
-        if (fill != MGPU_VALUES_MULTI) {
+        if (MANY == 0 || (MANY < 0 && fill != MGPU_VALUES_MULTI)) {
             const __amdgpu_buffer_rsrc_t rv = words_rsrc(io.vals_out(0), n);
 #pragma unroll
             for (int j = 0; j < IT; ++j)
                 __builtin_amdgcn_raw_buffer_store_b32(pay[j], rv, (int)(off + j * 256u), 0, 0);
-        } else {
+        } else if constexpr (MANY != 0) {
             // Two or more arrays, each through a stage in LDS: read in order,
             // taken in the keys' order, written in order, so that every global
             // access is whole lines.  Against a gather from global memory through
@@ -200,15 +201,15 @@ __device__ __forceinline__ void local_sort_items(const IO& io, const LocalMem& s
 }
 
 // The same with the least IT that holds n <= 16 * B elements.
-template <bool PAY, int B = kLocalBlock, typename IO>
+template <bool PAY, int B = kLocalBlock, int MANY = -1, typename IO>
 __device__ __forceinline__ void local_sort(const IO& io, const LocalMem& sh, uint32_t n,
                                            uint32_t base, uint32_t shift, uint32_t bits) {
-    if (n <= 1 * B) local_sort_items<B, 1, PAY>(io, sh, n, base, shift, bits);
-    else if (n <= 2 * B) local_sort_items<B, 2, PAY>(io, sh, n, base, shift, bits);
-    else if (n <= 4 * B) local_sort_items<B, 4, PAY>(io, sh, n, base, shift, bits);
-    else if (n <= 8 * B) local_sort_items<B, 8, PAY>(io, sh, n, base, shift, bits);
-    else if (n <= 12 * B) local_sort_items<B, 12, PAY>(io, sh, n, base, shift, bits);
-    else local_sort_items<B, 16, PAY>(io, sh, n, base, shift, bits);
+    if (n <= 1 * B) local_sort_items<B, 1, PAY, MANY>(io, sh, n, base, shift, bits);
+    else if (n <= 2 * B) local_sort_items<B, 2, PAY, MANY>(io, sh, n, base, shift, bits);
+    else if (n <= 4 * B) local_sort_items<B, 4, PAY, MANY>(io, sh, n, base, shift, bits);
+    else if (n <= 8 * B) local_sort_items<B, 8, PAY, MANY>(io, sh, n, base, shift, bits);
+    else if (n <= 12 * B) local_sort_items<B, 12, PAY, MANY>(io, sh, n, base, shift, bits);
+    else local_sort_items<B, 16, PAY, MANY>(io, sh, n, base, shift, bits);
 }
 
 // A segment's descriptor does not change while a kernel that sorts it runs, so

@@ -1122,7 +1122,8 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
     static_assert(LANES == 2 || LANES == 4, "a group of bins is held by neighbouring lanes");
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const bool writes = blockIdx.x == a.num_tiles;  // the workgroup without a tile
+    // The writer: the last workgroup, which has no tile where OWN.
+    const bool writes = blockIdx.x + 1 == gridDim.x;
     const uint32_t field_shift = a.mid_field[0] & 0xFFu;
     auto put_plan = [&](uint32_t b, uint32_t start, uint32_t base, uint32_t bits) {
         a.mid_plan->start[b] = start;
@@ -1295,19 +1296,28 @@ __device__ bool mid_plan_tile(const mgpuPassArgs& a, const uint32_t (&c)[MGPU_MI
 // without a tile: the last digits are the bins' top bits.
 template <int BLOCK>
 __device__ void mid_later_starts(const mgpuPassArgs& a, uint32_t* s_tmp) {
+    constexpr int LATER = MGPU_MAX_PASSES - 1;
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    for (uint32_t p = 1; p < a.mid_passes; ++p) {
-        const uint32_t width = a.mid_field[p] >> 8;
-        uint32_t c = 0;
+    uint32_t c[LATER];
+#pragma unroll
+    for (int q = 0; q < LATER; ++q) {
+        const uint32_t p = (uint32_t)q + 1;
+        c[q] = 0;
         if (p + 1 < a.mid_passes) {
-            if (tid < RADIX) c = a.mid_hist[MGPU_MID_BINS + p * RADIX + tid];
-        } else if (tid < 1u << width) {
-            const uint32_t per = MGPU_MID_BINS >> width;
-            for (uint32_t i = 0; i < per; ++i) c += a.mid_hist[tid * per + i];
+            if (tid < RADIX) c[q] = a.mid_hist[MGPU_MID_BINS + p * RADIX + tid];
+        } else if (p + 1 == a.mid_passes) {
+            const uint32_t width = a.mid_field[p] >> 8, per = MGPU_MID_BINS >> width;
+            if (tid < 1u << width)
+                for (uint32_t i = 0; i < per; ++i) c[q] += a.mid_hist[tid * per + i];
         }
-        __syncthreads();  // (s_tmp was read)
-        const uint32_t start = mgpu::block_exclusive_scan_dpp<BLOCK>(c, s_tmp, lane, wave);
+    }
+#pragma unroll
+    for (int q = 0; q < LATER; ++q) {
+        const uint32_t p = (uint32_t)q + 1;
+        if (p >= a.mid_passes) break;
+        if (q > 0) __syncthreads();  // (s_tmp was read)
+        const uint32_t start = mgpu::block_exclusive_scan_dpp<BLOCK>(c[q], s_tmp, lane, wave);
         if (tid < RADIX) a.mid_starts[p * RADIX + tid] = start;
     }
 }
@@ -1376,6 +1386,11 @@ __device__ void rank_scatter_body(const Args& a) {
     if constexpr (MID == 2 || MID == 3) {
         if (a.mid_plan->buckets) return;
     }
+    // The first scatter where the launch after it makes passes (MID 4): a
+    // workgroup more writes the plan and the later passes' digit starts, which
+    // mgpu_local_sort makes otherwise (below 2^19 keys the launch took 0.7 us
+    // longer with it: 20001 keys 21.7 and 22.9 us a sort).
+    constexpr bool MID_OWN = MID == 1 && BLOCK * IPT == MGPU_LOCAL_MAX_KEYS;
     constexpr int LAUX = MID == 3 ? kCoherentAux : kTileLoadAux;
     constexpr int SAUX = MID == 3 ? kCoherentAux : 0;
     static_assert(!EE || RANK == 1, "early exit builds on the atomic-add ranking");
@@ -1453,9 +1468,9 @@ __device__ void rank_scatter_body(const Args& a) {
                 return;
             }
             const mgpu::LocalMem mem{&s_count[0][0], s_tmp, s_stage, s_aux};
-            mgpu::local_sort<VMODE != MGPU_VALUES_NONE>(MidBucket<VMODE>{a, begin}, mem, n,
-                                                        plan.base[blockIdx.x], a.mid_field[0] & 0xFFu,
-                                                        plan.bits[blockIdx.x]);
+            mgpu::local_sort<VMODE != MGPU_VALUES_NONE, mgpu::kLocalBlock, VMODE == MGPU_VALUES_MULTI>(
+                MidBucket<VMODE>{a, begin}, mem, n, plan.base[blockIdx.x], a.mid_field[0] & 0xFFu,
+                plan.bits[blockIdx.x]);
             return;
         }
         if (blockIdx.x >= a.num_tiles) return;
@@ -1532,7 +1547,7 @@ __device__ void rank_scatter_body(const Args& a) {
     auto take_tile = [&]() {
         uint32_t t = seg_tiles;  // a workgroup of an XCD without a segment takes none
         if constexpr (MID == 1)
-            if (blockIdx.x == a.num_tiles) return t;
+            if (MID_OWN && blockIdx.x == a.num_tiles) return t;
         bool grouped = false;
         if constexpr (MULTI && !XSEG) grouped = a.num_xcds > 1;
         if (grouped) {
@@ -1678,11 +1693,10 @@ __device__ void rank_scatter_body(const Args& a) {
             set_error(a.error_flag, 2u);
         if (gtile < seg_tiles && !start_tile(gtile)) skip_tiles();
     }
-    if constexpr (MID == 1)
-    {
+    if constexpr (MID == 1) {
         mapped = mid_plan_tile<BLOCK>(a, mid_bins, mid_digit0, s_map, s_global, s_tmp, s_stage, shift, width,
                              mask);
-        if (blockIdx.x == a.num_tiles) {
+        if (MID_OWN && blockIdx.x == a.num_tiles) {
             mid_later_starts<BLOCK>(a, s_tmp);
             return;
         }
@@ -2603,19 +2617,38 @@ MGPU_PACKED(512, 16)
 MGPU_PACKED(1024, 16)
 
 // One workgroup sorts a small array, or a bucket of a mid-sized one, through
-// every pass: keys only, or with a payload (a value, a generated index, or the
-// source index of several values).
-template <bool PAY>
+// every pass: keys only, with a payload (a value or a generated index), or with
+// the source index of several values (a kernel of its own: the registers of
+// that part cost the other 0.7 us at 16 keys per thread).
+template <bool PAY, int MANY>
 __device__ __forceinline__ void local_sort_array(const mgpuLocalArgs& a) {
     __shared__ mgpu::LocalShared<mgpu::kLocalBlock, mgpu::kLocalTile, PAY> sh;
     if (!a.plan) {
-        mgpu::local_sort<PAY>(mgpu::LocalArrays{a, 0u}, local_mem(sh), a.n, 0u, a.first_bit,
-                              a.num_bits);
+        mgpu::local_sort<PAY, mgpu::kLocalBlock, MANY>(mgpu::LocalArrays{a, 0u}, local_mem(sh), a.n, 0u,
+                                                       a.first_bit, a.num_bits);
         return;
     }
+    // The counts go back to zero; when the digit passes go on, workgroup p first
+    // makes pass p's digit starts of them (the last digits are the bins' top
+    // bits).
     const uint32_t b = blockIdx.x;
-    if (b == 0)
-        for (uint32_t i = threadIdx.x; i < MGPU_MID_HIST_WORDS; i += MGPU_LOCAL_THREADS) a.hist[i] = 0;
+    if (b < a.num_passes) {
+        const uint32_t tid = threadIdx.x, first = b + 1 == a.num_passes ? 0u : MGPU_MID_BINS + b * RADIX;
+        uint32_t* const h = a.hist + first;
+        uint32_t cnt = 0;
+        if (first == 0) {
+            const uint32_t per = MGPU_MID_BINS >> a.last_width;
+            if (tid < (1u << a.last_width))
+                for (uint32_t i = 0; i < per; ++i) cnt += h[tid * per + i];
+        } else if (tid < RADIX) {
+            cnt = h[tid];
+        }
+        const uint32_t st = mgpu::block_exclusive_scan_dpp<MGPU_LOCAL_THREADS>(
+            cnt, sh.tmp, tid & 63, (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)));
+        if (tid < RADIX) a.starts[b * RADIX + tid] = st;
+        __syncthreads();
+        if (first == 0 || tid < RADIX) h[tid] = 0;
+    }
     if (!a.plan->buckets) return;
     const uint32_t begin = a.plan->start[b], n = a.plan->start[b + 1] - begin;
     if (n == 0) return;
@@ -2623,16 +2656,20 @@ __device__ __forceinline__ void local_sort_array(const mgpuLocalArgs& a) {
         if (threadIdx.x == 0) set_error(a.error_flag, 8u);
         return;
     }
-    mgpu::local_sort<PAY>(mgpu::LocalArrays{a, begin}, local_mem(sh), n, a.plan->base[b],
-                          a.first_bit, a.plan->bits[b]);
+    mgpu::local_sort<PAY, mgpu::kLocalBlock, MANY>(mgpu::LocalArrays{a, begin}, local_mem(sh), n,
+                                                   a.plan->base[b], a.first_bit, a.plan->bits[b]);
 }
 
 extern "C" __global__ void __launch_bounds__(MGPU_LOCAL_THREADS) mgpu_local_sort_k(mgpuLocalArgs a) {
-    local_sort_array<false>(a);
+    local_sort_array<false, 0>(a);
 }
 
 extern "C" __global__ void __launch_bounds__(MGPU_LOCAL_THREADS) mgpu_local_sort_kv(mgpuLocalArgs a) {
-    local_sort_array<true>(a);
+    local_sort_array<true, 0>(a);
+}
+
+extern "C" __global__ void __launch_bounds__(MGPU_LOCAL_THREADS) mgpu_local_sort_kvs(mgpuLocalArgs a) {
+    local_sort_array<true, 1>(a);
 }
 
 // Check of the ordering RANK 1 relies on: wave w of one 1024-thread

@@ -22,7 +22,8 @@ class LocalArgs(ctypes.Structure):  # mgpuLocalArgs
     _fields_ = [("keys_in", P), ("keys_out", P), ("vals_in", P * 6), ("vals_out", P * 6),
                 ("n", U), ("first_bit", U), ("num_bits", U), ("vals_mode", U), ("num_values", U),
                 ("in_lo", U), ("in_hi", U), ("out_lo", U), ("out_hi", U), ("pad", U),
-                ("plan", P), ("hist", P), ("error_flag", P)]
+                ("plan", P), ("hist", P), ("starts", P), ("num_passes", U), ("last_width", U),
+                ("error_flag", P)]
 
 
 class Plan(ctypes.Structure):  # mgpuMidPlan
@@ -72,7 +73,8 @@ def test_bucket_of_an_array(begin, size, n, code):
         plan.bits[b] = 32
     dev_plan, scratch = _dev(plan), empty_dev(4096)
     a = LocalArgs(keys_in=src.data_ptr(), keys_out=out.data_ptr(), n=n, num_bits=32,
-                  plan=dev_plan.data_ptr(), hist=scratch.data_ptr(), error_flag=flag.data_ptr())
+                  plan=dev_plan.data_ptr(), hist=scratch.data_ptr(), starts=scratch.data_ptr(),
+                  num_passes=0, last_width=8, error_flag=flag.data_ptr())
     _launch("mgpusort_radix.hsaco", "mgpu_local_sort_k", 256, 1024, a)
     assert to_host(flag, 1)[0] == code
     want = keys.copy()
