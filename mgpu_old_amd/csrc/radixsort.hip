@@ -2623,41 +2623,43 @@ MGPU_PACKED(1024, 16)
 template <bool PAY, int MANY>
 __device__ __forceinline__ void local_sort_array(const mgpuLocalArgs& a) {
     __shared__ mgpu::LocalShared<mgpu::kLocalBlock, mgpu::kLocalTile, PAY> sh;
-    if (!a.plan) {
-        mgpu::local_sort<PAY, mgpu::kLocalBlock, MANY>(mgpu::LocalArrays{a, 0u}, local_mem(sh), a.n, 0u,
-                                                       a.first_bit, a.num_bits);
-        return;
-    }
-    // The counts go back to zero; when the digit passes go on, workgroup p first
-    // makes pass p's digit starts of them (the last digits are the bins' top
-    // bits).
-    const uint32_t b = blockIdx.x;
-    if (b < a.num_passes) {
-        const uint32_t tid = threadIdx.x, first = b + 1 == a.num_passes ? 0u : MGPU_MID_BINS + b * RADIX;
-        uint32_t* const h = a.hist + first;
-        uint32_t cnt = 0;
-        if (first == 0) {
-            const uint32_t per = MGPU_MID_BINS >> a.last_width;
-            if (tid < (1u << a.last_width))
-                for (uint32_t i = 0; i < per; ++i) cnt += h[tid * per + i];
-        } else if (tid < RADIX) {
-            cnt = h[tid];
+    // (One call of the sort for both: its forms by size are most of the code.)
+    uint32_t begin = 0, n = a.n, base = 0, bits = a.num_bits;
+    if (a.plan) {
+        // The counts go back to zero; when the digit passes go on, workgroup p first
+        // makes pass p's digit starts of them (the last digits are the bins' top
+        // bits).
+        const uint32_t b = blockIdx.x;
+        if (b < a.num_passes) {
+            const uint32_t tid = threadIdx.x, first = b + 1 == a.num_passes ? 0u : MGPU_MID_BINS + b * RADIX;
+            uint32_t* const h = a.hist + first;
+            uint32_t cnt = 0;
+            if (first == 0) {
+                const uint32_t per = MGPU_MID_BINS >> a.last_width;
+                if (tid < (1u << a.last_width))
+                    for (uint32_t i = 0; i < per; ++i) cnt += h[tid * per + i];
+            } else if (tid < RADIX) {
+                cnt = h[tid];
+            }
+            const uint32_t st = mgpu::block_exclusive_scan_dpp<MGPU_LOCAL_THREADS>(
+                cnt, sh.tmp, tid & 63, (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)));
+            if (tid < RADIX) a.starts[b * RADIX + tid] = st;
+            __syncthreads();
+            if (first == 0 || tid < RADIX) h[tid] = 0;
         }
-        const uint32_t st = mgpu::block_exclusive_scan_dpp<MGPU_LOCAL_THREADS>(
-            cnt, sh.tmp, tid & 63, (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)));
-        if (tid < RADIX) a.starts[b * RADIX + tid] = st;
-        __syncthreads();
-        if (first == 0 || tid < RADIX) h[tid] = 0;
+        if (!a.plan->buckets) return;
+        begin = a.plan->start[b];
+        n = a.plan->start[b + 1] - begin;
+        base = a.plan->base[b];
+        bits = a.plan->bits[b];
+        if (n == 0) return;
+        if (n > MGPU_LOCAL_MAX_KEYS || begin > a.n || n > a.n - begin) {  // only from a broken count
+            if (threadIdx.x == 0) set_error(a.error_flag, 8u);
+            return;
+        }
     }
-    if (!a.plan->buckets) return;
-    const uint32_t begin = a.plan->start[b], n = a.plan->start[b + 1] - begin;
-    if (n == 0) return;
-    if (n > MGPU_LOCAL_MAX_KEYS || begin > a.n || n > a.n - begin) {  // only from a broken count
-        if (threadIdx.x == 0) set_error(a.error_flag, 8u);
-        return;
-    }
-    mgpu::local_sort<PAY, mgpu::kLocalBlock, MANY>(mgpu::LocalArrays{a, begin}, local_mem(sh), n,
-                                                   a.plan->base[b], a.first_bit, a.plan->bits[b]);
+    mgpu::local_sort<PAY, mgpu::kLocalBlock, MANY>(mgpu::LocalArrays{a, begin}, local_mem(sh), n, base,
+                                                   a.first_bit, bits);
 }
 
 extern "C" __global__ void __launch_bounds__(MGPU_LOCAL_THREADS) mgpu_local_sort_k(mgpuLocalArgs a) {

@@ -377,8 +377,9 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
     // Beside device-wide passes, a launch that sorts no more whole segments than
     // there are CUs costs what a full one does, and the passes would take those
     // segments along for nothing.  So few of them
-    // * are sorted in one launch on the side stream where small ones are there
-    //   anyway and the passes are more than two (40 segments log-uniform in [1,
+    // * are sorted in one launch on the side stream (up to a bucket's size with
+    //   the buckets, if there are any) where small ones are there anyway and the
+    //   passes are more than two (40 segments log-uniform in [1,
     //   2^16], key + value, 97 -> 92 us);
     // * else go through buckets above a bucket's size and are sorted with these
     //   up to it, where there are buckets (20 in [4097, 40000] 63 us by passes
@@ -389,18 +390,18 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
     // segments join the buckets' launch as well: 27 requests log-uniform in
     // [2^10, 2^18] ran 14 and 25 us longer with a launch for each of the two.
     const bool few = numWhole <= (uint32_t)e->numCUs;
-    bool smallInSlots = false, withBuckets = !few;
+    bool smallInSlots = false;
     const uint64_t bucketedKeys = lane.noSide ? longKeys : wholeKeys;
     const bool buckets = keep != 0 && directCount && use_buckets(e, P, pack_mode(e), bucketedKeys);
     if (lane.noSide ? buckets && keep > MGPU_BUCKET_KEYS
                     : buckets && few && (numSmall == 0 || P.sortPasses <= 2)) {
         keep = std::min<uint32_t>(keep, MGPU_BUCKET_KEYS);
-        withBuckets = true;
         smallInSlots = lane.noSide && numSmall <= (uint32_t)e->numCUs;
     } else if (few && longestSeg > keep &&
                (lane.noSide || numSmall == 0 || P.sortPasses <= 2)) {
         keep = 0;
     }
+    const bool withBuckets = buckets || !few;  // a launch for those of a bucket's size
     const bool noneAboveTile = longestSeg <= keep && seg_fits_tile(e, longestSeg);
     struct Group {
         std::vector<uint32_t> big, small;
