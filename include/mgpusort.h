@@ -196,8 +196,10 @@ sortStatus_t SORTAPI sortArrayNoAlloc(sortEngine_t engine, sortData_t data);
  * chosen by the caller: ceil(bits / bitPass) passes of bitPass bits (the first
  * ones a bit narrower when it does not divide), bitPass outside 1..6 taken as
  * 6.  The split sets the parity and the side of the result; without earlyExit
- * the engine runs fewer, wider passes where they leave both the same.  numSortThreads must be 128 or 256 and valuesPerThread 8, as in the
- * reference; the engine picks its own tile shape. */
+ * the engine runs fewer, wider passes where they leave both the same (what the
+ * split itself needs is asked for all the same).  numSortThreads must be 128 or
+ * 256 and valuesPerThread 8, as in the reference; the engine picks its own tile
+ * shape. */
 sortStatus_t SORTAPI sortArrayEx(sortEngine_t engine, sortData_t data, int numSortThreads,
                                  int valuesPerThread, int bitPass, bool useTransList);
 

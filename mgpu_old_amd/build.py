@@ -9,6 +9,7 @@ host code under UndefinedBehaviorSanitizer (load it with MGPUSORT_LIBRARY).
 """
 import hashlib
 import os
+import re
 import subprocess
 import sys
 
@@ -41,12 +42,14 @@ HIP_HOST_SOURCES = ["noalloc.hip"]
 def args_layout(text=None):
     """Number of the argument layouts in kernel_args.h (`text`, or the file):
     host library and code objects carry it, and an engine refuses code objects
-    of another number.  Any change of the file changes it, so that nothing has
-    to be raised by hand where sizes stay and meanings change."""
+    of another number.  Any change of the file but in comments and spacing
+    changes it, so that nothing has to be raised by hand where sizes stay and
+    meanings change."""
     if text is None:
         with open(os.path.join(CSRC, "kernel_args.h"), "rb") as f:
             text = f.read()
-    return int.from_bytes(hashlib.sha256(text).digest()[:4], "little") | 1
+    code = b" ".join(re.sub(rb"//[^\n]*", b"", text).split())
+    return int.from_bytes(hashlib.sha256(code).digest()[:4], "little") | 1
 
 
 def layout_flag():

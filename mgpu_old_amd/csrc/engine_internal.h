@@ -244,8 +244,9 @@ constexpr uint32_t kCountColsMinKeys = 1u << 20;
 const PassVariant& mgpu_pick_variant(const sortEngine_d* e, uint64_t keys);
 // Arrays of at most this many keys are sorted by one workgroup in one launch:
 // all that its LDS holds beside the digit counts (key and payload staged), and
-// still ahead of the device-wide passes there (16384 keys: 18.8 against 38.8
-// us, with one value 23.1 against 44.5, with three 38.9 against 56.0).
+// still ahead of the device-wide passes there (16384 keys: 19.0 against 39.0
+// us, with one value 23.7 against 44.7, with three 28.2 against 56.2, and by one
+// digit with six values 20.5 against 23.0).
 constexpr uint32_t kLocalSortMaxKeys = MGPU_LOCAL_MAX_KEYS;
 // Larger arrays of up to this many keys, by more than two passes, are sorted in
 // buckets: evenly spread keys fill 256 buckets of n / 256 keys plus one bin of

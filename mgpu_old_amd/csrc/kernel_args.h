@@ -274,8 +274,9 @@ struct mgpuMultiScanArgs {
     uint32_t pad_;
 };
 
-// A workgroup per slot, of 512 threads (up to MGPU_BUCKET_KEYS keys) or 1024: a bucket of a device-wide segment, or
-// a whole segment (MGPU_SLOT_WHOLE: seg indexes segs, else wide).
+// A workgroup per slot, of 512 threads (up to MGPU_BUCKET_KEYS keys) or 1024: a
+// bucket of a device-wide segment, or a whole segment (MGPU_SLOT_WHOLE: seg
+// indexes segs, else wide).
 #define MGPU_SLOT_WHOLE 0xFFFFFFFFu
 #define MGPU_BUCKET_THREADS 512
 #define MGPU_BUCKET_KEYS 8192

@@ -4,12 +4,13 @@
 //
 // Bound: a pass is a chain of LDS round trips and four barriers, not
 // bandwidth (16384 pairs are 256 KB): key + value, with the fill of the input,
-// 1000 keys 34.3 -> 6.9 us a sort, 4096 35.8 -> 10.1, 16384 44.5 -> 23.1
+// 1000 keys 34.6 -> 8.9 us a sort, 4096 36.3 -> 10.7, 16384 44.7 -> 23.7
 // against the device-wide passes (a launch each, ~6 us whatever the size);
-// keys only 32.2 -> 7.0, 33.2 -> 8.8, 38.8 -> 18.8.  So every slot's rank is requested
-// before the first one is used, and the digit scan runs over all threads at
-// once: thread (digit, group) adds the counts of four waves, and one scan over
-// the threads in that order gives each wave's start of each digit directly.
+// keys only 32.5 -> 8.8, 33.4 -> 9.1, 39.0 -> 19.0.  So every slot's rank is
+// requested before the first one is used, and the digit scan runs over all
+// threads at once: thread (digit, group) adds the counts of four waves, and one
+// scan over the threads in that order gives each wave's start of each digit
+// directly.
 #pragma once
 #include "kernel_args.h"
 #include "radix_device.h"

@@ -1,8 +1,18 @@
 // LSD radix sort pass kernels for gfx950 (CDNA4, wave64).
 //
-// One sort = digit_count (one read of the keys: the digit histogram of every
-// pass) -> digit_scan (exclusive scan of those histograms) -> one
-// rank_scatter launch per digit pass.
+// A large sort = digit_count (one read of the keys: the digit histogram of
+// every pass) -> digit_scan (exclusive scan of those histograms) -> one
+// rank_scatter launch per digit pass.  Smaller ones take fewer launches:
+//   up to 16384 keys   mgpu_local_sort_*: one workgroup, every pass in LDS;
+//   up to 3 * 2^20     mgpu_mid_count, one scatter into buckets (_m_) and a
+//                      workgroup's sort per bucket (mgpu_local_sort_*, or in
+//                      the next pass's launch, _l_); the passes after it (_c_,
+//                      or all in one launch, _f_) find that there is nothing
+//                      to do, or go on where no buckets would fit.
+// Batches take the multi_* kernels: a count per segment, which also plans its
+// buckets, then passes over the tiles of all segments; bucketed ones the
+// routed forms (_r_, _xr_), the second pass with the buckets' sorts in its
+// launch (mgpu_multi_scatter_slots_*).
 //
 // Reference kernels this replaces (seanbaxter/mgpu_old, sort/src/kernels):
 //   CountBuckets_n            count.cu:48-333      -> mgpu_digit_count,
@@ -702,14 +712,14 @@ __device__ __forceinline__ bool plan_buckets(const mgpuMultiCountArgs& a, uint32
     return true;
 }
 
-// The same over whole arrays (or 64K-key pieces of larger ones), one
+// The same over whole arrays (or pieces of them), one
 // 1024-thread workgroup each, with lane-column histograms: per (pass, digit
 // pair) a row of 32 words, word c counting the keys of the lanes with
 // lane % 32 == c in two 16-bit halves (even digit low, odd digit high).  The
 // 32 lanes of a half-wave then always add to distinct banks, and the lanes
 // that share a word (lane and lane + 32 of a wave) are at most two, where the
 // per-wave histograms had same-digit lanes serialize on one word.  A column
-// counts at most 32 threads x 64 keys of a 64K-key piece: 16 bits suffice.
+// counts a 32nd of a piece's keys, of at most 2^20: 16 bits suffice.
 __device__ void multi_count_cols_body(const mgpuMultiCountArgs& a) {
     constexpr int BLOCK = 1024;
     constexpr uint32_t COLS = 32, ROWS = MGPU_MAX_PASSES * RADIX / 2;
@@ -762,7 +772,7 @@ __device__ void multi_count_cols_body(const mgpuMultiCountArgs& a) {
     for (uint32_t i = begin + tid; i < vbeg; i += BLOCK) count_key(keys[i]);
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const auto v = mgpu::to_global(reinterpret_cast<const u32x4*>(kp + vbeg));
-    constexpr int UNROLL = 16;  // a 64K-key piece: every vector of a thread in flight
+    constexpr int UNROLL = 16;  // vectors of a thread in flight (all of them up to 64K keys)
     for (uint32_t i0 = tid; i0 < nvec; i0 += UNROLL * BLOCK) {
         u32x4 q[UNROLL];
 #pragma unroll
@@ -808,7 +818,7 @@ __device__ void multi_count_cols_body(const mgpuMultiCountArgs& a) {
         // one piece needs no global histogram.  Workgroup 0 zeroes the
         // passes' tile counters, as that launch would.
         // (With every array one piece, the longest set the time of a small
-        // batch: 4 of 200000 keys, key + value, 80 -> 54 us.)
+        // batch: 4 of 200000 keys, key + value, 80 -> 57 us.)
         __shared__ uint32_t s_tmp[BLOCK / 64], s_last;
         if (blockIdx.x == 0 && tid < MGPU_LSD_SLOT) a.tile_counters[tid] = 0;
         if (pieces > 1) {
@@ -1900,8 +1910,6 @@ __device__ void rank_scatter_body(const Args& a) {
         // The LDS reads of every slot are issued before the first store, so
         // that their latencies overlap instead of adding up slot by slot
         // (slots past the tile's keys read LDS words that are not used).
-        // (XSEG: the next tile's number is asked for here and read after the
-        // write-out, which covers the counter's answer.)
         const int32_t vrem = (int32_t)(tile_valid - tid);  // positions i*BLOCK < vrem are real
         uint32_t* const vout0 = JOINT ? vals_out(job, 0) : nullptr;
         uint32_t kout[IPT], dest[IPT], vout[JOINT ? IPT : 1];

@@ -37,6 +37,9 @@ constexpr uint32_t kDirectCountMax = 1u << 18;
 // keys 62 us in pieces of 8192, 58 whole; 4 of 200000 47 in pieces of up to
 // 32768, 73 whole (keys only; one workgroup counts 200000 keys in 43 us).
 constexpr uint32_t kCountPieceMin = 32768, kCountPieceMax = 1u << 18;
+// (The count's 16-bit counters hold a 32nd of a piece.)
+constexpr uint32_t kPieceLimit = 1u << 20;
+static_assert(kPieceLimit / 32 <= 0xFFFF && kCountPieceMax <= kPieceLimit, "16-bit counters");
 
 // Keys of a bucket of a device-wide segment, about (its last bin can make it
 // longer: see plan_buckets), where the batch is large and small, and keys of a
@@ -61,7 +64,7 @@ uint32_t device_wide_min(const sortEngine_d* e) {
 // Keys per digit_count workgroup on that path (a multiple of 1024 up to 2^20,
 // where the 16-bit lane-column counts of the 1024-thread count kernel would
 // start to overflow; MGPUSORT_SEG_WIDE_CHUNK overrides the table).
-uint32_t clamp_chunk(long x) { return (uint32_t)std::min<long>(std::max<long>(x, 1024), 1L << 20) & ~1023u; }
+uint32_t clamp_chunk(long x) { return (uint32_t)std::min<long>(std::max<long>(x, 1024), (long)kPieceLimit) & ~1023u; }
 uint32_t wide_chunk(const sortEngine_d* e) {
     const char* v = std::getenv("MGPUSORT_SEG_WIDE_CHUNK");
     const long x = v ? std::strtol(v, nullptr, 10) : 0;

@@ -132,7 +132,9 @@ struct SegPlanData {
     // call on the lane may free and replace it) unless the plan owns its
     // own, which a captured plan does: its graph's kernels address it.
     uint32_t* ownLookback = nullptr;  // [passes][wideTiles][MGPU_RADIX]
-    uint32_t* ownMulti = nullptr;     // hist then digit starts, [wide][4][MGPU_RADIX] each
+    // hist [wide][4][MGPU_RADIX], done [MGPU_MULTI_DONE_WORDS(wide)], digit
+    // starts (as hist).
+    uint32_t* ownMulti = nullptr;
 };
 
 sortStatus_t mgpu_seg_load(sortEngine_d* e);

@@ -680,8 +680,8 @@ __device__ __forceinline__ void block_sort8(const mgpuSegArgs& a, const SegArray
 
 // The small list, one segment per wave at a time, dealt round-robin over the
 // grid's waves.  A wave's segments are a chain of dependent reads (list,
-// descriptor, keys) and little else, so the list entry is read three segments
-// ahead, the descriptor two and the keys one.
+// descriptor, keys) and little else, so while one is sorted the next one's
+// descriptor and keys are read, and the list entry of the one after.
 template <int IPT, int BLOCK, bool PAY>
 __device__ __forceinline__ void wave_phase8(const mgpuSegArgs& a, uint32_t* row, uint32_t* skey, uint32_t* spay,
                             uint32_t lane, uint32_t wave) {
