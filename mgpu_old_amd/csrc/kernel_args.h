@@ -290,8 +290,13 @@ struct mgpuSegSlotArgs {
     uint32_t result_side;
     uint32_t first_bit;
     uint32_t num_bits;
-    uint32_t pad_;
+    uint32_t num_whole;           // slots before the first bucket
     uint32_t* error_flag;
+    // Slots with buckets (else null): the segments that take every pass, of
+    // num_wide (the second word at MGPU_LSD_SLOT).
+    const uint32_t* lsd_segments;
+    uint32_t num_wide;
+    uint32_t pad_;
 };
 
 // rank_scatter over the tiles of all arrays.

@@ -280,8 +280,9 @@ uint32_t keep_in_workgroup(const sortEngine_d* e) {
 // 512 in [2^15, 2^17] 400 -> 316 / 629 -> 452 / 905 -> 543; 32 of 32768 61 ->
 // 51 / 70 -> 58 / 106 -> 64; 8 of 32768 53 -> 44 / 61 -> 48; equal keys 344 ->
 // 172 / 515 -> 235 us (4096 segments).  Keys with two thirds in one digit
-// value, which take every pass, 512 in [2^15, 2^17] 515 -> 548 / 725 -> 787:
-// the chains per XCD that they would take otherwise.  Below 2^18 keys the
+// value, which take every pass (with a copy of the keys in each replay): 512 in
+// [2^15, 2^17] 562 -> 538 / 759 -> 775, 2000 of 16385 to 20000 602 -> 606 / 901
+// -> 935, 4096 in [1, 2^16] 390 -> 354 / 605 -> 527.  Below 2^18 keys the
 // launches are what counts, and the passes have no more of them.
 bool use_buckets(const sortEngine_d* e, const SegPlanData& P, int packMode, uint64_t wideKeys) {
     const char* v = std::getenv("MGPUSORT_SEG_XCD");
@@ -430,6 +431,7 @@ sortStatus_t mgpu_seg_build(sortEngine_d* e, SortLane& lane, const mgpuSegDesc* 
         if (n <= 64u * (uint32_t)ipt) g.small.push_back((uint32_t)i);
         else g.big.push_back((uint32_t)i);
     }
+    P.slotsWhole = (uint32_t)(P.slots.size() / 2);
 
     // Persistent kernels forked beside device-wide passes take at most
     // mixed_workgroups_per_cu() workgroups per CU.
@@ -824,6 +826,9 @@ mgpuSegSlotArgs slot_args(const SegPlanData& P, const SortLane& lane, bool large
     a.first_bit = (uint32_t)P.firstBit;
     a.num_bits = (uint32_t)P.numBits;
     a.error_flag = lane.errorDev;
+    a.num_whole = P.slotsWhole;
+    a.num_wide = (uint32_t)P.wide.size();
+    if (P.wideBuckets && !large) a.lsd_segments = lane.tileCounters + MGPU_LSD_SLOT + 1;
     return a;
 }
 

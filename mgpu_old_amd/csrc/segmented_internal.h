@@ -107,6 +107,7 @@ struct SegPlanData {
     // (512 threads a workgroup, then from slots1024 on 1024.)
     std::vector<uint32_t> slots;
     uint32_t slots1024 = 0;
+    uint32_t slotsWhole = 0;  // slots before the first bucket
     bool wideBuckets = false;
     uint32_t* devSlots = nullptr;
     mgpuSegDesc* devWide = nullptr;
